@@ -238,6 +238,21 @@ int bem_potential_dk(const bem_mesh* mesh, const float* points, int64_t np, floa
 int bem_potential_batch_k(const bem_mesh* mesh, const float* points, int64_t np, const float* ks, int nk, int op,
                           int basis, int clamp, void* out, int64_t ld, int64_t stride, void* stream);
 
+/* The exterior pressure p = D phi - S psi at np points (solver.py:140-147)
+ * without forming the two operators: psi, phi [n] complex64 (Neumann and
+ * Dirichlet data of the basis), out [np].  work: bem_field_work_size(mesh, np,
+ * nk) bytes of device scratch (nk = 1 here).  _batch_k: nk wavenumbers on one
+ * mesh (ks host [nk]; psi, phi [nk, n]; out [nk, np]); _samples: every sample of
+ * a geometry set at its own points (device [ns, np, 3]) and wavenumber (work
+ * sized with the set's mesh and nk = ns).  Deterministic. */
+int64_t bem_field_work_size(const bem_mesh* mesh, int64_t np, int nk);
+int bem_field(const bem_mesh* mesh, const float* points, int64_t np, float k, int basis, int clamp, const void* psi,
+              const void* phi, void* out, void* work, void* stream);
+int bem_field_batch_k(const bem_mesh* mesh, const float* points, int64_t np, const float* ks, int nk, int basis,
+                      int clamp, const void* psi, const void* phi, void* out, void* work, void* stream);
+int bem_field_samples(const bem_geomset* set, const float* points, int64_t np, const float* ks, int basis, int clamp,
+                      const void* psi, const void* phi, void* out, void* work, void* stream);
+
 /* y = alpha op(A) x + beta y, A complex64 [rows, cols] row-major, trans:
  * 0 = A, 1 = A^T, 2 = A^H.  work: device scratch of
  * bem_matvec_work_size() bytes (may be NULL when that is 0).  Replaces the

@@ -88,6 +88,10 @@ SIGNATURES = {
     "bem_triangle2vertex_raw": (_I32, [_P, _I64, _I64, _P, _P, _P, _P]),
     "bem_potential": (_I32, [_P, _P, _I64, _F, _I32, _I32, _I32, _P, _I64, _P]),
     "bem_potential_dk": (_I32, [_P, _P, _I64, _F, _I32, _I32, _I32, _P, _I64, _P]),
+    "bem_field_work_size": (_I64, [_P, _I64, _I32]),
+    "bem_field": (_I32, [_P, _P, _I64, _F, _I32, _I32, _P, _P, _P, _P, _P]),
+    "bem_field_batch_k": (_I32, [_P, _P, _I64, _P, _I32, _I32, _I32, _P, _P, _P, _P, _P]),
+    "bem_field_samples": (_I32, [_P, _P, _I64, _P, _I32, _I32, _P, _P, _P, _P, _P]),
     "bem_mesh_set_vertices": (_I32, [_P, _P, _I32, _P]),
     "bem_potential_batch_k": (_I32, [_P, _P, _I64, _P, _I32, _I32, _I32, _I32, _P, _I64, _I64, _P]),
     "bem_matvec_work_size": (_I64, [_I64, _I64, _I32]),

@@ -207,10 +207,32 @@ def boundary2potential_samples(gs: GeometrySet, ks, neumanns, dirichlets, points
     (solver.py:140-147): [ns, np]."""
     psi = torch.as_tensor(neumanns, device=gs.device).to(torch.complex64).reshape(gs.ns, -1).contiguous()
     phi = torch.as_tensor(dirichlets, device=gs.device).to(torch.complex64).reshape(gs.ns, -1).contiguous()
-    S = gs.potential(ks, points, "single", clamp=clamp)
-    D = gs.potential(ks, points, "double", clamp=clamp)
-    p = matvec_strided(D, phi)
-    return matvec_strided(S, psi, alpha=-1.0, beta=1.0, out=p)
+    psi, phi = _rows_of(psi, gs.mesh.nv), _rows_of(phi, gs.mesh.nv)
+    kh = gs._ks(ks)
+    pts = torch.as_tensor(points, dtype=torch.float32, device=gs.device).reshape(gs.ns, -1, 3).contiguous()
+    npts = pts.shape[1]
+    out, work = _field_buffers(gs.mesh, npts, gs.ns, gs.mesh.nv, psi, phi)
+    _lib.check(_lib.load().bem_field_samples(gs.handle, _ptr(pts), npts, kh.ctypes.data, _lib.BASES["P1"], int(clamp),
+                                             _ptr(psi), _ptr(phi), _ptr(out), _ptr(work), _stream()),
+               "bem_field_samples")
+    return out
+
+
+def _rows_of(x, n):
+    """The first n entries of each row of x, contiguous."""
+    return x[:, :n].contiguous() if x.shape[1] > n else x
+
+
+def _field_buffers(mesh, npts, nk, n, psi, phi):
+    """(out [nk, npts], work) of a pressure sweep, its boundary data checked."""
+    for v in (psi, phi):
+        check_tensor(v, torch.complex64)
+        if v.numel() < nk * n:
+            raise ValueError(f"boundary data must hold {n} values per system")
+    out = torch.empty((nk, npts), dtype=torch.complex64, device=mesh.device)
+    work = torch.empty(max(int(_lib.load().bem_field_work_size(mesh.handle, npts, nk)), 1), dtype=torch.uint8,
+                       device=mesh.device)
+    return out, work
 
 
 def preprocess(vertices, triangles):
@@ -583,15 +605,22 @@ class BEM_Solver:
     # -- potentials -----------------------------------------------------------
     def boundary2potential_batch(self, ks, neumanns, dirichlets, points):
         """boundary2potential at every wavenumber of ``ks``: p [K, P] = D phi -
-        S psi, the potential operators of all wavenumbers in one launch each."""
+        S psi, all wavenumbers in one sweep."""
         ks = [float(k) for k in ks]
         neumanns = torch.as_tensor(neumanns, device=self.device).to(torch.complex64).reshape(len(ks), -1)
         dirichlets = torch.as_tensor(dirichlets, device=self.device).to(torch.complex64).reshape(len(ks), -1)
         neumanns, dirichlets = neumanns.contiguous(), dirichlets.contiguous()
-        S = self.potential_matrix_batch(ks, points, "single")
-        D = self.potential_matrix_batch(ks, points, "double")
-        p = matvec_strided(D, dirichlets)
-        return matvec_strided(S, neumanns, alpha=-1.0, beta=1.0, out=p)
+        points = points.to(torch.float32).contiguous()
+        check_tensor(points, torch.float32)
+        n = self._n(self.basis)
+        neumanns, dirichlets = _rows_of(neumanns, n), _rows_of(dirichlets, n)
+        kh = np.ascontiguousarray(np.asarray(ks, dtype=np.float32))
+        out, work = _field_buffers(self.mesh, points.shape[0], len(ks), n, neumanns, dirichlets)
+        _lib.check(_lib.load().bem_field_batch_k(self.mesh.handle, _ptr(points), points.shape[0], kh.ctypes.data,
+                                                 len(ks), _lib.BASES[self.basis], int(self.clamp), _ptr(neumanns),
+                                                 _ptr(dirichlets), _ptr(out), _ptr(work), _stream()),
+                   "bem_field_batch_k")
+        return out
 
     def potential_matrix(self, k, points, layer_type, basis=None, clamp=None):
         basis = basis or self.basis
@@ -639,11 +668,16 @@ class BEM_Solver:
         return matvec(self.potential_matrix(k, points, "double"), dirichlet.to(torch.complex64).contiguous())
 
     def boundary2potential(self, k, neumann, dirichlet, points):
-        """p = -S psi + D phi (solver.py:140-147)."""
-        S = self.potential_matrix(k, points, "single")
-        D = self.potential_matrix(k, points, "double")
-        p = matvec(D, dirichlet.to(torch.complex64).contiguous())
-        return matvec(S, neumann.to(torch.complex64).contiguous(), alpha=-1.0, beta=1.0, out=p)
+        """p = -S psi + D phi (solver.py:140-147), neither operator formed
+        (bem_field: the boundary data contracted inside the evaluation)."""
+        points = points.to(torch.float32).contiguous()
+        check_tensor(points, torch.float32)
+        psi, phi = neumann.to(torch.complex64).contiguous(), dirichlet.to(torch.complex64).contiguous()
+        out, work = _field_buffers(self.mesh, points.shape[0], 1, self._n(self.basis), psi, phi)
+        _lib.check(_lib.load().bem_field(self.mesh.handle, _ptr(points), points.shape[0], float(k),
+                                         _lib.BASES[self.basis], int(self.clamp), _ptr(psi), _ptr(phi), _ptr(out),
+                                         _ptr(work), _stream()), "bem_field")
+        return out[0]
 
 
 def map_triangle2vertex(vertices, triangles, features):

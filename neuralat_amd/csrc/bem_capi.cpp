@@ -732,6 +732,52 @@ int bem_potential(const bem_mesh* mesh, const float* points, int64_t np, float k
     return BEM_OK;
 }
 
+int64_t bem_field_work_size(const bem_mesh* mesh, int64_t np, int nk)
+{
+    return mesh && np > 0 && nk > 0 ? bem::field_work_bytes(mesh->dev.nt, np, nk) : 0;
+}
+
+static int field_checked(const bem::MeshDev& m, int64_t gstride, const float* points, int64_t np, int64_t pstride,
+                         const float* ks, int nk, int basis, int clamp, const void* psi, const void* phi, void* out,
+                         void* work, void* stream, const char* what)
+{
+    if (np < 0) return fail(BEM_ERR_BAD_ARG, "negative point count");
+    if (!psi || !phi || (np > 0 && (!points || !out || !work))) return fail(BEM_ERR_BAD_ARG, "null pointer");
+    if (basis != BEM_BASIS_P1 && basis != BEM_BASIS_DP0) return fail(BEM_ERR_BAD_ARG, "unknown basis");
+    DeviceGuard g(m.device);
+    if (!g.ok) return fail(BEM_ERR_HIP, "cannot select the mesh's device");
+    hipError_t e = bem::launch_field(m, gstride, points, np, pstride, ks, nk, basis, clamp, (const float2*)psi,
+                                     (const float2*)phi, (float2*)out, work, S(stream));
+    if (e != hipSuccess) return hip_fail(e, what);
+    return BEM_OK;
+}
+
+int bem_field(const bem_mesh* mesh, const float* points, int64_t np, float k, int basis, int clamp, const void* psi,
+              const void* phi, void* out, void* work, void* stream)
+{
+    if (!mesh) return fail(BEM_ERR_BAD_ARG, "null mesh");
+    return field_checked(mesh->dev, 0, points, np, 0, &k, 1, basis, clamp, psi, phi, out, work, stream,
+                         "bem_field launch");
+}
+
+int bem_field_batch_k(const bem_mesh* mesh, const float* points, int64_t np, const float* ks, int nk, int basis,
+                      int clamp, const void* psi, const void* phi, void* out, void* work, void* stream)
+{
+    if (!mesh) return fail(BEM_ERR_BAD_ARG, "null mesh");
+    if (int rc = check_ks(ks, nk, BEM_OP_SINGLE)) return rc;
+    return field_checked(mesh->dev, 0, points, np, 0, ks, nk, basis, clamp, psi, phi, out, work, stream,
+                         "bem_field_batch_k launch");
+}
+
+int bem_field_samples(const bem_geomset* gs, const float* points, int64_t np, const float* ks, int basis, int clamp,
+                      const void* psi, const void* phi, void* out, void* work, void* stream)
+{
+    if (!gs) return fail(BEM_ERR_BAD_ARG, "null geometry set");
+    if (int rc = check_ks(ks, gs->ns, BEM_OP_SINGLE)) return rc;
+    return field_checked(gs->view, gs->gstride, points, np, 3 * np, ks, gs->ns, basis, clamp, psi, phi, out, work,
+                         stream, "bem_field_samples launch");
+}
+
 int bem_potential_dk(const bem_mesh* mesh, const float* points, int64_t np, float k, int op, int basis, int clamp,
                      void* out, int64_t ld, void* stream)
 {

@@ -191,6 +191,14 @@ hipError_t launch_potential(const MeshDev& m, const float* pts, int64_t np, floa
 hipError_t launch_potential_batch_k(const MeshDev& m, const float* pts, int64_t np, const float* ks, int nk, int op,
                                     int basis, int clamp, float2* out, int64_t ld, int64_t stride, hipStream_t s);
 
+// p_z = D phi_z - S psi_z at points (boundary data contracted inside the
+// sweep), nk systems: geometry z gstride floats on, points z at pts + z pstride,
+// wavenumber ks[z] (host), psi, phi [nk, n], out [nk, np]
+int64_t field_work_bytes(int64_t nt, int64_t np, int nk);
+hipError_t launch_field(const MeshDev& mg, int64_t gstride, const float* pts, int64_t np, int64_t pstride,
+                        const float* ks, int nk, int basis, int clamp, const float2* psi, const float2* phi,
+                        float2* out, void* work, hipStream_t s);
+
 // Builds all device data from host copies of the mesh; returns 0 or a
 // bem_status code with a message in `err`.
 int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t nt, MeshDev& m, std::string& err);
