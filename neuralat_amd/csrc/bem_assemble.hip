@@ -429,47 +429,65 @@ hipError_t launch_batch_cbie_persistent(const BatchItemDev* items, int nitems, i
 int64_t batch_cbie_tasks(int64_t nt, int rt) { return cbie_sym_tasks(nt, rt); }
 
 // rhs_i = -(row partials + column partials + singular V psi terms of row i);
-// lhs_ii += |T_i| / 2 (the M/2 of the CBIE).  One thread per row, fixed
-// summation order; column slots of one 64-row block are combined pairwise
-// exactly as a 64-row task combines its 16-row chunks.
-__global__ __launch_bounds__(256) void cbie_finalize_kernel(const float2* __restrict__ prow,
-                                                            const float2* __restrict__ pcol, int nsub,
-                                                            const float2* __restrict__ vpsi,
-                                                            const int64_t* __restrict__ pair_ptr,
-                                                            const float* __restrict__ geo, int64_t nt,
-                                                            float2* __restrict__ lhs, int64_t ld,
-                                                            float2* __restrict__ rhs)
+// lhs_ii += |T_i| / 2 (the M/2 of the CBIE).  A workgroup owns 64 rows; its 16
+// wavefronts take every 16th block partial of a row (coalesced over the rows)
+// and meet in LDS in a fixed order.  One thread per row walked the partials
+// of 320 blocks alone on 80 workgroups: 172 us at 20480 triangles.  Column slots
+// of one 64-row block are combined pairwise exactly as a 64-row task combines
+// its 16-row chunks.  grid (row blocks of 64, items)
+constexpr int kFinWaves = 16;
+__device__ __forceinline__ void cbie_finalize_rows(const CbiePairItem& it, double2 (*__restrict__ red)[64])
 {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= nt) return;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int64_t nt = it.nt, bi = blockIdx.x, i = bi * kSymBlock + lane;
     const int64_t nb = (nt + kSymBlock - 1) / kSymBlock;
-    const int64_t bi = i / kSymBlock;
+    if (bi >= nb) return;  // uniform: this item is shorter
     double sr = 0.0, si = 0.0;
-    for (int64_t J = bi; J < nb; ++J) {
-        const float2 p = prow[J * nt + i];
-        sr += p.x;
-        si += p.y;
-    }
-    for (int64_t I = 0; I <= bi; ++I) {
-        const float2* c = pcol + I * nsub * nt + i;
-        float2 v;
-        if (nsub == 1) {
-            v = c[0];
-        } else if (nsub == 2) {
-            v = make_float2(c[0].x + c[nt].x, c[0].y + c[nt].y);
-        } else {
-            v = make_float2((c[0].x + c[nt].x) + (c[2 * nt].x + c[3 * nt].x),
-                            (c[0].y + c[nt].y) + (c[2 * nt].y + c[3 * nt].y));
+    if (i < nt) {
+        for (int64_t J = bi + wv; J < nb; J += kFinWaves) {
+            const float2 p = it.prow[J * nt + i];
+            sr += p.x;
+            si += p.y;
         }
-        sr += v.x;
-        si += v.y;
+        for (int64_t I = wv; I <= bi; I += kFinWaves) {
+            const float2* c = it.pcol + I * it.nsub * nt + i;
+            float2 v;
+            if (it.nsub == 1) {
+                v = c[0];
+            } else if (it.nsub == 2) {
+                v = make_float2(c[0].x + c[nt].x, c[0].y + c[nt].y);
+            } else {
+                v = make_float2((c[0].x + c[nt].x) + (c[2 * nt].x + c[3 * nt].x),
+                                (c[0].y + c[nt].y) + (c[2 * nt].y + c[3 * nt].y));
+            }
+            sr += v.x;
+            si += v.y;
+        }
+        const int64_t e1 = it.pair_ptr[i + 1];
+        for (int64_t e = it.pair_ptr[i] + wv; e < e1; e += kFinWaves) {
+            sr += it.vpsi[e].x;
+            si += it.vpsi[e].y;
+        }
     }
-    for (int64_t e = pair_ptr[i]; e < pair_ptr[i + 1]; ++e) {
-        sr += vpsi[e].x;
-        si += vpsi[e].y;
+    red[wv][lane] = make_double2(sr, si);
+    __syncthreads();
+    if (wv != 0 || i >= nt) return;
+    for (int q = 1; q < kFinWaves; ++q) {
+        sr += red[q][lane].x;
+        si += red[q][lane].y;
     }
-    rhs[i] = make_float2((float)-sr, (float)-si);
-    lhs[i * ld + i].x += 0.25f * geo[i * 16 + 12];  // M_ii / 2 = |T_i| / 2 = |J_i| / 4
+    it.rhs[i] = make_float2((float)-sr, (float)-si);
+    it.lhs[i * it.ld + i].x += 0.25f * it.geo[i * 16 + 12];  // M_ii / 2 = |T_i| / 2 = |J_i| / 4
+}
+__global__ __launch_bounds__(64 * kFinWaves) void cbie_finalize_kernel(const CbiePairItem it)
+{
+    __shared__ double2 red[kFinWaves][64];
+    cbie_finalize_rows(it, red);
+}
+__global__ __launch_bounds__(64 * kFinWaves) void batch_cbie_finalize_kernel(const CbiePairItem* __restrict__ items)
+{
+    __shared__ double2 red[kFinWaves][64];
+    cbie_finalize_rows(items[blockIdx.y], red);
 }
 
 // ---------------------------------------------------------------------------
@@ -1253,8 +1271,76 @@ __device__ __forceinline__ double group_sum(double v)
     }
 }
 
+// A neighbour pair made ready for its quadrature: the shared vertices moved to
+// local 0 (and 1) on both triangles, edge vectors, normals, |J_i| |J_j|.
+// Everything is picked by selects: arrays indexed at run time went to scratch
+// memory (128 bytes per lane).
+__device__ __forceinline__ int pick3(const int (&v)[3], int i) { return i == 0 ? v[0] : (i == 1 ? v[1] : v[2]); }
+struct SSPair {
+    int pi[3], pj[3];   // local index in the caller's order of reordered corner a / b
+    int ia[3], ja[3];   // vertex ids (caller's order)
+    float e1[3], e2[3], f1[3], f2[3], nx[3], ny[3];
+    float jij;
+};
+__device__ __forceinline__ void ss_pair_setup(const float* __restrict__ geo, const int4* __restrict__ tris, int i,
+                                              int j, int shared, SSPair& g)
+{
+    const int4 ti = tris[i], tj = tris[j];
+    g.ia[0] = ti.x; g.ia[1] = ti.y; g.ia[2] = ti.z;
+    g.ja[0] = tj.x; g.ja[1] = tj.y; g.ja[2] = tj.z;
+    // m_b: the row corner equal to column corner b, -1 if none
+    auto match = [&](int v) { return ti.x == v ? 0 : (ti.y == v ? 1 : (ti.z == v ? 2 : -1)); };
+    const int m0 = match(tj.x), m1 = match(tj.y), m2 = match(tj.z);
+    g.pi[0] = g.pj[0] = 0;
+    g.pi[1] = g.pj[1] = 1;
+    g.pi[2] = g.pj[2] = 2;
+    if (shared == 2) {
+        // common edge first, same order on both triangles, ordered by position
+        // in the column triangle (integrand.h:351-364)
+        const int ub = m0 < 0 ? 0 : (m1 < 0 ? 1 : 2);
+        g.pj[0] = ub == 0 ? 1 : 0;
+        g.pj[1] = ub == 2 ? 1 : 2;
+        g.pj[2] = ub;
+        g.pi[0] = ub == 0 ? m1 : m0;
+        g.pi[1] = ub == 2 ? m1 : m2;
+        g.pi[2] = 3 - g.pi[0] - g.pi[1];
+    } else if (shared == 1) {
+        // common vertex swapped to local 0 (integrand.h:365-382)
+        const int b = m0 >= 0 ? 0 : (m1 >= 0 ? 1 : 2), a = m0 >= 0 ? m0 : (m1 >= 0 ? m1 : m2);
+        g.pi[0] = a;
+        g.pi[1] = a == 1 ? 0 : 1;
+        g.pi[2] = a == 2 ? 0 : 2;
+        g.pj[0] = b;
+        g.pj[1] = b == 1 ? 0 : 1;
+        g.pj[2] = b == 2 ? 0 : 2;
+    }
+    // geo record: v0 v1 v2 (9), n (3), jac (1), pad
+    const float* gi = geo + (int64_t)i * 16;
+    const float* gj = geo + (int64_t)j * 16;
+    float v[3][3], w[3][3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            v[a][d] = gi[3 * g.pi[a] + d];
+            w[a][d] = gj[3 * g.pj[a] + d];
+        }
+    // x = v0 + x1 (v1 - v0) + x2 (v2 - v1) on (0,0),(1,0),(1,1); the shared
+    // local vertex 0 (v0 = w0 in all three cases) cancels in d = y - x.
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        g.e1[d] = v[1][d] - v[0][d];
+        g.e2[d] = v[2][d] - v[1][d];
+        g.f1[d] = w[1][d] - w[0][d];
+        g.f2[d] = w[2][d] - w[1][d];
+        g.nx[d] = gi[9 + d];
+        g.ny[d] = gj[9 + d];
+    }
+    g.jij = gi[12] * gj[12];
+}
+
 // MODE 0: write (DP0: out = alpha * entry) or add (P1) the entries;
-// MODE 1 (DP0): vpsi[p] = entry * psi[j], the pair's term of V psi.
+// MODE 2 (P1): contract them with psi into vpsi, nothing stored.
 template <int OP, int NL, int BASIS, bool CLAMP, int MODE = 0>
 __global__ __launch_bounds__(256) void singular_kernel(const float* __restrict__ geo, const int4* __restrict__ tris,
                                                        const float* __restrict__ curls,
@@ -1275,7 +1361,7 @@ __global__ __launch_bounds__(256) void singular_kernel(const float* __restrict__
     // lanes per pair: a wavefront per pair, except the 2-point line rule of the
     // P1 operators (16 points): 16 lanes per pair, 4 pairs per wavefront, so
     // the FP64 reductions run over 16 lanes and serve four pairs
-    constexpr int LPP = (NL == 2 && BASIS == P1 && MODE != 1) ? 16 : 64;
+    constexpr int LPP = (NL == 2 && BASIS == P1) ? 16 : 64;
     constexpr int PPW = 64 / LPP;
     const int ll = lane % LPP;
     const int64_t pw = p0 + ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * PPW;  // the wavefront's first pair
@@ -1286,51 +1372,10 @@ __global__ __launch_bounds__(256) void singular_kernel(const float* __restrict__
     const int i = PPW == 1 ? __builtin_amdgcn_readfirstlane(pr.x) : pr.x;
     const int j = PPW == 1 ? __builtin_amdgcn_readfirstlane(pr.y) : pr.y;
     const int shared = PPW == 1 ? __builtin_amdgcn_readfirstlane(pr.z) : pr.z;
-    const int4 ti = tris[i], tj = tris[j];
-    const int ia[3] = {ti.x, ti.y, ti.z}, ja[3] = {tj.x, tj.y, tj.z};
-    int pi[3] = {0, 1, 2}, pj[3] = {0, 1, 2};
-    if (shared == 2) {
-        // common edge first, same order on both triangles, ordered by position
-        // in the column triangle (integrand.h:351-364)
-        int c = 0;
-        for (int b = 0; b < 3; ++b)
-            for (int a = 0; a < 3; ++a)
-                if (ia[a] == ja[b]) { pi[c] = a; pj[c] = b; ++c; }
-        pi[2] = 3 - pi[0] - pi[1];
-        pj[2] = 3 - pj[0] - pj[1];
-    } else if (shared == 1) {
-        // common vertex swapped to local 0 (integrand.h:365-382)
-        for (int a = 0; a < 3; ++a)
-            for (int b = 0; b < 3; ++b)
-                if (ia[a] == ja[b]) {
-                    if (a != 0) { pi[0] = a; pi[a] = 0; }
-                    if (b != 0) { pj[0] = b; pj[b] = 0; }
-                }
-    }
-    // geo record: v0 v1 v2 (9), n (3), jac (1), pad
-    const float* gi = geo + (int64_t)i * 16;
-    const float* gj = geo + (int64_t)j * 16;
-    float v[3][3], w[3][3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            v[a][d] = gi[3 * pi[a] + d];
-            w[a][d] = gj[3 * pj[a] + d];
-        }
-    // x = v0 + x1 (v1 - v0) + x2 (v2 - v1) on (0,0),(1,0),(1,1); the shared
-    // local vertex 0 (v0 = w0 in all three cases) cancels in d = y - x.
-    float e1[3], e2[3], f1[3], f2[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        e1[d] = v[1][d] - v[0][d];
-        e2[d] = v[2][d] - v[1][d];
-        f1[d] = w[1][d] - w[0][d];
-        f2[d] = w[2][d] - w[1][d];
-    }
-    const float nx0 = gi[9], nx1 = gi[10], nx2 = gi[11];
-    const float ny0 = gj[9], ny1 = gj[10], ny2 = gj[11];
-    const float jij = gi[12] * gj[12];
+    SSPair g;
+    ss_pair_setup(geo, tris, i, j, shared, g);
+    const float nx0 = g.nx[0], nx1 = g.nx[1], nx2 = g.nx[2], ny0 = g.ny[0], ny1 = g.ny[1], ny2 = g.ny[2];
+    const float jij = g.jij;
     const float krev = k * kInv2Pi;
 
     double ar[10], ai[10];
@@ -1356,7 +1401,7 @@ __global__ __launch_bounds__(256) void singular_kernel(const float* __restrict__
             for (int r = 0; r < NR; ++r) {
                 const float x1 = reg[r][0], x2 = reg[r][1], y1 = reg[r][2], y2 = reg[r][3];
                 float dx, dy, dz;
-                ss_disp<S>(reg[r], e1, e2, f1, f2, dx, dy, dz);
+                ss_disp<S>(reg[r], g.e1, g.e2, g.f1, g.f2, dx, dy, dz);
                 float vr, vi, gr = 0.f, gg = 0.f;
                 kernel4pi<OP, CLAMP>(dx, dy, dz, nx0, nx1, nx2, ny0, ny1, ny2, k, krev, vr, vi, gr, gg);
                 const float ww = reg[r][4];
@@ -1395,12 +1440,7 @@ __global__ __launch_bounds__(256) void singular_kernel(const float* __restrict__
         ar[e] = group_sum<LPP>(ar[e]) * (double)kInv4Pi;
         ai[e] = group_sum<LPP>(ai[e]) * (double)kInv4Pi;
     }
-    if constexpr (MODE == 1) {
-        if (lane == 0) {
-            const float2 pj = psi[j];
-            vpsi[p] = make_float2((float)(ar[9] * pj.x - ai[9] * pj.y), (float)(ar[9] * pj.y + ai[9] * pj.x));
-        }
-    } else if constexpr (BASIS == DP0) {
+    if constexpr (BASIS == DP0) {
         if (lane == 0)
             out[((int64_t)i - row0) * ld + j] = make_float2((float)(alpha * ar[9]), (float)(alpha * ai[9]));
     } else if constexpr (MODE == 2) {
@@ -1418,8 +1458,8 @@ __global__ __launch_bounds__(256) void singular_kernel(const float* __restrict__
 #pragma unroll
             for (int e = 0; e < 9; ++e)
                 if (e == ll) { vr = ar[e]; vi = ai[e]; }
-            oa = pi[a];
-            const float2 gv = psi[ja[pj[b]]];
+            oa = pick3(g.pi, a);
+            const float2 gv = psi[pick3(g.ja, pick3(g.pj, b))];
             cr = (float)(vr * gv.x - vi * gv.y);
             cim = (float)(vr * gv.y + vi * gv.x);
         }
@@ -1427,19 +1467,19 @@ __global__ __launch_bounds__(256) void singular_kernel(const float* __restrict__
         const float r1 = __shfl_down(cr, 1, 64), i1 = __shfl_down(cim, 1, 64);
         const float r2 = __shfl_down(cr, 2, 64), i2 = __shfl_down(cim, 2, 64);
         if (valid && ll < 9 && ll % 3 == 0) {
-            float* dst = reinterpret_cast<float*>(&vpsi[ia[oa]]);
+            float* dst = reinterpret_cast<float*>(&vpsi[pick3(g.ia, oa)]);
             unsafeAtomicAdd(dst, cr + r1 + r2);
             unsafeAtomicAdd(dst + 1, cim + i1 + i2);
         }
     } else {
         if (valid && ll < 9) {
-            // ll = reordered (a, b) pair; its original local indices are (pi[a], pj[b])
+            // ll = reordered (a, b) pair; its original local indices are (g.pi[a], g.pj[b])
             const int a = ll / 3, b = ll % 3;
             double vr = 0.0, vi = 0.0;
 #pragma unroll
             for (int e = 0; e < 9; ++e)
                 if (e == ll) { vr = ar[e]; vi = ai[e]; }
-            const int oa = pi[a], ob = pj[b];
+            const int oa = pick3(g.pi, a), ob = pick3(g.pj, b);
             if constexpr (OP == HYP || base_op(OP) == BM_LHS) {
                 float ci[9], cj[9], cp[9];
 #pragma unroll
@@ -1448,7 +1488,10 @@ __global__ __launch_bounds__(256) void singular_kernel(const float* __restrict__
                     cj[e] = curls[(int64_t)j * 12 + e];
                 }
                 curl_product(ci, cj, cp);
-                const double c = cp[3 * oa + ob];
+                double c = 0.0;
+#pragma unroll
+                for (int e = 0; e < 9; ++e)
+                    if (e == 3 * oa + ob) c = cp[e];
                 if constexpr (OP == HYP) {
                     const double kk = (double)k * (double)k * (double)(nx0 * ny0 + nx1 * ny1 + nx2 * ny2);
                     // sum over all 9 reordered entries = plain-G integral (phi sums to 1)
@@ -1460,11 +1503,100 @@ __global__ __launch_bounds__(256) void singular_kernel(const float* __restrict__
                     vi += ar[9] * invk * c;
                 }
             }
-            float* dst = reinterpret_cast<float*>(&out[(int64_t)ia[oa] * ld + ja[ob]]);
+            float* dst = reinterpret_cast<float*>(&out[(int64_t)pick3(g.ia, oa) * ld + pick3(g.ja, ob)]);
             unsafeAtomicAdd(dst, (float)vr);
             unsafeAtomicAdd(dst + 1, (float)vi);
         }
     }
+}
+
+// The neighbour pairs of the fused DP0 CBIE system: one evaluation per point
+// gives the pair's K entry (lhs = -K) and its term V_ij psi_j of the
+// right-hand side (vpsi), which share the displacement, r and e^{ikr}; as two
+// singular_kernel launches they took 256 + 211 us at 20480 triangles, and the
+// 3 x 24 launches of a batch of 24 small systems 2.0 ms of 9.6.  A
+// wavefront per pair (256 points), or 16 lanes for the 2-point rule (16
+// points, four pairs per wavefront); FP64 sums over the points.
+template <int NL, bool CLAMP>
+__device__ __forceinline__ void cbie_pair(const CbiePairItem& it, int64_t group)
+{
+    constexpr int LPP = NL == 2 ? 16 : 64;
+    constexpr int PPW = 64 / LPP;
+    const int lane = threadIdx.x & 63;
+    const int ll = lane % LPP;
+    const int64_t pw = group * PPW;
+    if (pw >= it.npairs) return;  // uniform per wavefront
+    const int64_t p = pw + lane / LPP;
+    const bool valid = p < it.npairs;  // groups past the end compute on the last pair and write nothing
+    const int4 pr = it.pairs[valid ? p : it.npairs - 1];
+    const int i = PPW == 1 ? __builtin_amdgcn_readfirstlane(pr.x) : pr.x;
+    const int j = PPW == 1 ? __builtin_amdgcn_readfirstlane(pr.y) : pr.y;
+    const int shared = PPW == 1 ? __builtin_amdgcn_readfirstlane(pr.z) : pr.z;
+    SSPair g;
+    ss_pair_setup(it.geo, it.tris, i, j, shared, g);
+    const float krev = it.k * kInv2Pi;
+    double vr = 0.0, vi = 0.0, kr = 0.0, ki = 0.0;
+    constexpr int NP = NL * NL * NL * NL;
+    ss_dispatch(shared, [&](auto kind) {
+        constexpr int S = decltype(kind)::value;
+        constexpr int NR = kSSRegions<S>;
+        for (int q = ll; q < NP; q += LPP) {
+            const int q0 = q / (NL * NL * NL), q1 = (q / (NL * NL)) % NL, q2 = (q / NL) % NL, q3 = q % NL;
+            const float wq =
+                LineRule01<NL>::w[q0] * LineRule01<NL>::w[q1] * LineRule01<NL>::w[q2] * LineRule01<NL>::w[q3];
+            float reg[NR][7];
+            const float jac = ss_regions<S>(LineRule01<NL>::t[q0], LineRule01<NL>::t[q1], LineRule01<NL>::t[q2],
+                                            LineRule01<NL>::t[q3], reg);
+            float a[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                float dx, dy, dz, s0, s1, d0, d1, u0 = 0.f, u1 = 0.f;
+                ss_disp<S>(reg[r], g.e1, g.e2, g.f1, g.f2, dx, dy, dz);
+                kernel4pi<SLP, CLAMP>(dx, dy, dz, 0.f, 0.f, 0.f, g.ny[0], g.ny[1], g.ny[2], it.k, krev, s0, s1, u0,
+                                      u1);
+                kernel4pi<DLP, CLAMP>(dx, dy, dz, 0.f, 0.f, 0.f, g.ny[0], g.ny[1], g.ny[2], it.k, krev, d0, d1, u0,
+                                      u1);
+                const float ww = reg[r][4];
+                a[0] += s0 * ww;
+                a[1] += s1 * ww;
+                a[2] += d0 * ww;
+                a[3] += d1 * ww;
+            }
+            const double sc = (double)(jac * wq) * (double)g.jij;
+            vr += sc * (double)a[0];
+            vi += sc * (double)a[1];
+            kr += sc * (double)a[2];
+            ki += sc * (double)a[3];
+        }
+    });
+    vr = group_sum<LPP>(vr) * (double)kInv4Pi;
+    vi = group_sum<LPP>(vi) * (double)kInv4Pi;
+    kr = group_sum<LPP>(kr) * (double)kInv4Pi;
+    ki = group_sum<LPP>(ki) * (double)kInv4Pi;
+    if (valid && ll == 0) {
+        const float2 pj = it.psi[j];
+        it.lhs[(int64_t)i * it.ld + j] = make_float2((float)-kr, (float)-ki);
+        it.vpsi[p] = make_float2((float)(vr * pj.x - vi * pj.y), (float)(vr * pj.y + vi * pj.x));
+    }
+}
+template <int NL, bool CLAMP>
+__global__ __launch_bounds__(256) void cbie_pairs_kernel(const CbiePairItem it)
+{
+    cbie_pair<NL, CLAMP>(it, (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6));
+}
+// every item of a batch (full rules): wavefront w takes the pair w - pair0 of
+// the item with the largest pair0 <= w
+template <bool CLAMP>
+__global__ __launch_bounds__(256) void batch_cbie_pairs_kernel(const CbiePairItem* __restrict__ items, int nitems)
+{
+    const int64_t w = uniform_i64((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6));
+    int lo = 0, hi = nitems - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (items[mid].pair0 <= w) lo = mid;
+        else hi = mid - 1;
+    }
+    cbie_pair<4, CLAMP>(items[lo], w - items[lo].pair0);
 }
 
 // rhs[caller id of slot s] += sum over column tiles (fixed order) of
@@ -1901,6 +2033,48 @@ CbieWork cbie_work_split(const MeshDev& m, int rt, void* work)
     return w;
 }
 
+CbiePairItem cbie_pair_item(const MeshDev& m, float k, const float2* psi, float2* lhs, int64_t ld, float2* rhs,
+                            const CbieWork& w)
+{
+    CbiePairItem it{};
+    it.geo = m.geo;
+    it.tris = m.tris;
+    it.pairs = m.pairs;
+    it.pair_ptr = m.pair_ptr;
+    it.npairs = m.npairs;
+    it.nt = m.nt;
+    it.k = k;
+    it.nsub = w.nsub;
+    it.psi = psi;
+    it.lhs = lhs;
+    it.ld = ld;
+    it.rhs = rhs;
+    it.prow = w.prow;
+    it.pcol = w.pcol;
+    it.vpsi = w.vpsi;
+    return it;
+}
+
+// the neighbour pairs and the row reduction of every item (full rules), one
+// launch each: items in table order, nwaves = the sum of their pair counts,
+// ntmax the largest item
+hipError_t launch_batch_cbie_finish(const CbiePairItem* items, int nitems, int64_t nwaves, int64_t ntmax, int clamp,
+                                    hipStream_t s)
+{
+    const unsigned g = (unsigned)((nwaves + 3) / 4);
+    if (nwaves > 0) {
+        if (clamp) hipLaunchKernelGGL(batch_cbie_pairs_kernel<true>, dim3(g), dim3(256), 0, s, items, nitems);
+        else hipLaunchKernelGGL(batch_cbie_pairs_kernel<false>, dim3(g), dim3(256), 0, s, items, nitems);
+    }
+    for (int q0 = 0; q0 < nitems; q0 += 65535) {  // grid y limit
+        const int cq = nitems - q0 < 65535 ? nitems - q0 : 65535;
+        hipLaunchKernelGGL(batch_cbie_finalize_kernel,
+                           dim3((unsigned)((ntmax + kSymBlock - 1) / kSymBlock), (unsigned)cq), dim3(64 * kFinWaves),
+                           0, s, items + q0);
+    }
+    return hipGetLastError();
+}
+
 template <int Q, int NL, bool CLAMP>
 static hipError_t cbie_t(const MeshDev& m, float k, const float2* psi, float2* lhs, int64_t ld, float2* rhs,
                          const CbieWork& w, int parts, hipStream_t s)
@@ -1913,13 +2087,13 @@ static hipError_t cbie_t(const MeshDev& m, float k, const float2* psi, float2* l
                            s, rec, m.tris, m.nt, k, psi, lhs, ld, w.prow, w.pcol, ntasks);
     }
     if (!(parts & 2)) return hipGetLastError();
-    const unsigned g = (unsigned)((m.npairs + 3) / 4);
-    hipLaunchKernelGGL((singular_kernel<DLP, NL, DP0, CLAMP, 0>), dim3(g), dim3(256), 0, s, m.geo, m.tris, m.curls,
-                       m.pairs, (int64_t)0, m.npairs, kbatch1(k), lhs, ld, (int64_t)0, -1.0f, nullptr, nullptr);
-    hipLaunchKernelGGL((singular_kernel<SLP, NL, DP0, CLAMP, 1>), dim3(g), dim3(256), 0, s, m.geo, m.tris, m.curls,
-                       m.pairs, (int64_t)0, m.npairs, kbatch1(k), lhs, ld, (int64_t)0, 1.0f, psi, w.vpsi);
-    hipLaunchKernelGGL(cbie_finalize_kernel, dim3(grid1d(m.nt)), dim3(256), 0, s, w.prow, w.pcol, w.nsub, w.vpsi,
-                       m.pair_ptr, m.geo, m.nt, lhs, ld, rhs);
+    const CbiePairItem it = cbie_pair_item(m, k, psi, lhs, ld, rhs, w);
+    const int64_t per = NL == 2 ? 16 : 4;  // pairs per workgroup
+    if (m.npairs > 0)
+        hipLaunchKernelGGL((cbie_pairs_kernel<NL, CLAMP>), dim3((unsigned)((m.npairs + per - 1) / per)), dim3(256), 0, s,
+                           it);
+    hipLaunchKernelGGL(cbie_finalize_kernel, dim3((unsigned)((m.nt + kSymBlock - 1) / kSymBlock)),
+                       dim3(64 * kFinWaves), 0, s, it);
     return hipGetLastError();
 }
 

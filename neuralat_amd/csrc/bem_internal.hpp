@@ -137,10 +137,33 @@ struct CbieWork {
     float2* vpsi;
     int nsub;
 };
+// The neighbour pairs and the row reduction of one fused CBIE system
+// (device-resident table of a batch, or a kernel argument).
+struct CbiePairItem {
+    const float* geo;
+    const int4* tris;
+    const int4* pairs;
+    const int64_t* pair_ptr;
+    int64_t npairs, nt;
+    float k;
+    int nsub;            // column partial slots per 64-row block
+    const float2* psi;
+    float2* lhs;
+    int64_t ld;
+    float2* rhs;
+    const float2* prow;
+    const float2* pcol;
+    float2* vpsi;
+    int64_t pair0;       // first wavefront of the item in the batch's pair launch
+};
 int64_t cbie_work_bytes(const MeshDev& m, int rt);
 CbieWork cbie_work_split(const MeshDev& m, int rt, void* work);
 hipError_t launch_cbie_dp0(const MeshDev& m, float k, int quad, int clamp, int parts, const float2* psi, float2* lhs,
                            int64_t ld, float2* rhs, const CbieWork& w, hipStream_t s);
+CbiePairItem cbie_pair_item(const MeshDev& m, float k, const float2* psi, float2* lhs, int64_t ld, float2* rhs,
+                            const CbieWork& w);
+hipError_t launch_batch_cbie_finish(const CbiePairItem* items, int nitems, int64_t nwaves, int64_t ntmax, int clamp,
+                                    hipStream_t s);
 int64_t adjoint_work_bytes(const MeshDev& m);
 hipError_t launch_adjoint_pairs(const MeshDev& m, float k, int clamp, const float2* lam, const float2* psi,
                                 const float2* phi, double* gvert, double* gk, double* vhl, void* work, hipStream_t s);
