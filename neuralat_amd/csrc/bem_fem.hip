@@ -118,10 +118,36 @@ __global__ __launch_bounds__(256) void fem_assemble_kernel(const float* __restri
 }
 
 // Y = A X for block-CSR A (3 x 3 blocks) and X, Y row-major [3 nv][m] with
-// leading dimensions ldx, ldy, all of type T (float or double).  One
-// wavefront per block row; lane j owns column j (columns beyond 64 in further
-// passes); the block values are wave-uniform loads, the X rows of a block
-// column are contiguous across lanes.
+// leading dimensions ldx, ldy, all of type T (float or double).  One wavefront
+// per block row, lane = column of X (columns beyond 64 in further passes).  The
+// row is wave-uniform, so its column indices and block values are scalar loads; the
+// gathered rows of X of up to kSpmmAhead blocks are requested before the first
+// is used (one block at a time, with the index and the values fetched by every
+// lane, the loop waited twice per block: 70 us for 18081 vertices x 48 columns
+// in FP64, 52 MB of matrix; now 29 us).  The workgroup numbers are dealt so that
+// each XCD takes a contiguous range of rows and finds its neighbours' rows of X
+// in its own L2 (workgroup b runs on XCD b % 8).  Summed in block order.
+constexpr int kSpmmAhead = 4;
+constexpr unsigned kXcds = 8;
+template <int U, typename T>
+__device__ __forceinline__ void fem_spmm_blocks(const int32_t* __restrict__ col, const T* __restrict__ A,
+                                                const T* __restrict__ Xj, int64_t ldx, T& y0, T& y1, T& y2)
+{
+    T x[U][3];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const T* xr = Xj + 3 * (int64_t)col[u] * ldx;
+        x[u][0] = xr[0];
+        x[u][1] = xr[ldx];
+        x[u][2] = xr[2 * ldx];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u, A += 9) {
+        y0 = fma(A[0], x[u][0], fma(A[1], x[u][1], fma(A[2], x[u][2], y0)));
+        y1 = fma(A[3], x[u][0], fma(A[4], x[u][1], fma(A[5], x[u][2], y1)));
+        y2 = fma(A[6], x[u][0], fma(A[7], x[u][1], fma(A[8], x[u][2], y2)));
+    }
+}
 template <typename T>
 __global__ __launch_bounds__(256) void fem_spmm_kernel(const int32_t* __restrict__ row_ptr,
                                                        const int32_t* __restrict__ col,
@@ -129,20 +155,23 @@ __global__ __launch_bounds__(256) void fem_spmm_kernel(const int32_t* __restrict
                                                        const T* __restrict__ X, int64_t ldx, int m,
                                                        T* __restrict__ Y, int64_t ldy)
 {
-    const int64_t u = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const unsigned per = gridDim.x / kXcds;  // the grid is a multiple of kXcds
+    const int64_t b = (int64_t)(blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
+    const int64_t u = b * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     if (u >= nv) return;
     const int lane = threadIdx.x & 63;
     const int32_t e0 = row_ptr[u], e1 = row_ptr[u + 1];
     for (int j = lane; j < m; j += 64) {
         T y0 = 0, y1 = 0, y2 = 0;
-        for (int32_t e = e0; e < e1; ++e) {
-            const T* A = values + (int64_t)e * 9;
-            const int64_t c = col[e];
-            const T x0 = X[(3 * c) * ldx + j], x1 = X[(3 * c + 1) * ldx + j], x2 = X[(3 * c + 2) * ldx + j];
-            y0 = fma(A[0], x0, fma(A[1], x1, fma(A[2], x2, y0)));
-            y1 = fma(A[3], x0, fma(A[4], x1, fma(A[5], x2, y1)));
-            y2 = fma(A[6], x0, fma(A[7], x1, fma(A[8], x2, y2)));
+        const T* Xj = X + j;
+        int32_t e = e0;
+        for (; e + kSpmmAhead <= e1; e += kSpmmAhead)
+            fem_spmm_blocks<kSpmmAhead>(col + e, values + (int64_t)e * 9, Xj, ldx, y0, y1, y2);
+        if (e + 2 <= e1) {
+            fem_spmm_blocks<2>(col + e, values + (int64_t)e * 9, Xj, ldx, y0, y1, y2);
+            e += 2;
         }
+        if (e < e1) fem_spmm_blocks<1>(col + e, values + (int64_t)e * 9, Xj, ldx, y0, y1, y2);
         Y[(3 * u) * ldy + j] = y0;
         Y[(3 * u + 1) * ldy + j] = y1;
         Y[(3 * u + 2) * ldy + j] = y2;
@@ -336,7 +365,7 @@ int bem_fem_spmm(const bem_fem* fem, int fp64, const void* values, const void* X
     if (!fem || !values || !X || !Y) return fem_fail(BEM_ERR_BAD_ARG, "null pointer");
     if (m <= 0 || ldx < m || ldy < m) return fem_fail(BEM_ERR_BAD_ARG, "bad shape");
     const FemDev& d = fem->dev;
-    const dim3 g((unsigned)((d.nv + 3) / 4));
+    const dim3 g((unsigned)(((d.nv + 3) / 4 + kXcds - 1) / kXcds * kXcds));
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if (fp64)
         hipLaunchKernelGGL(fem_spmm_kernel<double>, g, dim3(256), 0, s, d.row_ptr, d.col, (const double*)values, d.nv,
