@@ -658,10 +658,10 @@ namespace {
 size_t al(size_t b) { return (b + 255) / 256 * 256; }
 
 struct XLayout {
-    size_t sys, vec, V, w, r, b, x, H, h, h2, cs, sn, g, y, res, rn2, wn2, tgt, done, nk, conv, total;
+    size_t sys, vec, V, w, r, b, x, H, h, h2, cs, sn, g, y, part, partn, res, rn2, wn2, tgt, done, nk, conv, total;
 };
 
-XLayout xlayout(int ns, int64_t ntot, int m)
+XLayout xlayout(int ns, int64_t ntot, int64_t nmax, int m)
 {
     XLayout L{};
     size_t o = 0;
@@ -684,6 +684,8 @@ XLayout xlayout(int ns, int64_t ntot, int m)
     L.sn = take(sizeof(double2) * (size_t)ns * m);
     L.g = take(sizeof(double2) * (size_t)ns * (m + 1));
     L.y = take(sizeof(double2) * (size_t)ns * m);
+    L.part = take(sizeof(double2) * (size_t)arnoldi_part_elems(nmax, m, ns));
+    L.partn = take(sizeof(double) * (size_t)ns * (size_t)arnoldi_chunks(nmax));
     L.res = take(sizeof(double) * ns);
     L.rn2 = take(sizeof(double) * ns);
     L.wn2 = take(sizeof(double) * ns);
@@ -712,6 +714,7 @@ struct XEng {
     double2 *H = nullptr, *h = nullptr, *h2 = nullptr, *cs = nullptr, *sn = nullptr, *g = nullptr, *y = nullptr;
     double *res = nullptr, *rn2 = nullptr, *wn2 = nullptr, *tgt = nullptr;
     int *done = nullptr, *nk = nullptr, *conv = nullptr;
+    ArnoldiDesc D;
 };
 
 XEng xeng_at(char* W, const XLayout& L, const BSys* dsys, int ns, int64_t ntot, int64_t nmax, int m)
@@ -741,6 +744,26 @@ XEng xeng_at(char* W, const XLayout& L, const BSys* dsys, int ns, int64_t ntot, 
     E.done = (int*)(W + L.done);
     E.nk = (int*)(W + L.nk);
     E.conv = (int*)(W + L.conv);
+    ArnoldiDesc& D = E.D;
+    D.sys = dsys;
+    D.ns = ns;
+    D.m = m;
+    D.hs = m + 1;
+    D.n = nmax;
+    D.qstride = ntot;
+    D.V = E.V;
+    D.w = E.w;
+    D.H = E.H;
+    D.h = E.h;
+    D.cs = E.cs;
+    D.sn = E.sn;
+    D.g = E.g;
+    D.res = E.res;
+    D.wn2 = E.wn2;
+    D.target = E.tgt;
+    D.done = E.done;
+    D.nk = E.nk;
+    arnoldi_set_part(D, (double2*)(W + L.part), (double*)(W + L.partn));
     return E;
 }
 
@@ -796,43 +819,35 @@ hipError_t xcycle_init(const XEng& E, hipStream_t st)
     return hipGetLastError();
 }
 
-// Steps whose Gram-Schmidt reads at most this many basis entries per system
-// ((j + 1) n) run after the product as one launch, a workgroup per system
-// (launch_barnoldi_small); larger ones spread each system's dot products and
-// combination over many workgroups in separate launches.
-constexpr int64_t kXFusedStep = (int64_t)1 << 16;
-
-// Arnoldi steps [j0, j1): product, classical Gram-Schmidt with one
-// re-orthogonalisation, normalisation, Givens rotation and convergence flag
-hipError_t xcycle_steps(const XEng& E, int j0, int j1, hipStream_t st)
+// The rest of Arnoldi step j after the product w = A v_j (or A z_j): Gram-Schmidt
+// (passes: 1 or 2; with 1, h2 is zero), normalisation, Givens rotation,
+// convergence flag
+hipError_t xarnoldi(const XEng& E, int j, int passes, hipStream_t st)
 {
+    if (arnoldi_fused(E.D, j)) return launch_arnoldi_step(E.D, j, passes, st);
     const int m = E.m;
     const dim3 gx((unsigned)((E.nmax + 255) / 256), (unsigned)E.ns);
     const dim3 gc((unsigned)((E.nmax + 63) / 64), (unsigned)E.ns);
+    for (int pass = 0; pass < passes; ++pass) {
+        double2* h = pass ? E.h2 : E.h;
+        hipLaunchKernelGGL(xmultidot_kernel, dim3(j + 1, E.ns), dim3(256), 0, st, E.dsys, E.V, E.ntot, E.w, h, m + 1,
+                           (const int*)E.done);
+        hipLaunchKernelGGL(xcombine_kernel, gc, dim3(64 * kXWaves), 0, st, E.dsys, E.V, E.ntot, j + 1,
+                           (const int*)nullptr, h, m + 1, -1.0, E.w, (const int*)E.done);
+    }
+    hipLaunchKernelGGL(xnorm2_kernel, dim3(E.ns), dim3(256), 0, st, E.dsys, E.w, E.wn2);
+    hipLaunchKernelGGL(xnormalize_kernel, gx, dim3(256), 0, st, E.dsys, E.w, E.wn2, E.V + (int64_t)(j + 1) * E.ntot,
+                       (const int*)E.done);
+    return launch_bgivens(E.H, m, j, E.h, E.h2, m + 1, E.wn2, E.cs, E.sn, E.g, E.res, E.tgt, E.done, E.nk, E.ns, st);
+}
+
+// Arnoldi steps [j0, j1): product, then the rest of the step
+hipError_t xcycle_steps(const XEng& E, int j0, int j1, hipStream_t st)
+{
     for (int j = j0; j < j1; ++j) {
         hipError_t e = xmatvec(E, E.V + (int64_t)j * E.ntot, E.w, kOne, kZero, 1, E.done, st);
         if (e != hipSuccess) return e;
-        if ((int64_t)(j + 1) * E.nmax <= kXFusedStep) {  // small Gram-Schmidt: the rest of the step in one launch
-            e = launch_barnoldi_small(E.dsys, E.ns, E.V, E.ntot, j, E.w, E.h, E.h2, m + 1, E.H, m, E.cs, E.sn, E.g,
-                                      E.res, E.tgt, E.done, E.nk, E.wn2, E.one_pass ? 1 : 2, st);
-            if (e != hipSuccess) return e;
-            continue;
-        }
-        hipLaunchKernelGGL(xmultidot_kernel, dim3(j + 1, E.ns), dim3(256), 0, st, E.dsys, E.V, E.ntot, E.w, E.h,
-                           m + 1, (const int*)E.done);
-        hipLaunchKernelGGL(xcombine_kernel, gc, dim3(64 * kXWaves), 0, st, E.dsys, E.V, E.ntot, j + 1,
-                           (const int*)nullptr, E.h, m + 1, -1.0, E.w, (const int*)E.done);
-        if (!E.one_pass) {
-            hipLaunchKernelGGL(xmultidot_kernel, dim3(j + 1, E.ns), dim3(256), 0, st, E.dsys, E.V, E.ntot, E.w,
-                               E.h2, m + 1, (const int*)E.done);
-            hipLaunchKernelGGL(xcombine_kernel, gc, dim3(64 * kXWaves), 0, st, E.dsys, E.V, E.ntot, j + 1,
-                               (const int*)nullptr, E.h2, m + 1, -1.0, E.w, (const int*)E.done);
-        }
-        hipLaunchKernelGGL(xnorm2_kernel, dim3(E.ns), dim3(256), 0, st, E.dsys, E.w, E.wn2);
-        hipLaunchKernelGGL(xnormalize_kernel, gx, dim3(256), 0, st, E.dsys, E.w, E.wn2,
-                           E.V + (int64_t)(j + 1) * E.ntot, (const int*)E.done);
-        e = launch_bgivens(E.H, m, j, E.h, E.h2, m + 1, E.wn2, E.cs, E.sn, E.g, E.res, E.tgt, E.done, E.nk, E.ns,
-                           st);
+        e = xarnoldi(E, j, E.one_pass ? 1 : 2, st);
         if (e != hipSuccess) return e;
     }
     return hipGetLastError();
@@ -948,12 +963,14 @@ FLayout flayout(const bem_batch_system* sys, int ns, int64_t ntot, int mo, int m
 {
     FLayout F;
     size_t o = 0;
-    F.o = xlayout(ns, ntot, mo);
+    int64_t nmax = 0;
+    for (int q = 0; q < ns; ++q) nmax = std::max(nmax, sys[q].n);
+    F.o = xlayout(ns, ntot, nmax, mo);
     F.o_at = o;
     o += F.o.total;
     F.z_at = o;
     o += al(sizeof(float2) * (size_t)ntot * mo);
-    F.in = xlayout(ns, ntot, mi);
+    F.in = xlayout(ns, ntot, nmax, mi);
     F.in_at = o;
     o += F.in.total;
     F.low_at = o;
@@ -1140,8 +1157,12 @@ int64_t bem_batch_gmres_work_size(const bem_batch_system* sys, int ns, int resta
 {
     if (!sys || ns <= 0 || restart <= 0) return 0;
     int64_t ntot = 0;
-    for (int q = 0; q < ns; ++q) ntot += padded(sys[q].n);
-    return (int64_t)xlayout(ns, ntot, restart).total;
+    int64_t nmax = 0;
+    for (int q = 0; q < ns; ++q) {
+        ntot += padded(sys[q].n);
+        nmax = std::max(nmax, sys[q].n);
+    }
+    return (int64_t)xlayout(ns, ntot, nmax, restart).total;
 }
 
 static int check_systems(const bem_batch_system* sys, int ns, std::vector<BSys>& hs, int64_t& ntot, int64_t& nmax)
@@ -1198,7 +1219,7 @@ int bem_batch_gmres(const bem_batch_system* sys, int ns, float tol, int restart,
     std::vector<BSys> hs;
     int64_t ntot = 0, nmax = 0;
     if (int rc = check_systems(sys, ns, hs, ntot, nmax)) return rc;
-    const XLayout L = xlayout(ns, ntot, restart);
+    const XLayout L = xlayout(ns, ntot, nmax, restart);
     char* W = (char*)work;
     const XEng E = xeng_at(W, L, (const BSys*)(W + L.sys), ns, ntot, nmax, restart);
     std::vector<double> hb, hr(ns);
@@ -1343,20 +1364,7 @@ int bem_batch_fgmres(const bem_batch_system* sys, int ns, int dtype, float tol, 
             hipLaunchKernelGGL(xcopy_kernel, dim3((unsigned)((ntot + 255) / 256)), dim3(256), 0, s, Ei.X, zj, ntot);
             // w = A z_j in FP32, orthogonalised against the FP32 basis
             XTRY(xmatvec(Eo, zj, Eo.w, kOne, kZero, 1, Eo.done, s));
-            hipLaunchKernelGGL(xmultidot_kernel, dim3(j + 1, ns), dim3(256), 0, s, dsys, Eo.V, ntot, Eo.w, Eo.h,
-                               mo + 1, (const int*)Eo.done);
-            hipLaunchKernelGGL(xcombine_kernel, gc, dim3(64 * kXWaves), 0, s, dsys, Eo.V, ntot, j + 1,
-                               (const int*)nullptr, Eo.h, mo + 1, -1.0, Eo.w, (const int*)Eo.done);
-            hipLaunchKernelGGL(xmultidot_kernel, dim3(j + 1, ns), dim3(256), 0, s, dsys, Eo.V, ntot, Eo.w, Eo.h2,
-                               mo + 1, (const int*)Eo.done);
-            hipLaunchKernelGGL(xcombine_kernel, gc, dim3(64 * kXWaves), 0, s, dsys, Eo.V, ntot, j + 1,
-                               (const int*)nullptr, Eo.h2, mo + 1, -1.0, Eo.w, (const int*)Eo.done);
-            hipLaunchKernelGGL(xnorm2_kernel, dim3(ns), dim3(256), 0, s, dsys, Eo.w, Eo.wn2);
-            hipLaunchKernelGGL(xnormalize_kernel, gx, dim3(256), 0, s, dsys, Eo.w, Eo.wn2,
-                               Eo.V + (int64_t)(j + 1) * ntot, (const int*)Eo.done);
-            XTRY(hipGetLastError());
-            XTRY(launch_bgivens(Eo.H, mo, j, Eo.h, Eo.h2, mo + 1, Eo.wn2, Eo.cs, Eo.sn, Eo.g, Eo.res, Eo.tgt,
-                                Eo.done, Eo.nk, ns, s));
+            XTRY(xarnoldi(Eo, j, 2, s));
             XTRY(hipMemcpyAsync(hd.data(), Eo.done, sizeof(int) * ns, hipMemcpyDeviceToHost, s));
             XTRY(hipStreamSynchronize(s));
             bool alldone = true;

@@ -945,7 +945,29 @@ int bem_gmres_timed(const void* A_, int64_t n, int64_t lda, int trans, const voi
     int its = 0;
     double rnorm = 0.0, implicit = 0.0;
     bool conv = false;
-    const int chk = (n <= bem::kArnoldiSmallN && !timed) ? 8 : 1;  // steps per read of the residuals
+    // The implicit residuals are read every few steps (a read idles the GPU for
+    // about 20 us): up to chk steps at a time, fewer once the decay seen so far
+    // says the target is near.  Steps taken past convergence are dropped, so
+    // only their time is lost: long windows where a step costs no more than
+    // a read, none where a product takes hundreds of microseconds.
+    constexpr int kMaxWindow = 8;
+    const int chk = timed ? 1 : (n <= 4096 ? kMaxWindow : (n <= 12288 ? 4 : 1));
+    bem::ArnoldiDesc D;
+    D.m = m;
+    D.hs = m + 1;
+    D.n = D.qstride = n;
+    D.V = V;
+    D.w = w;
+    D.H = H;
+    D.h = h;
+    D.cs = cs;
+    D.sn = sn;
+    D.g = g;
+    D.wn2 = sc + 1;
+    // the step's partial sums: in the dot products' scratch (up to 8 chunks),
+    // beyond in the transposed product's, both idle then; r is idle between
+    // the cycle's start and its end
+    bem::arnoldi_set_part(D, bem::arnoldi_chunks(n) <= 8 ? hp : (double2*)tw, (double*)r);
     while (true) {
         // r = b - A x
         HIP_TRY(hipMemcpyAsync(r, b, sizeof(float2) * (size_t)n, hipMemcpyDeviceToDevice, s));
@@ -962,12 +984,14 @@ int bem_gmres_timed(const void* A_, int64_t n, int64_t lda, int trans, const voi
         if (its >= maxiter) break;
         HIP_TRY(bem::launch_normalize(r, n, sc, V, s));
         HIP_TRY(bem::launch_init_g(g, m, sc, s));
-        int nk = 0, checked = 0;
+        int nk = 0, checked = 0, window = chk;
+        double before = rnorm;  // the residual at the last read
         for (int j = 0; j < m && its < maxiter; ++j) {
             float2* vj = V + (size_t)j * n;
             HIP_TRY(gemv_timed(vj, w, one, zero));
-            if (n <= bem::kArnoldiSmallN) {  // launch-bound sizes: the step in one workgroup
-                HIP_TRY(bem::launch_arnoldi_small(V, n, j, w, h, h2, H, m, cs, sn, g, res, sc + 1, s));
+            D.res = res + j;
+            if (bem::arnoldi_fused(D, j)) {
+                HIP_TRY(bem::launch_arnoldi_step(D, j, 2, s));
             } else {
                 // classical Gram-Schmidt, twice
                 HIP_TRY(bem::launch_multidot(V, n, n, j + 1, w, h, hp, s));
@@ -980,15 +1004,13 @@ int bem_gmres_timed(const void* A_, int64_t n, int64_t lda, int trans, const voi
             }
             ++its;
             nk = j + 1;
-            // the implicit residuals are read every `chk` steps (small systems:
-            // the read is most of a step's time); on convergence the steps past
-            // the first converged one are dropped from the update (columns and
-            // g entries of earlier steps are final when a step ends), so the
-            // solution is the one of stopping there
+            // on convergence the steps past the first converged one are
+            // dropped from the update (columns and g entries of earlier steps
+            // are final when a step ends), so the solution is the one of
+            // stopping there
             const bool last = j + 1 == m || its >= maxiter;
-            if (nk - checked < chk && !last) continue;
-            // at most chk (<= 8) residuals per read: a fixed host array
-            double rs[8];
+            if (nk - checked < window && !last) continue;
+            double rs[kMaxWindow];
             const int nrs = nk - checked;
             HIP_TRY(hipMemcpyAsync(rs, res + checked, sizeof(double) * (size_t)nrs, hipMemcpyDeviceToHost, s));
             HIP_TRY(hipStreamSynchronize(s));
@@ -1005,6 +1027,13 @@ int bem_gmres_timed(const void* A_, int64_t n, int64_t lda, int trans, const voi
             }
             checked = nk;
             if (hit) break;
+            if (chk > 1) {
+                // steps to the target at the decay since the last read
+                const double rate = std::log(before / implicit) / nrs;
+                const double left = rate > 0.0 ? std::log(implicit / target) / rate : (double)chk;
+                window = (int)std::min<double>(chk, std::max(1.0, std::ceil(left)));
+                before = implicit;
+            }
         }
         HIP_TRY(bem::launch_backsolve(H, m, nk, g, y, s));
         HIP_TRY(bem::launch_update_x(V, n, n, nk, y, x, s));

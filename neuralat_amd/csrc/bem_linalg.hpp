@@ -77,11 +77,6 @@ hipError_t launch_dot(const float2* a, const float2* b, int64_t n, int conj, dou
 hipError_t launch_normalize(const float2* src, int64_t n, const double* nrm2, float2* out, hipStream_t s);
 hipError_t launch_givens(double2* H, int m, int j, const double2* h, const double2* h2, const double* wn2,
                          double2* cs, double2* sn, double2* g, double* res, hipStream_t s);
-// one Arnoldi step after w = A v_j (Gram-Schmidt twice, norm into *wn2,
-// v_{j+1}, Givens) in one workgroup, for systems of at most kArnoldiSmallN
-constexpr int64_t kArnoldiSmallN = 4096;
-hipError_t launch_arnoldi_small(float2* V, int64_t n, int j, float2* w, double2* h, double2* h2, double2* H, int m,
-                                double2* cs, double2* sn, double2* g, double* res, double* wn2, hipStream_t s);
 hipError_t launch_backsolve(const double2* H, int m, int nk, const double2* g, double2* y, hipStream_t s);
 hipError_t launch_update_x(const float2* V, int64_t ldv, int64_t n, int nk, const double2* y, float2* x,
                            hipStream_t s);
@@ -107,18 +102,43 @@ hipError_t launch_bgivens(double2* H, int m, int j, const double2* h, const doub
                           int ns, hipStream_t s);
 hipError_t launch_bbacksolve(const double2* H, int m, const int* nk, const double2* g, double2* y, int ns,
                              hipStream_t s);
-// One lockstep Arnoldi step after w = A v_j, one workgroup per system (meant
-// for small systems, whose steps are launch-bound): Gram-Schmidt (passes = 1
-// or 2; with 1, h2 is left as it is), |w|^2 into wn2, v_{j+1}, and the
-// Givens bookkeeping of launch_bgivens.  Vector q of system s at
-// V + q ntot + sys[s].off; h, h2 [ns, hs]; H [ns, (m + 1) m].
-hipError_t launch_barnoldi_small(const BSys* sys, int ns, float2* V, int64_t ntot, int j, float2* w, double2* h,
-                                 double2* h2, int hs, double2* H, int m, double2* cs, double2* sn, double2* g,
-                                 double* res, const double* target, int* done, int* nk, double* wn2, int passes,
-                                 hipStream_t s);
 hipError_t launch_bupdate_x(const float2* V, int64_t ldn, int ns, int64_t n, const int* nk, const double2* y, int m,
                             float2* x, int64_t ldx, hipStream_t s);
 hipError_t launch_bcopy(const float2* src, int64_t lds, float2* dst, int64_t ldd, int64_t n, int ns, hipStream_t s);
 hipError_t launch_badd(float2* x, int64_t ldx, const float2* d, int64_t ldd, int64_t n, int ns, hipStream_t s);
+
+// The state of a GMRES instance that an Arnoldi step works on (ns systems in
+// lockstep).  Basis vector q of system s starts at V + q qstride + off_s and w
+// at w + off_s, with off_s = sys[s].off and length sys[s].n when sys is given,
+// else s sstride and n.  n: the longest system.  H [ns, (m + 1) m], h [ns, hs]
+// (scratch), cs, sn [ns, m], g [ns, m + 1]; res, wn2 [ns].  With done, systems
+// whose flag is set are left alone and the flag is raised when the residual
+// estimate meets target; nk (with done) counts a system's steps.
+struct ArnoldiDesc {
+    const BSys* sys = nullptr;
+    int ns = 1, m = 0, hs = 0;
+    int64_t n = 0, qstride = 0, sstride = 0;
+    float2* V = nullptr;
+    float2* w = nullptr;
+    double2 *H = nullptr, *h = nullptr, *cs = nullptr, *sn = nullptr, *g = nullptr;
+    double *res = nullptr, *wn2 = nullptr;
+    const double* target = nullptr;
+    int *done = nullptr, *nk = nullptr;
+    // scratch of the chunked form (arnoldi_set_part)
+    int nch = 0, qcap = 0;
+    double2 *part = nullptr, *part2 = nullptr;
+    double* partn = nullptr;
+};
+// workgroups a system of n unknowns is cut into; basis vectors the chunked
+// form takes; its scratch: arnoldi_part_elems double2 and ns arnoldi_chunks(n)
+// doubles
+int arnoldi_chunks(int64_t n);
+int arnoldi_qcap(int64_t n, int m);
+int64_t arnoldi_part_elems(int64_t n, int m, int ns);
+void arnoldi_set_part(ArnoldiDesc& D, double2* part, double* partn);
+// whether step j has a fused form; the step itself after w = A v_j (passes: 1
+// or 2 Gram-Schmidt passes)
+bool arnoldi_fused(const ArnoldiDesc& D, int j);
+hipError_t launch_arnoldi_step(const ArnoldiDesc& D, int j, int passes, hipStream_t s);
 
 }  // namespace bem

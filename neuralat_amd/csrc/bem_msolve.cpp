@@ -20,6 +20,7 @@ namespace bem {
 
 namespace {
 size_t al(size_t b) { return (b + 255) / 256 * 256; }
+constexpr int kFirstWindow = 3, kMaxWindow = 8;  // steps per read of the convergence flags
 }  // namespace
 
 hipError_t MultiOp::apply(const float2* X, int64_t ldx, int ns, float2* Y, int64_t ldy, float2 alpha, float2 beta,
@@ -57,7 +58,7 @@ float2* lowp_scratch_part(void* scratch, int64_t ldlp)
 }
 
 struct MLayout {
-    size_t V, w, r, H, h, h2, cs, sn, g, y, res, rn2, wn2, tgt, done, nk, total;
+    size_t V, w, r, H, h, h2, cs, sn, g, y, part, partn, rn2, wn2, tgt, res, done, nk, total;
 };
 
 static MLayout mlayout(int64_t n, int ns, int m)
@@ -80,10 +81,13 @@ static MLayout mlayout(int64_t n, int ns, int m)
     L.sn = take(sizeof(double2) * (size_t)ns * m);
     L.g = take(sizeof(double2) * (size_t)ns * (m + 1));
     L.y = take(sizeof(double2) * (size_t)ns * m);
-    L.res = take(sizeof(double) * ns);
+    L.part = take(sizeof(double2) * (size_t)arnoldi_part_elems(n, m, ns));
+    L.partn = take(sizeof(double) * (size_t)ns * (size_t)arnoldi_chunks(n));
     L.rn2 = take(sizeof(double) * ns);
     L.wn2 = take(sizeof(double) * ns);
     L.tgt = take(sizeof(double) * ns);
+    // res, done, nk: read by the host in one copy
+    L.res = take(sizeof(double) * ns);
     L.done = take(sizeof(int) * ns);
     L.nk = take(sizeof(int) * ns);
     L.total = o;
@@ -123,8 +127,32 @@ hipError_t gmres_multi(const MultiOp& op, int64_t n, int ns, const float2* B, in
     int* nk = (int*)(W + L.nk);
     const float2 one = make_float2(1.f, 0.f), zero = make_float2(0.f, 0.f), mone = make_float2(-1.f, 0.f);
 
-    std::vector<double> hb(ns), ht(ns), hr(ns), hres(ns), irel(ns);
-    std::vector<int> hd(ns);
+    ArnoldiDesc D;
+    D.ns = ns;
+    D.m = m;
+    D.hs = m + 1;
+    D.n = n;
+    D.qstride = ldn * ns;
+    D.sstride = ldn;
+    D.V = V;
+    D.w = w;
+    D.H = H;
+    D.h = h;
+    D.cs = cs;
+    D.sn = sn;
+    D.g = g;
+    D.res = res;
+    D.wn2 = wn2;
+    D.target = tgt;
+    D.done = done;
+    D.nk = nk;
+    arnoldi_set_part(D, (double2*)(W + L.part), (double*)(W + L.partn));
+    // res, done and nk of every system, read by one copy
+    std::vector<char> hstate(L.total - L.res);
+    const double* hres = (const double*)hstate.data();
+    const int* hd = (const int*)(hstate.data() + (L.done - L.res));
+    const int* hk = (const int*)(hstate.data() + (L.nk - L.res));
+    std::vector<double> hb(ns), ht(ns), hr(ns), irel(ns), before(ns);
     TRY(launch_bnorm2(B, ldb, n, ns, rn2, s));
     TRY(hipMemcpyAsync(hb.data(), rn2, sizeof(double) * ns, hipMemcpyDeviceToHost, s));
     TRY(hipStreamSynchronize(s));
@@ -143,7 +171,13 @@ hipError_t gmres_multi(const MultiOp& op, int64_t n, int ns, const float2* B, in
         if (all_conv || its >= maxiter) break;
         TRY(launch_binit(g, m, rn2, tgt, done, nk, ns, s));
         TRY(launch_bnormalize(r, ldn, n, ns, rn2, V, ldn, nullptr, s));
-        for (int j = 0; j < m && its < maxiter; ++j) {
+        // The flags are read every few steps: a read idles the GPU for about
+        // 20 us, a step costs 50 us and more.  The systems' own step counts
+        // stop at convergence, so steps past it change nothing; the window is
+        // the number of steps the slowest system needs at the decay seen so far.
+        int checked = 0, window = prec ? 1 : kFirstWindow, steps = 0;
+        for (int q = 0; q < ns; ++q) before[q] = std::sqrt(hr[q]);
+        for (int j = 0; j < m && its + steps < maxiter; ++j) {
             const float2* Vj = V + (int64_t)j * ns * ldn;
             const float2* dir = Vj;
             if (prec) {
@@ -164,21 +198,40 @@ hipError_t gmres_multi(const MultiOp& op, int64_t n, int ns, const float2* B, in
                 dir = Zj;
             }
             TRY(op.apply(dir, ldn, ns, w, ldn, one, zero, s));
-            TRY(launch_bmultidot(V, ldn, ns, n, j + 1, w, h, m + 1, done, s));
-            TRY(launch_bgs_update(V, ldn, ns, n, j + 1, h, m + 1, w, done, s));
-            TRY(launch_bmultidot(V, ldn, ns, n, j + 1, w, h2, m + 1, done, s));
-            TRY(launch_bgs_update(V, ldn, ns, n, j + 1, h2, m + 1, w, done, s));
-            TRY(launch_bnorm2(w, ldn, n, ns, wn2, s));
-            TRY(launch_bnormalize(w, ldn, n, ns, wn2, V + (int64_t)(j + 1) * ns * ldn, ldn, done, s));
-            TRY(launch_bgivens(H, m, j, h, h2, m + 1, wn2, cs, sn, g, res, tgt, done, nk, ns, s));
-            ++its;
-            TRY(hipMemcpyAsync(hd.data(), done, sizeof(int) * ns, hipMemcpyDeviceToHost, s));
-            if (prec) TRY(hipMemcpyAsync(hres.data(), res, sizeof(double) * ns, hipMemcpyDeviceToHost, s));
+            if (arnoldi_fused(D, j)) {
+                TRY(launch_arnoldi_step(D, j, 2, s));
+            } else {
+                TRY(launch_bmultidot(V, ldn, ns, n, j + 1, w, h, m + 1, done, s));
+                TRY(launch_bgs_update(V, ldn, ns, n, j + 1, h, m + 1, w, done, s));
+                TRY(launch_bmultidot(V, ldn, ns, n, j + 1, w, h2, m + 1, done, s));
+                TRY(launch_bgs_update(V, ldn, ns, n, j + 1, h2, m + 1, w, done, s));
+                TRY(launch_bnorm2(w, ldn, n, ns, wn2, s));
+                TRY(launch_bnormalize(w, ldn, n, ns, wn2, V + (int64_t)(j + 1) * ns * ldn, ldn, done, s));
+                TRY(launch_bgivens(H, m, j, h, h2, m + 1, wn2, cs, sn, g, res, tgt, done, nk, ns, s));
+            }
+            ++steps;
+            const bool last = j + 1 == m || its + steps >= maxiter;
+            if (steps - checked < window && !last) continue;
+            TRY(hipMemcpyAsync(hstate.data(), res, hstate.size(), hipMemcpyDeviceToHost, s));
             TRY(hipStreamSynchronize(s));
             bool all = true;
-            for (int q = 0; q < ns; ++q) all = all && hd[q];
-            if (all) break;
+            double left = 1.0;
+            for (int q = 0; q < ns; ++q) {
+                all = all && hd[q];
+                if (hd[q] || prec) continue;
+                const double rate = std::log(before[q] / hres[q]) / (steps - checked);
+                left = std::max(left, rate > 0.0 ? std::log(hres[q] / ht[q]) / rate : (double)kMaxWindow);
+                before[q] = hres[q];
+            }
+            checked = steps;
+            if (!prec) window = (int)std::min<double>(kMaxWindow, std::ceil(left));
+            if (all) {
+                steps = 0;  // the steps the slowest system took
+                for (int q = 0; q < ns; ++q) steps = std::max(steps, hk[q]);
+                break;
+            }
         }
+        its += steps;
         TRY(launch_bbacksolve(H, m, nk, g, y, ns, s));
         TRY(launch_bupdate_x(prec ? prec->Z : V, ldn, ns, n, nk, y, m, X, ldx, s));
     }

@@ -1,0 +1,89 @@
+"""The fused Arnoldi step of the GMRES solvers (basis in LDS; chunked kernels;
+separate kernels beyond both) at the edges of its forms: 64-lane, 512-element
+chunk and LDS limits, step counts that cross from one form to the next, and
+systems of unequal length in lockstep.  Solutions against FP64 residuals and
+direct solves at the bars the solver tests use (1e-5)."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev():
+    return torch.device("cuda:0")
+
+
+def _system(n, radius, seed, nrhs=1):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    A = torch.randn(n, n, 2, generator=g, device=_dev())
+    A = torch.view_as_complex(A) * (radius / np.sqrt(2 * n))
+    A.diagonal().add_(1.0)
+    b = torch.view_as_complex(torch.randn(nrhs, n, 2, generator=g, device=_dev()))
+    return A.contiguous(), b.contiguous()
+
+
+def _err(A, x, b, adjoint=False):
+    """Relative residual in FP64."""
+    M = A.to(torch.complex128)
+    M = M.conj().T if adjoint else M
+    b = b.to(torch.complex128)
+    return float(torch.linalg.vector_norm(b - M @ x.to(torch.complex128)) / torch.linalg.vector_norm(b))
+
+
+@pytest.mark.parametrize("n,radius,restart", [(1, 0.0, 5), (2, 0.3, 5), (63, 0.5, 60), (512, 0.5, 60), (513, 0.7, 60),
+                                              (1100, 0.7, 60), (4097, 0.6, 40)])
+def test_single_system(n, radius, restart):
+    from neuralat_amd.bem.grad import _adjoint_solve
+    from neuralat_amd.bem.solver import gmres
+
+    print("arnoldi single", n, restart, flush=True)
+    A, b = _system(n, radius, n)
+    x, info = gmres(A, b[0], tol=1e-6, restart=restart, maxiter=1000)
+    assert info["converged"], info
+    assert _err(A, x, b[0]) < 2e-6, info
+    if n in (513, 4097):  # the adjoint product's scratch is shared with the step's
+        y, info = _adjoint_solve(A, b[0], 1e-6, restart, 1000)
+        assert info["converged"] and _err(A, y, b[0], adjoint=True) < 2e-6, info
+
+
+def test_long_basis():
+    """Steps past the chunked form's partial sums (18 chunks: 227 steps) take
+    the separate kernels.  The target is 1e-5: such a slowly converging
+    system's FP32 residual bottoms out near 1e-6."""
+    from neuralat_amd.bem.solver import gmres
+
+    print("arnoldi long basis", flush=True)
+    A, b = _system(9000, 0.98, 9)
+    x, info = gmres(A, b[0], tol=1e-5, restart=400, maxiter=1000)
+    assert info["converged"] and 227 < info["iterations"] <= 400, info
+    assert _err(A, x, b[0]) < 1.2e-5, info
+
+
+@pytest.mark.parametrize("n,nrhs", [(65, 3), (700, 17), (5000, 2)])
+def test_many_right_hand_sides(n, nrhs):
+    from neuralat_amd.bem.precision import gmres_multi
+
+    print("arnoldi multi", n, nrhs, flush=True)
+    A, B = _system(n, 0.6, n, nrhs)
+    X, infos = gmres_multi(A, B, tol=1e-6, restart=50)
+    assert all(i["converged"] for i in infos)
+    for q in range(nrhs):
+        assert _err(A, X[q], B[q]) < 2e-6, q
+
+
+@pytest.mark.parametrize("use_graph", [True, False])
+def test_uneven_lockstep(use_graph):
+    from neuralat_amd.bem.batch import batch_gmres, batch_solve_mixed
+
+    sizes = (1, 40, 513, 700, 2100)
+    print("arnoldi lockstep", use_graph, flush=True)
+    systems = [_system(n, 0.6, n) for n in sizes]
+    As, bs = [a for a, _ in systems], [b[0] for _, b in systems]
+    xs, infos = batch_gmres(As, bs, tol=1e-6, restart=20, max_cycles=30, use_graph=use_graph)
+    for n, A, b, x, i in zip(sizes, As, bs, xs, infos):
+        assert i["converged"] and _err(A, x, b) < 2e-6, (n, i)
+    xs, infos = batch_solve_mixed(As, bs, dtype="fp16", tol=1e-6, inner_tol=1e-3, inner_restart=30, max_inner_cycles=1,
+                                  max_outer_cycles=6, use_graph=use_graph)
+    for n, A, b, x, i in zip(sizes, As, bs, xs, infos):
+        assert i["converged"] and _err(A, x, b) < 2e-6, (n, i)
