@@ -3,10 +3,8 @@
 
 #include <cmath>
 #include <algorithm>
-#include <cstring>
-#include <mutex>
+#include <new>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "../../include/bem_hip.h"
@@ -142,7 +140,7 @@ int bem_mesh_create(const float* verts, int64_t nv, const int32_t* tris, int64_t
     bem_mesh* m = new (std::nothrow) bem_mesh();
     if (!m) return fail(BEM_ERR_OOM, "host allocation failed");
     std::string err;
-    int rc = bem::mesh_build(pv, nv, pt, nt, m->dev, err);
+    int rc = bem::mesh_build(pv, nv, pt, nt, S(stream), m->dev, err);
     if (rc != 0) {
         delete m;
         return fail(rc, err);
@@ -157,16 +155,8 @@ int bem_mesh_set_vertices(bem_mesh* mesh, const float* verts, int on_device, voi
     auto& m = mesh->dev;
     DeviceGuard g(m.device);
     if (!g.ok) return fail(BEM_ERR_HIP, "cannot select the mesh's device");
-    std::vector<float> hv;
-    const float* pv = verts;
-    if (on_device) {
-        hv.resize((size_t)m.nv * 3);
-        HIP_TRY(hipMemcpyAsync(hv.data(), verts, hv.size() * 4, hipMemcpyDeviceToHost, S(stream)));
-        HIP_TRY(hipStreamSynchronize(S(stream)));
-        pv = hv.data();
-    }
     std::string err;
-    const int rc = bem::mesh_set_vertices(m, pv, S(stream), err);
+    const int rc = bem::mesh_set_vertices(m, verts, on_device != 0, S(stream), err);
     if (rc != 0) return fail(rc == 3 ? BEM_ERR_HIP : (rc == 1 ? BEM_ERR_BAD_ARG : BEM_ERR_BAD_MESH), err);
     return BEM_OK;
 }
@@ -337,104 +327,24 @@ struct bem_geomset {
     void* block = nullptr;
 };
 
-// Pinned host staging for geometry-set uploads (a DMA copy instead of a
-// staged pageable one: 9.6 MB of 48 two-sphere samples took 0.5-1 ms
-// pageable).  One process-wide buffer, grown on demand up to
-// kPinnedStageMax and kept until the process ends; larger sets stage in
-// pageable memory.  g_stage_mu is held from the first write to the end of
-// the copy.
-static constexpr size_t kPinnedStageMax = (size_t)64 << 20;
-static std::mutex g_stage_mu;
-static char* g_stage = nullptr;
-static size_t g_stage_cap = 0;
-
 int bem_geomset_create(const bem_mesh* mesh, const float* verts, int ns, void* stream, bem_geomset** out)
 {
     if (!mesh || !verts || !out) return fail(BEM_ERR_BAD_ARG, "null pointer");
     *out = nullptr;
     if (ns < 1) return fail(BEM_ERR_BAD_ARG, "need at least one sample");
     const auto& m = mesh->dev;
-    const size_t gb = m.geom_bytes;
     DeviceGuard g(m.device);
     if (!g.ok) return fail(BEM_ERR_HIP, "cannot select the mesh's device");
-    const size_t bytes = gb * (size_t)ns;
-    std::unique_lock<std::mutex> lk(g_stage_mu, std::defer_lock);
-    char* host = nullptr;
-    std::vector<char> pageable;
-    if (bytes <= kPinnedStageMax) {
-        lk.lock();
-        if (g_stage_cap < bytes) {
-            if (g_stage) (void)hipHostFree(g_stage);
-            g_stage = nullptr;
-            g_stage_cap = 0;
-            const size_t want = std::min(kPinnedStageMax, (bytes + ((size_t)1 << 20) - 1) >> 20 << 20);
-            if (hipHostMalloc((void**)&g_stage, want, hipHostMallocDefault) == hipSuccess) {
-                g_stage_cap = want;
-            } else {
-                (void)hipGetLastError();
-                g_stage = nullptr;
-            }
-        }
-        if (g_stage) host = g_stage;
-        else lk.unlock();
-    }
-    if (!host) {
-        pageable.resize(bytes);
-        host = pageable.data();
-    }
-    // Each sample's geometry is independent host work (quadrature records,
-    // curls): up to 16 threads, each on an interleaved share of the samples.
-    std::vector<int> rcs((size_t)ns, 0);
-    std::vector<std::string> errs((size_t)ns);
-    auto work = [&](int t0, int step) {
-        for (int z = t0; z < ns; z += step)
-            rcs[z] = bem::mesh_geometry_region(m, verts + (size_t)z * 3 * (size_t)m.nv, host + z * gb, errs[z]);
-    };
-    const int nth = (int)std::min<int64_t>({(int64_t)ns, 16, (int64_t)std::max(1u, std::thread::hardware_concurrency()),
-                                            std::max<int64_t>(1, (int64_t)ns * m.nt / 4096)});
-    if (nth <= 1) {
-        work(0, 1);
-    } else {
-        // a thread that cannot be started (std::system_error) leaves its
-        // share to this one: no exception crosses the C ABI
-        std::vector<std::thread> pool;
-        int started = 1;
-        try {
-            pool.reserve(nth - 1);
-            for (; started < nth; ++started) pool.emplace_back(work, started, nth);
-        } catch (...) {
-        }
-        work(0, nth);
-        for (int t = started; t < nth; ++t) work(t, nth);
-        for (auto& th : pool) th.join();
-    }
-    for (int z = 0; z < ns; ++z)
-        if (rcs[z])
-            return fail(rcs[z] == 2 ? BEM_ERR_BAD_MESH : BEM_ERR_BAD_ARG, "sample " + std::to_string(z) + ": " + errs[z]);
-    auto* gs = new bem_geomset();
-    if (hipMalloc(&gs->block, bytes) != hipSuccess) {
-        (void)hipGetLastError();
+    auto* gs = new (std::nothrow) bem_geomset();
+    if (!gs) return fail(BEM_ERR_OOM, "host allocation failed");
+    std::string err;
+    if (const int rc = bem::geomset_build(m, verts, ns, S(stream), gs->view, &gs->block, err)) {
         delete gs;
-        return fail(BEM_ERR_OOM, "device allocation of " + std::to_string(bytes) + " bytes failed");
-    }
-    hipError_t e = hipMemcpyAsync(gs->block, host, bytes, hipMemcpyHostToDevice, S(stream));
-    if (e == hipSuccess) e = hipStreamSynchronize(S(stream));
-    if (e != hipSuccess) {
-        (void)hipFree(gs->block);
-        delete gs;
-        return hip_fail(e, "bem_geomset_create copy");
+        return fail(rc, err);
     }
     gs->mesh = mesh;
     gs->ns = ns;
-    gs->gstride = (int64_t)(gb / sizeof(float));
-    gs->view = m;
-    auto rebase = [&](float*& p) { p = (float*)((char*)gs->block + ((char*)p - (char*)m.block)); };
-    rebase(gs->view.verts);
-    rebase(gs->view.rec6);
-    rebase(gs->view.rec3);
-    rebase(gs->view.rec1);
-    rebase(gs->view.curls);
-    rebase(gs->view.geo);
+    gs->gstride = (int64_t)(m.geom_bytes / sizeof(float));
     *out = gs;
     return BEM_OK;
 }

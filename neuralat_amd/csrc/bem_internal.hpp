@@ -75,8 +75,7 @@ struct MeshDev {
     std::vector<int64_t> h_pair_ptr;  // [nt+1] host copy: pair range of each row triangle
     int64_t h_row_slots = 0;          // total vertex slots of the row tiles (tiles.row_vptr[nrow_tiles])
     int32_t max_neighbors = 0;
-    double diameter = 0.0;  // bounding-box diagonal
-    std::vector<int32_t> h_tris;  // [nt*3] host copy (for mesh_set_vertices)
+    unsigned long long* geom_flag = nullptr;  // one word for checks of new positions
     size_t geom_bytes = 0;  // the position-dependent arrays: the first geom_bytes of block
     void* block = nullptr;  // the single device allocation
 };
@@ -222,17 +221,22 @@ hipError_t launch_field(const MeshDev& mg, int64_t gstride, const float* pts, in
                         const float* ks, int nk, int basis, int clamp, const float2* psi, const float2* phi,
                         float2* out, void* work, hipStream_t s);
 
-// Builds all device data from host copies of the mesh; returns 0 or a
-// bem_status code with a message in `err`.
-int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t nt, MeshDev& m, std::string& err);
-// New vertex positions for a built mesh (same triangles): recomputes the
-// position-dependent arrays on the host and uploads them in one copy on s,
-// then waits for it.  Connectivity data and the tiling are kept.
-int mesh_set_vertices(MeshDev& m, const float* h_verts, hipStream_t s, std::string& err);
-// The position-dependent region of m (the first m.geom_bytes of its block:
-// vertices, quadrature records, curls, singular-pair geometry) for new
-// positions h_verts [nv, 3] of the same triangles, written to region (host).
-int mesh_geometry_region(const MeshDev& m, const float* h_verts, char* region, std::string& err);
+// Builds all device data from host copies of the mesh (uploads and the geometry
+// kernel on stream, waited for); returns 0 or a bem_status code with a message
+// in `err`.
+int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t nt, hipStream_t stream, MeshDev& m,
+               std::string& err);
+// New vertex positions (host or device) for a built mesh (same triangles):
+// checked, then the position-dependent arrays recomputed by a kernel on s, which
+// is waited for.  Connectivity data and the tiling are kept; after a fault so
+// are the old positions.
+int mesh_set_vertices(MeshDev& m, const float* verts, bool on_device, hipStream_t s, std::string& err);
+// ns placements h_verts [ns, nv, 3] (host) of m's triangles: one allocation
+// *block with a copy of m's position-dependent region (geom_bytes) per sample,
+// filled on s, which is waited for; view = m with its position-dependent
+// pointers at sample 0.
+int geomset_build(const MeshDev& m, const float* h_verts, int ns, hipStream_t s, MeshDev& view, void** block,
+                  std::string& err);
 void mesh_free(MeshDev& m);
 
 }  // namespace bem

@@ -1,15 +1,19 @@
-// Host-side mesh preprocessing: validation, per-triangle quadrature records,
-// surface curls, neighbour pairs, vertex->triangle lists and the P1 tiling.
+// Mesh set-up: validation, neighbour pairs, vertex->triangle lists and the P1
+// tiling on the host; the position-dependent arrays (quadrature records,
+// surface curls, singular-pair geometry) by a kernel from the vertex positions.
 //
 // The reference recomputes normals and curls in torch (solver.py:40-58) and
 // finds neighbour pairs with an O(N) scan per triangle inside the singular
 // kernel (bind.cu:90-97); here they are built once per mesh in O(N log N).
+// The lists are made by counting and stamping (sorting the pairs by kind and
+// searching the tiles' vertex lists took most of 4.4 ms at 5120 triangles),
+// and what is uploaded goes through one pinned buffer.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <numeric>
+#include <mutex>
 #include <vector>
 
 #include "bem_device.hpp"
@@ -22,35 +26,15 @@ namespace {
 struct V3 {
     double x, y, z;
 };
-inline V3 sub(V3 a, V3 b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
-inline V3 add(V3 a, V3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
-inline V3 mul(double s, V3 a) { return {s * a.x, s * a.y, s * a.z}; }
-inline double dot(V3 a, V3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
-inline V3 cross(V3 a, V3 b) { return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x}; }
-
-// quadrature rules in double (same points as the device TriRule<Q>)
-struct HostRule {
-    std::vector<double> x1, x2, w;
-};
-HostRule host_rule(int q)
+// no fused multiply-adds: host and device round alike
+#pragma clang fp contract(off)
+__host__ __device__ inline V3 sub(V3 a, V3 b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
+__host__ __device__ inline V3 add(V3 a, V3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
+__host__ __device__ inline V3 mul(double s, V3 a) { return {s * a.x, s * a.y, s * a.z}; }
+__host__ __device__ inline double dot(V3 a, V3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+__host__ __device__ inline V3 cross(V3 a, V3 b)
 {
-    HostRule r;
-    if (q == 6) {
-        const double a = 0.445948490915965, b = 0.091576213509771;
-        const double wa = 0.223381589678011, wb = 0.109951743655322;
-        r.x1 = {a, b, 1 - 2 * a, a, 1 - 2 * b, b};
-        r.x2 = {a, b, a, 1 - 2 * a, b, 1 - 2 * b};
-        r.w = {wa, wb, wa, wa, wb, wb};
-    } else if (q == 3) {
-        r.x1 = {1.0 / 6, 2.0 / 3, 1.0 / 6};
-        r.x2 = {1.0 / 6, 1.0 / 6, 2.0 / 3};
-        r.w = {1.0 / 3, 1.0 / 3, 1.0 / 3};
-    } else {
-        r.x1 = {1.0 / 3};
-        r.x2 = {1.0 / 3};
-        r.w = {1.0};
-    }
-    return r;
+    return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
 }
 
 uint32_t spread10(uint32_t v)
@@ -71,7 +55,7 @@ struct Tiling {
 // Greedy tiling of the ordered triangle list: a tile closes when it holds
 // max_tris triangles, one more would exceed max_verts distinct vertices, or
 // the next position is in stops (sorted; tiles never cross one).
-Tiling make_tiling(const std::vector<int32_t>& perm, const int32_t* tris, int max_tris, int max_verts,
+Tiling make_tiling(const std::vector<int32_t>& perm, const int32_t* tris, int64_t nv, int max_tris, int max_verts,
                    const std::vector<int32_t>& stops = {})
 {
     Tiling T;
@@ -79,143 +63,240 @@ Tiling make_tiling(const std::vector<int32_t>& perm, const int32_t* tris, int ma
     T.slot.assign((size_t)nt * 4, 0);
     T.ptr.push_back(0);
     T.vptr.push_back(0);
+    T.verts.reserve((size_t)nt * 2);
     int64_t pos = 0;
     std::vector<int32_t> local;
+    // tile (plus 1) a vertex was last seen in, and its slot there
+    std::vector<int32_t> seen((size_t)nv, 0), slot((size_t)nv, 0);
+    int32_t tile = 0;
     size_t next_stop = 0;
     while (pos < nt) {
+        ++tile;
         local.clear();
         int64_t start = pos;
         while (next_stop < stops.size() && stops[next_stop] <= start) ++next_stop;
         const int64_t limit = next_stop < stops.size() ? std::min<int64_t>(nt, stops[next_stop]) : nt;
         while (pos < limit && pos - start < max_tris) {
             const int32_t* t = tris + 3 * (int64_t)perm[pos];
-            int fresh = 0;
-            for (int a = 0; a < 3; ++a)
-                if (std::find(local.begin(), local.end(), t[a]) == local.end()) ++fresh;
+            const int fresh = (seen[t[0]] != tile) + (seen[t[1]] != tile) + (seen[t[2]] != tile);
             if ((int)local.size() + fresh > max_verts) break;
             for (int a = 0; a < 3; ++a)
-                if (std::find(local.begin(), local.end(), t[a]) == local.end()) local.push_back(t[a]);
+                if (seen[t[a]] != tile) {
+                    seen[t[a]] = tile;
+                    local.push_back(t[a]);
+                }
             ++pos;
         }
-        std::vector<int32_t> sorted = local;
-        std::sort(sorted.begin(), sorted.end());
+        std::sort(local.begin(), local.end());
+        for (size_t q = 0; q < local.size(); ++q) slot[local[q]] = (int32_t)q;
         for (int64_t p = start; p < pos; ++p) {
             const int32_t* t = tris + 3 * (int64_t)perm[p];
-            for (int a = 0; a < 3; ++a)
-                T.slot[4 * p + a] = (int32_t)(std::lower_bound(sorted.begin(), sorted.end(), t[a]) - sorted.begin());
+            for (int a = 0; a < 3; ++a) T.slot[4 * p + a] = slot[t[a]];
         }
-        T.verts.insert(T.verts.end(), sorted.begin(), sorted.end());
+        T.verts.insert(T.verts.end(), local.begin(), local.end());
         T.ptr.push_back((int32_t)pos);
         T.vptr.push_back((int32_t)T.verts.size());
     }
     return T;
 }
 
-}  // namespace
+// Pinned host staging for uploads (a DMA copy instead of a staged pageable
+// one: 1 MB takes 27 us against 140 to 315).  One process-wide buffer, grown
+// on demand up to kPinnedStageMax and kept until the process ends; larger
+// uploads stage in pageable memory.  The lock is held until the copy is done.
+constexpr size_t kPinnedStageMax = (size_t)64 << 20;
+std::mutex g_stage_mu;
+char* g_stage = nullptr;
+size_t g_stage_cap = 0;
 
-// Position-dependent host data of a mesh: quadrature records, P1 curls,
-// singular-kernel geometry, centroids, bounding-box diagonal (FP64, rounded
-// once).  Fails on non-finite coordinates and zero-area triangles.
-struct HostGeom {
-    std::vector<float> rec6, rec3, rec1, curls, geo;
-    std::vector<V3> cent;
-    V3 lo{0.0, 0.0, 0.0}, hi{0.0, 0.0, 0.0};  // bounding box
-    double diameter = 0.0;
+class Stage {
+public:
+    char* get(size_t bytes)
+    {
+        if (bytes <= kPinnedStageMax) {
+            lk_ = std::unique_lock<std::mutex>(g_stage_mu);
+            if (g_stage_cap < bytes) {
+                if (g_stage) (void)hipHostFree(g_stage);
+                g_stage = nullptr;
+                g_stage_cap = 0;
+                const size_t want = std::min(kPinnedStageMax, (bytes + ((size_t)1 << 20) - 1) >> 20 << 20);
+                if (hipHostMalloc((void**)&g_stage, want, hipHostMallocDefault) == hipSuccess) {
+                    g_stage_cap = want;
+                } else {
+                    (void)hipGetLastError();
+                    g_stage = nullptr;
+                }
+            }
+            if (g_stage) return g_stage;
+            lk_.unlock();
+        }
+        pageable_.resize(bytes);
+        return pageable_.data();
+    }
+
+private:
+    std::unique_lock<std::mutex> lk_;
+    std::vector<char> pageable_;
 };
 
-static int build_geometry(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t nt, HostGeom& g,
-                          std::string& err)
-{
-    for (int64_t v = 0; v < 3 * nv; ++v)
-        if (!std::isfinite(h_verts[v])) {
-            err = "non-finite vertex coordinate";
-            return 2;
-        }
-    constexpr int S6 = Rec<6>::kFloats, S3 = Rec<3>::kFloats, S1 = Rec<1>::kFloats;
-    g.rec6.assign((size_t)nt * S6, 0.f);
-    g.rec3.assign((size_t)nt * S3, 0.f);
-    g.rec1.assign((size_t)nt * S1, 0.f);
-    g.curls.assign((size_t)nt * 12, 0.f);
-    g.geo.assign((size_t)nt * 16, 0.f);
-    g.cent.assign((size_t)nt, V3{0.0, 0.0, 0.0});
-    auto& rec6 = g.rec6;
-    auto& rec3 = g.rec3;
-    auto& rec1 = g.rec1;
-    auto& curls = g.curls;
-    auto& geo = g.geo;
-    auto& cent = g.cent;
-    const HostRule R6 = host_rule(6), R3 = host_rule(3), R1 = host_rule(1);
-    V3 lo{1e300, 1e300, 1e300}, hi{-1e300, -1e300, -1e300};
-    for (int64_t v = 0; v < nv; ++v) {
-        lo.x = std::min(lo.x, (double)h_verts[3 * v]);
-        hi.x = std::max(hi.x, (double)h_verts[3 * v]);
-        lo.y = std::min(lo.y, (double)h_verts[3 * v + 1]);
-        hi.y = std::max(hi.y, (double)h_verts[3 * v + 1]);
-        lo.z = std::min(lo.z, (double)h_verts[3 * v + 2]);
-        hi.z = std::max(hi.z, (double)h_verts[3 * v + 2]);
-    }
-    g.diameter = std::sqrt(dot(sub(hi, lo), sub(hi, lo)));
-    g.lo = lo;
-    g.hi = hi;
-    for (int64_t t = 0; t < nt; ++t) {
-        const int32_t* tr = h_tris + 3 * t;
-        V3 v[3];
-        for (int a = 0; a < 3; ++a) {
-            v[a] = {h_verts[3 * (int64_t)tr[a]], h_verts[3 * (int64_t)tr[a] + 1], h_verts[3 * (int64_t)tr[a] + 2]};
-        }
-        const V3 e1 = sub(v[1], v[0]), e2 = sub(v[2], v[0]);
-        const V3 c = cross(e1, e2);
-        const double J = std::sqrt(dot(c, c));
-        if (!(J > 0.0) || !std::isfinite(J)) {
-            err = "triangle " + std::to_string(t) + " has zero area";
-            return 2;
-        }
-        const V3 n = mul(1.0 / J, c);
-        cent[t] = mul(1.0 / 3.0, add(add(v[0], v[1]), v[2]));
-        auto fill = [&](float* r, const HostRule& R) {
-            const int Q = (int)R.w.size();
-            for (int q = 0; q < Q; ++q) {
-                const V3 p = add(v[0], add(mul(R.x1[q], e1), mul(R.x2[q], e2)));
-                r[3 * q] = (float)p.x;
-                r[3 * q + 1] = (float)p.y;
-                r[3 * q + 2] = (float)p.z;
-                r[3 * Q + q] = (float)(R.w[q] * 0.5 * J);
-            }
-            r[4 * Q] = (float)n.x;
-            r[4 * Q + 1] = (float)n.y;
-            r[4 * Q + 2] = (float)n.z;
-        };
-        fill(&rec6[(size_t)t * S6], R6);
-        fill(&rec3[(size_t)t * S3], R3);
-        fill(&rec1[(size_t)t * S1], R1);
-        // P1 surface curls: row a = n x grad(phi_a), grad from the dual basis
-        const double g11 = dot(e1, e1), g12 = dot(e1, e2), g22 = dot(e2, e2);
-        const double det = g11 * g22 - g12 * g12;
-        const V3 b1 = add(mul(g22 / det, e1), mul(-g12 / det, e2));
-        const V3 b2 = add(mul(-g12 / det, e1), mul(g11 / det, e2));
-        const V3 grad[3] = {mul(-1.0, add(b1, b2)), b1, b2};
-        for (int a = 0; a < 3; ++a) {
-            const V3 cu = cross(n, grad[a]);
-            curls[(size_t)t * 12 + 3 * a] = (float)cu.x;
-            curls[(size_t)t * 12 + 3 * a + 1] = (float)cu.y;
-            curls[(size_t)t * 12 + 3 * a + 2] = (float)cu.z;
-        }
-        float* gr = &geo[(size_t)t * 16];
-        for (int a = 0; a < 3; ++a) {
-            gr[3 * a] = (float)v[a].x;
-            gr[3 * a + 1] = (float)v[a].y;
-            gr[3 * a + 2] = (float)v[a].z;
-        }
-        gr[9] = (float)n.x;
-        gr[10] = (float)n.y;
-        gr[11] = (float)n.z;
-        gr[12] = (float)J;
-    }
+}  // namespace
 
-    return 0;
+// A fault of one sample's positions: kind 0 = a non-finite coordinate, 1 = a
+// triangle of zero area; the first (kind, triangle) is kept as the smallest key.
+constexpr unsigned long long kGeomOk = ~0ull;
+static __host__ __device__ inline unsigned long long geom_key(int kind, int64_t t)
+{
+    return ((unsigned long long)kind << 32) | (unsigned long long)t;
+}
+static std::string geom_fault(unsigned long long key)
+{
+    return (key >> 32) == 0 ? "non-finite vertex coordinate"
+                            : "triangle " + std::to_string((int64_t)(key & 0xffffffffu)) + " has zero area";
 }
 
-int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t nt, MeshDev& m, std::string& err)
+__device__ __forceinline__ void load_triangle(const float* __restrict__ verts, int4 tr, V3 (&v)[3])
+{
+    const int id[3] = {tr.x, tr.y, tr.z};
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const float* p = verts + 3 * (int64_t)id[a];
+        v[a] = {p[0], p[1], p[2]};
+    }
+}
+
+// keys[z] = the first fault of sample z (verts + z vstride), kGeomOk without one
+// (every vertex belongs to a triangle, so the triangles see every coordinate)
+__global__ __launch_bounds__(256) void geometry_check_kernel(const float* __restrict__ verts, int64_t vstride,
+                                                             const int4* __restrict__ tris, int64_t nt,
+                                                             unsigned long long* __restrict__ keys)
+{
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= nt) return;
+    V3 v[3];
+    load_triangle(verts + (int64_t)blockIdx.y * vstride, tris[t], v);
+    bool finite = true;
+    for (int a = 0; a < 3; ++a) finite = finite && isfinite(v[a].x) && isfinite(v[a].y) && isfinite(v[a].z);
+    const V3 c = cross(sub(v[1], v[0]), sub(v[2], v[0]));
+    const double J = sqrt(dot(c, c));
+    if (!finite) atomicMin(&keys[blockIdx.y], geom_key(0, t));
+    else if (!(J > 0.0) || !isfinite(J)) atomicMin(&keys[blockIdx.y], geom_key(1, t));
+}
+
+template <int Q>
+__device__ __forceinline__ void write_record(float* __restrict__ r, V3 v0, V3 e1, V3 e2, V3 n, double J)
+{
+    // the device rules' points in double
+    constexpr double a = 0.445948490915965, b = 0.091576213509771;
+    constexpr double wa = 0.223381589678011, wb = 0.109951743655322;
+    constexpr double x6[6] = {a, b, 1 - 2 * a, a, 1 - 2 * b, b}, y6[6] = {a, b, a, 1 - 2 * a, b, 1 - 2 * b};
+    constexpr double w6[6] = {wa, wb, wa, wa, wb, wb};
+    constexpr double x3[3] = {1.0 / 6, 2.0 / 3, 1.0 / 6}, y3[3] = {1.0 / 6, 1.0 / 6, 2.0 / 3};
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const double x1 = Q == 6 ? x6[q] : (Q == 3 ? x3[q % 3] : 1.0 / 3);
+        const double x2 = Q == 6 ? y6[q] : (Q == 3 ? y3[q % 3] : 1.0 / 3);
+        const double w = Q == 6 ? w6[q] : (Q == 3 ? 1.0 / 3 : 1.0);
+        const V3 p = add(v0, add(mul(x1, e1), mul(x2, e2)));
+        r[3 * q] = (float)p.x;
+        r[3 * q + 1] = (float)p.y;
+        r[3 * q + 2] = (float)p.z;
+        r[3 * Q + q] = (float)(w * 0.5 * J);
+    }
+    r[4 * Q] = (float)n.x;
+    r[4 * Q + 1] = (float)n.y;
+    r[4 * Q + 2] = (float)n.z;
+#pragma unroll
+    for (int e = 4 * Q + 3; e < Rec<Q>::kFloats; ++e) r[e] = 0.f;
+}
+
+// The position-dependent arrays of every sample from its vertices (FP64,
+// rounded once); sample z's arrays lie gstride floats further on.  One thread
+// per triangle: a few hundred bytes written each, microseconds per mesh (the
+// host loop and the upload of its 368 bytes per triangle took 0.7 ms for 48
+// samples of 640 triangles on 16 threads).
+__global__ __launch_bounds__(256) void geometry_kernel(const int4* __restrict__ tris, int64_t nt, int64_t gstride,
+                                                       const float* __restrict__ verts, float* __restrict__ rec6,
+                                                       float* __restrict__ rec3, float* __restrict__ rec1,
+                                                       float* __restrict__ curls, float* __restrict__ geo)
+{
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= nt) return;
+    const int64_t off = (int64_t)blockIdx.y * gstride;
+    V3 v[3];
+    load_triangle(verts + off, tris[t], v);
+    const V3 e1 = sub(v[1], v[0]), e2 = sub(v[2], v[0]);
+    const V3 c = cross(e1, e2);
+    const double J = sqrt(dot(c, c));
+    const V3 n = mul(1.0 / J, c);
+    write_record<6>(rec6 + off + t * Rec<6>::kFloats, v[0], e1, e2, n, J);
+    write_record<3>(rec3 + off + t * Rec<3>::kFloats, v[0], e1, e2, n, J);
+    write_record<1>(rec1 + off + t * Rec<1>::kFloats, v[0], e1, e2, n, J);
+    // P1 surface curls: row a = n x grad(phi_a), grad from the dual basis
+    const double g11 = dot(e1, e1), g12 = dot(e1, e2), g22 = dot(e2, e2);
+    const double det = g11 * g22 - g12 * g12;
+    const V3 b1 = add(mul(g22 / det, e1), mul(-g12 / det, e2));
+    const V3 b2 = add(mul(-g12 / det, e1), mul(g11 / det, e2));
+    const V3 grad[3] = {mul(-1.0, add(b1, b2)), b1, b2};
+    float* cu = curls + off + t * 12;
+    float* gr = geo + off + t * 16;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const V3 w = cross(n, grad[a]);
+        cu[3 * a] = (float)w.x;
+        cu[3 * a + 1] = (float)w.y;
+        cu[3 * a + 2] = (float)w.z;
+        gr[3 * a] = (float)v[a].x;
+        gr[3 * a + 1] = (float)v[a].y;
+        gr[3 * a + 2] = (float)v[a].z;
+    }
+    cu[9] = cu[10] = cu[11] = 0.f;
+    gr[9] = (float)n.x;
+    gr[10] = (float)n.y;
+    gr[11] = (float)n.z;
+    gr[12] = (float)J;
+    gr[13] = gr[14] = gr[15] = 0.f;
+}
+
+static hipError_t launch_geometry(const MeshDev& g, int64_t gstride, int ns, hipStream_t s)
+{
+    for (int z0 = 0; z0 < ns; z0 += 65535) {  // grid y limit
+        const int64_t off = (int64_t)z0 * gstride;
+        hipLaunchKernelGGL(geometry_kernel, dim3((unsigned)((g.nt + 255) / 256), (unsigned)std::min(65535, ns - z0)),
+                           dim3(256), 0, s, g.tris, g.nt, gstride, g.verts + off, g.rec6 + off, g.rec3 + off,
+                           g.rec1 + off, g.curls + off, g.geo + off);
+    }
+    return hipGetLastError();
+}
+
+static hipError_t launch_geometry_check(const float* verts, int64_t vstride, int ns, const int4* tris, int64_t nt,
+                                        unsigned long long* keys, hipStream_t s)
+{
+    hipError_t e = hipMemsetAsync(keys, 0xff, sizeof(*keys) * (size_t)ns, s);
+    if (e != hipSuccess) return e;
+    for (int z0 = 0; z0 < ns; z0 += 65535)
+        hipLaunchKernelGGL(geometry_check_kernel, dim3((unsigned)((nt + 255) / 256), (unsigned)std::min(65535, ns - z0)),
+                           dim3(256), 0, s, verts + (int64_t)z0 * vstride, vstride, tris, nt, keys + z0);
+    return hipGetLastError();
+}
+
+// host check of a mesh's positions (the same faults)
+static unsigned long long check_positions(const float* v, int64_t nv, const int32_t* tris, int64_t nt)
+{
+    for (int64_t e = 0; e < 3 * nv; ++e)
+        if (!std::isfinite(v[e])) return geom_key(0, 0);
+    for (int64_t t = 0; t < nt; ++t) {
+        const float *a = v + 3 * (int64_t)tris[3 * t], *b = v + 3 * (int64_t)tris[3 * t + 1],
+                    *c = v + 3 * (int64_t)tris[3 * t + 2];
+        const V3 n = cross({(double)b[0] - a[0], (double)b[1] - a[1], (double)b[2] - a[2]},
+                           {(double)c[0] - a[0], (double)c[1] - a[1], (double)c[2] - a[2]});
+        const double J = std::sqrt(dot(n, n));
+        if (!(J > 0.0) || !std::isfinite(J)) return geom_key(1, t);
+    }
+    return kGeomOk;
+}
+
+int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t nt, hipStream_t stream, MeshDev& m,
+               std::string& err)
 {
     if (nv < 3 || nt < 1) {
         err = "mesh needs at least 3 vertices and 1 triangle";
@@ -240,20 +321,13 @@ int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t 
     m.nv = nv;
     m.nt = nt;
 
-    HostGeom hg;
-    if (int rc = build_geometry(h_verts, nv, h_tris, nt, hg, err)) return rc;
-    m.diameter = hg.diameter;
-    const auto& rec6 = hg.rec6;
-    const auto& rec3 = hg.rec3;
-    const auto& rec1 = hg.rec1;
-    const auto& curls = hg.curls;
-    const auto& geo = hg.geo;
-    const auto& cent = hg.cent;
-    const V3 lo = hg.lo, hi = hg.hi;
+    if (const unsigned long long key = check_positions(h_verts, nv, h_tris, nt); key != kGeomOk) {
+        err = geom_fault(key);
+        return 2;
+    }
     std::vector<int32_t> tris4((size_t)nt * 4, 0);
     for (int64_t t = 0; t < nt; ++t)
         for (int a = 0; a < 3; ++a) tris4[4 * t + a] = h_tris[3 * t + a];
-    m.h_tris.assign(h_tris, h_tris + 3 * nt);
 
     // ---- vertex -> triangle CSR ----
     std::vector<int32_t> vt_ptr((size_t)nv + 1, 0), vt_idx((size_t)nt * 3), vt_corner((size_t)nt * 3);
@@ -275,63 +349,94 @@ int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t 
         }
 
     // ---- neighbour pairs (share >= 1 vertex, self included) ----
-    std::vector<int32_t> pairs;
-    pairs.reserve((size_t)nt * 14 * 4);
+    struct Pair {
+        int32_t i, j, shared, pad;
+    };
+    std::vector<Pair> pairs;
+    pairs.reserve((size_t)nt * 14);
     m.h_pair_ptr.assign((size_t)nt + 1, 0);
-    std::vector<int32_t> cand;
     int32_t maxnb = 0;
-    for (int64_t t = 0; t < nt; ++t) {
-        cand.clear();
-        for (int a = 0; a < 3; ++a) {
-            const int32_t v = h_tris[3 * t + a];
-            cand.insert(cand.end(), vt_idx.begin() + vt_ptr[v], vt_idx.begin() + vt_ptr[v + 1]);
-        }
-        std::sort(cand.begin(), cand.end());
-        cand.erase(std::unique(cand.begin(), cand.end()), cand.end());
-        maxnb = std::max(maxnb, (int32_t)cand.size());
-        for (int32_t u : cand) {
-            int s = 0;
-            for (int a = 0; a < 3; ++a)
-                for (int b = 0; b < 3; ++b) s += (h_tris[3 * t + a] == h_tris[3 * (int64_t)u + b]);
-            if (s == 3 && u != t) {
-                err = "triangles " + std::to_string(t) + " and " + std::to_string(u) + " share all three vertices";
-                return 2;
+    int64_t kinds[4] = {0, 0, 0, 0};
+    {
+        // triangles around t's corners, counted: a triangle met s times shares s vertices
+        std::vector<int32_t> seen((size_t)nt, -1), at((size_t)nt, 0);
+        std::vector<std::pair<int32_t, int32_t>> cand;  // (triangle, vertices shared)
+        for (int64_t t = 0; t < nt; ++t) {
+            cand.clear();
+            for (int a = 0; a < 3; ++a) {
+                const int32_t v = h_tris[3 * t + a];
+                for (int32_t q = vt_ptr[v]; q < vt_ptr[v + 1]; ++q) {
+                    const int32_t u = vt_idx[q];
+                    if (seen[u] != (int32_t)t) {
+                        seen[u] = (int32_t)t;
+                        at[u] = (int32_t)cand.size();
+                        cand.push_back({u, 1});
+                    } else {
+                        ++cand[at[u]].second;
+                    }
+                }
             }
-            pairs.push_back((int32_t)t);
-            pairs.push_back(u);
-            pairs.push_back(s);
-            pairs.push_back(0);
+            std::sort(cand.begin(), cand.end());
+            maxnb = std::max(maxnb, (int32_t)cand.size());
+            for (const auto& [u, s] : cand) {
+                if (s == 3 && u != t) {
+                    err = "triangles " + std::to_string(t) + " and " + std::to_string(u) + " share all three vertices";
+                    return 2;
+                }
+                pairs.push_back({(int32_t)t, u, s, 0});
+                ++kinds[s];
+            }
+            m.h_pair_ptr[t + 1] = (int64_t)pairs.size();
         }
-        m.h_pair_ptr[t + 1] = (int64_t)pairs.size() / 4;
     }
-    m.npairs = (int64_t)pairs.size() / 4;
+    m.npairs = (int64_t)pairs.size();
     // the P1 neighbour-pair launches take every pair in any order: grouped by
     // kind, the pairs that share a wavefront take the same quadrature branch
-    std::vector<int32_t> pairs_kind(pairs.size());
+    std::vector<Pair> pairs_kind(pairs.size());
     {
-        std::vector<int64_t> idx((size_t)m.npairs);
-        std::iota(idx.begin(), idx.end(), (int64_t)0);
-        std::stable_sort(idx.begin(), idx.end(), [&](int64_t a, int64_t b) { return pairs[4 * a + 2] > pairs[4 * b + 2]; });
-        for (int64_t q = 0; q < m.npairs; ++q)
-            for (int c = 0; c < 4; ++c) pairs_kind[4 * q + c] = pairs[4 * idx[q] + c];
+        int64_t next[4] = {0, kinds[3] + kinds[2], kinds[3], 0};
+        for (const Pair& p : pairs) pairs_kind[(size_t)next[p.shared]++] = p;
     }
     m.max_neighbors = maxnb;
 
     // ---- P1 tiling on a Morton order of the centroids ----
     std::vector<int32_t> perm((size_t)nt);
     {
-        std::vector<uint32_t> code((size_t)nt);
+        V3 lo{1e300, 1e300, 1e300}, hi{-1e300, -1e300, -1e300};
+        for (int64_t v = 0; v < nv; ++v) {
+            const V3 p{h_verts[3 * v], h_verts[3 * v + 1], h_verts[3 * v + 2]};
+            lo = {std::min(lo.x, p.x), std::min(lo.y, p.y), std::min(lo.z, p.z)};
+            hi = {std::max(hi.x, p.x), std::max(hi.y, p.y), std::max(hi.z, p.z)};
+        }
         const double sx = hi.x - lo.x > 0 ? 1023.0 / (hi.x - lo.x) : 0.0;
         const double sy = hi.y - lo.y > 0 ? 1023.0 / (hi.y - lo.y) : 0.0;
         const double sz = hi.z - lo.z > 0 ? 1023.0 / (hi.z - lo.z) : 0.0;
+        // (code, triangle) keys sorted by three passes of ten bits (stable)
+        struct Key {
+            uint32_t code;
+            int32_t t;
+        };
+        std::vector<Key> key((size_t)nt), tmp((size_t)nt);
         for (int64_t t = 0; t < nt; ++t) {
-            const uint32_t ix = (uint32_t)((cent[t].x - lo.x) * sx);
-            const uint32_t iy = (uint32_t)((cent[t].y - lo.y) * sy);
-            const uint32_t iz = (uint32_t)((cent[t].z - lo.z) * sz);
-            code[t] = spread10(ix) | (spread10(iy) << 1) | (spread10(iz) << 2);
+            V3 v[3];
+            for (int a = 0; a < 3; ++a) {
+                const float* p = h_verts + 3 * (int64_t)h_tris[3 * t + a];
+                v[a] = {p[0], p[1], p[2]};
+            }
+            const V3 c = mul(1.0 / 3.0, add(add(v[0], v[1]), v[2]));
+            const uint32_t ix = (uint32_t)((c.x - lo.x) * sx);
+            const uint32_t iy = (uint32_t)((c.y - lo.y) * sy);
+            const uint32_t iz = (uint32_t)((c.z - lo.z) * sz);
+            key[t] = {spread10(ix) | (spread10(iy) << 1) | (spread10(iz) << 2), (int32_t)t};
         }
-        std::iota(perm.begin(), perm.end(), 0);
-        std::stable_sort(perm.begin(), perm.end(), [&](int32_t a, int32_t b) { return code[a] < code[b]; });
+        for (int shift = 0; shift < 30; shift += 10) {
+            std::vector<int32_t> first(1025, 0);
+            for (const Key& k : key) ++first[((k.code >> shift) & 1023) + 1];
+            for (int q = 0; q < 1024; ++q) first[q + 1] += first[q];
+            for (const Key& k : key) tmp[(size_t)first[(k.code >> shift) & 1023]++] = k;
+            key.swap(tmp);
+        }
+        for (int64_t t = 0; t < nt; ++t) perm[t] = key[t].t;
     }
     // P1 numbering: vertices in the order they first appear along the Morton
     // order of the triangles, so the vertices of a tile are (nearly)
@@ -356,8 +461,8 @@ int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t 
     for (int64_t e = 0; e < 3 * nt; ++e) tris_p1[e] = vnew[h_tris[e]];
     // row tiles nest in column tiles, so the symmetric sweep can pair a row
     // tile with the column tiles from its own on
-    const Tiling colT = make_tiling(perm, tris_p1.data(), kP1ColTris, kP1ColVerts);
-    const Tiling rowT = make_tiling(perm, tris_p1.data(), kP1RowTris, kP1RowVerts, colT.ptr);
+    const Tiling colT = make_tiling(perm, tris_p1.data(), nv, kP1ColTris, kP1ColVerts);
+    const Tiling rowT = make_tiling(perm, tris_p1.data(), nv, kP1RowTris, kP1RowVerts, colT.ptr);
     const int nrowt = (int)rowT.ptr.size() - 1, ncolt = (int)colT.ptr.size() - 1;
     std::vector<int32_t> row_ctile((size_t)nrowt);
     std::vector<int64_t> sym_ptr((size_t)nrowt + 1, 0);
@@ -391,20 +496,19 @@ int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t 
         void** dst;
     };
     std::vector<Part> parts;
+    // the position-dependent arrays first, one contiguous region that
+    // geometry_kernel fills from the vertices at its start
     float* d_verts = nullptr;
-    std::vector<float> vcopy(h_verts, h_verts + 3 * nv);
-    // the position-dependent arrays first: mesh_set_vertices rewrites them as
-    // one contiguous region
-    parts.push_back({vcopy.data(), vcopy.size() * 4, (void**)&d_verts});
-    parts.push_back({rec6.data(), rec6.size() * 4, (void**)&m.rec6});
-    parts.push_back({rec3.data(), rec3.size() * 4, (void**)&m.rec3});
-    parts.push_back({rec1.data(), rec1.size() * 4, (void**)&m.rec1});
-    parts.push_back({curls.data(), curls.size() * 4, (void**)&m.curls});
-    parts.push_back({geo.data(), geo.size() * 4, (void**)&m.geo});
+    parts.push_back({h_verts, (size_t)nv * 12, (void**)&d_verts});
+    parts.push_back({nullptr, (size_t)nt * Rec<6>::kFloats * 4, (void**)&m.rec6});
+    parts.push_back({nullptr, (size_t)nt * Rec<3>::kFloats * 4, (void**)&m.rec3});
+    parts.push_back({nullptr, (size_t)nt * Rec<1>::kFloats * 4, (void**)&m.rec1});
+    parts.push_back({nullptr, (size_t)nt * 12 * 4, (void**)&m.curls});
+    parts.push_back({nullptr, (size_t)nt * 16 * 4, (void**)&m.geo});
     constexpr size_t kGeomParts = 6;
     parts.push_back({tris4.data(), tris4.size() * 4, (void**)&m.tris});
-    parts.push_back({pairs.data(), pairs.size() * 4, (void**)&m.pairs});
-    parts.push_back({pairs_kind.data(), pairs_kind.size() * 4, (void**)&m.pairs_by_kind});
+    parts.push_back({pairs.data(), pairs.size() * sizeof(Pair), (void**)&m.pairs});
+    parts.push_back({pairs_kind.data(), pairs_kind.size() * sizeof(Pair), (void**)&m.pairs_by_kind});
     parts.push_back({m.h_pair_ptr.data(), m.h_pair_ptr.size() * 8, (void**)&m.pair_ptr});
     parts.push_back({vt_ptr.data(), vt_ptr.size() * 4, (void**)&m.vt_ptr});
     parts.push_back({vt_idx.data(), vt_idx.size() * 4, (void**)&m.vt_idx});
@@ -427,6 +531,7 @@ int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t 
     parts.push_back({sym_ptr.data(), sym_ptr.size() * 8, (void**)&d_sym});
     parts.push_back({vnew.data(), vnew.size() * 4, (void**)&m.p1_vnew});
     parts.push_back({vold.data(), vold.size() * 4, (void**)&m.p1_vold});
+    parts.push_back({nullptr, sizeof(unsigned long long), (void**)&m.geom_flag});
     size_t total = 0;
     std::vector<size_t> off;
     for (auto& p : parts) {
@@ -443,20 +548,32 @@ int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t 
         (void)hipGetLastError();
         return 6;
     }
-    // every array through one host staging buffer and one copy (a copy per
-    // array cost more than the rest of the set-up for small meshes)
-    std::vector<char> stage(total);
-    for (size_t q = 0; q < parts.size(); ++q) {
-        *parts[q].dst = (char*)m.block + off[q];
-        if (parts[q].bytes) std::memcpy(stage.data() + off[q], parts[q].src, parts[q].bytes);
-    }
-    if (hipMemcpy(m.block, stage.data(), total, hipMemcpyHostToDevice) != hipSuccess) {
-        err = "host to device copy failed";
-        (void)hipFree(m.block);
-        m.block = nullptr;
-        return 3;
-    }
+    // the vertices, then every connectivity array, through one host staging
+    // buffer and two copies (a copy per array cost more than the rest of the
+    // set-up for small meshes)
+    for (size_t q = 0; q < parts.size(); ++q) *parts[q].dst = (char*)m.block + off[q];
     m.verts = d_verts;
+    {
+        Stage st;
+        const size_t head = ((size_t)nv * 12 + 255) / 256 * 256, conn = off[kGeomParts];
+        char* host = st.get(head + (total - conn));
+        std::memcpy(host, h_verts, (size_t)nv * 12);
+        for (size_t q = kGeomParts; q < parts.size(); ++q)
+            if (parts[q].src && parts[q].bytes) std::memcpy(host + head + (off[q] - conn), parts[q].src, parts[q].bytes);
+        hipError_t e = hipMemcpyAsync(m.block, host, (size_t)nv * 12, hipMemcpyHostToDevice, stream);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync((char*)m.block + conn, host + head, total - conn, hipMemcpyHostToDevice, stream);
+        if (e == hipSuccess) e = launch_geometry(m, 0, 1, stream);
+        // the handle may be used on any stream from here on
+        const hipError_t es = hipStreamSynchronize(stream);
+        if (e == hipSuccess) e = es;
+        if (e != hipSuccess) {
+            err = std::string("mesh upload: ") + hipGetErrorString(e);
+            (void)hipFree(m.block);
+            m.block = nullptr;
+            return 3;
+        }
+    }
     m.tiles.perm = d_perm;
     m.tiles.row_ptr = d_rp;
     m.tiles.row_vptr = d_rvp;
@@ -477,44 +594,104 @@ int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t 
     return 0;
 }
 
-int mesh_geometry_region(const MeshDev& m, const float* h_verts, char* region, std::string& err)
+// the position-dependent pointers of m moved from its own block to region
+static void rebase_geometry(MeshDev& g, const MeshDev& m, void* region)
 {
-    if (!m.block || m.h_tris.size() != (size_t)m.nt * 3) {
+    auto at = [&](float* p) { return (float*)((char*)region + ((char*)p - (char*)m.block)); };
+    g.verts = at(m.verts);
+    g.rec6 = at(m.rec6);
+    g.rec3 = at(m.rec3);
+    g.rec1 = at(m.rec1);
+    g.curls = at(m.curls);
+    g.geo = at(m.geo);
+}
+
+int geomset_build(const MeshDev& m, const float* h_verts, int ns, hipStream_t s, MeshDev& view, void** block,
+                  std::string& err)
+{
+    const size_t vb = (size_t)m.nv * 12, bytes = m.geom_bytes * (size_t)ns;
+    const size_t key_at = (bytes + 255) / 256 * 256;
+    *block = nullptr;
+    if (hipMalloc(block, key_at + sizeof(unsigned long long) * (size_t)ns) != hipSuccess) {
+        (void)hipGetLastError();
+        err = "device allocation of " + std::to_string(bytes) + " bytes failed";
+        return 6;
+    }
+    view = m;
+    rebase_geometry(view, m, *block);
+    unsigned long long* keys = (unsigned long long*)((char*)*block + key_at);
+    std::vector<unsigned long long> hk((size_t)ns, kGeomOk);
+    hipError_t e;
+    {
+        Stage st;
+        char* host = st.get(vb * (size_t)ns);
+        std::memcpy(host, h_verts, vb * (size_t)ns);
+        // the vertices lead each sample's region
+        e = hipMemcpy2DAsync(*block, m.geom_bytes, host, vb, vb, (size_t)ns, hipMemcpyHostToDevice, s);
+        const int64_t gstride = (int64_t)(m.geom_bytes / sizeof(float));
+        if (e == hipSuccess) e = launch_geometry_check(view.verts, gstride, ns, m.tris, m.nt, keys, s);
+        if (e == hipSuccess) e = launch_geometry(view, gstride, ns, s);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(hk.data(), keys, sizeof(hk[0]) * hk.size(), hipMemcpyDeviceToHost, s);
+        const hipError_t es = hipStreamSynchronize(s);
+        if (e == hipSuccess) e = es;
+    }
+    int rc = 0;
+    if (e != hipSuccess) {
+        err = std::string("geometry set: ") + hipGetErrorString(e);
+        rc = 3;
+    }
+    for (int z = 0; z < ns && rc == 0; ++z)
+        if (hk[z] != kGeomOk) {
+            err = "sample " + std::to_string(z) + ": " + geom_fault(hk[z]);
+            rc = 2;
+        }
+    if (rc) {
+        (void)hipFree(*block);
+        *block = nullptr;
+    }
+    return rc;
+}
+
+int mesh_set_vertices(MeshDev& m, const float* verts, bool on_device, hipStream_t s, std::string& err)
+{
+    if (!m.block) {
         err = "mesh has no device data";
         return 1;
     }
-    HostGeom hg;
-    if (int rc = build_geometry(h_verts, m.nv, m.h_tris.data(), m.nt, hg, err)) return rc;
-    // the same 256-byte aligned layout as mesh_build's first six parts
-    const std::pair<const float*, size_t> sec[6] = {{h_verts, (size_t)m.nv * 3},   {hg.rec6.data(), hg.rec6.size()},
-                                                    {hg.rec3.data(), hg.rec3.size()}, {hg.rec1.data(), hg.rec1.size()},
-                                                    {hg.curls.data(), hg.curls.size()}, {hg.geo.data(), hg.geo.size()}};
-    std::memset(region, 0, m.geom_bytes);
-    size_t off = 0;
-    for (const auto& q : sec) {
-        const size_t bytes = q.second * 4;
-        if (off + bytes > m.geom_bytes) {
-            err = "geometry layout mismatch";
-            return 1;
+    const size_t vb = (size_t)m.nv * 12;
+    Stage st;
+    void* tmp = nullptr;
+    const float* src = verts;
+    hipError_t e = hipSuccess;
+    if (!on_device) {  // checked on the device as well: through a temporary
+        e = hipMallocAsync(&tmp, vb, s);
+        if (e == hipSuccess) {
+            char* host = st.get(vb);
+            std::memcpy(host, verts, vb);
+            e = hipMemcpyAsync(tmp, host, vb, hipMemcpyHostToDevice, s);
+            src = (const float*)tmp;
         }
-        std::memcpy(region + off, q.first, bytes);
-        off += (bytes + 255) / 256 * 256;
     }
-    if (off != m.geom_bytes) {
-        err = "geometry layout mismatch";
-        return 1;
+    unsigned long long key = kGeomOk;
+    if (e == hipSuccess) e = launch_geometry_check(src, 0, 1, m.tris, m.nt, m.geom_flag, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(&key, m.geom_flag, sizeof(key), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e == hipSuccess && key == kGeomOk) {
+        e = hipMemcpyAsync(m.verts, src, vb, hipMemcpyDeviceToDevice, s);
+        if (e == hipSuccess) e = launch_geometry(m, 0, 1, s);
     }
-    return 0;
-}
-
-int mesh_set_vertices(MeshDev& m, const float* h_verts, hipStream_t s, std::string& err)
-{
-    std::vector<char> stage(m.geom_bytes, 0);
-    if (int rc = mesh_geometry_region(m, h_verts, stage.data(), err)) return rc;
-    if (hipMemcpyAsync(m.block, stage.data(), stage.size(), hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess) {
-        err = "host to device copy failed";
+    if (tmp) (void)hipFreeAsync(tmp, s);
+    // other streams may use the new positions from here on
+    const hipError_t es = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = es;
+    if (e != hipSuccess) {
+        err = std::string("set_vertices: ") + hipGetErrorString(e);
         return 3;
+    }
+    if (key != kGeomOk) {
+        err = geom_fault(key);
+        return 2;
     }
     return 0;
 }

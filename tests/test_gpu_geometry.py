@@ -1,0 +1,68 @@
+"""The geometry kernel (normals, curls and records from the vertices) and its
+checks, on meshes around its 256-triangle workgroups.  The arrays are FP64
+values rounded once, so they match numpy's to one FP32 rounding."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from neuralat_amd import _lib, mesh
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev():
+    return torch.device("cuda:0")
+
+
+def _normals_curls(v, t):
+    e = v[t].astype(np.float64)
+    c = np.cross(e[:, 1] - e[:, 0], e[:, 2] - e[:, 0])
+    J = np.linalg.norm(c, axis=1)
+    curls = np.stack([e[:, 1] - e[:, 2], e[:, 2] - e[:, 0], e[:, 0] - e[:, 1]], 1) / J[:, None, None]
+    return c / J[:, None], curls
+
+
+@pytest.mark.parametrize("nt", [1, 255, 256, 257, 320])
+def test_normals_and_curls(nt):
+    from neuralat_amd.bem import Mesh
+
+    v, t = mesh.icosphere(2, 0.1)
+    v = mesh.sh_perturb(v, 4, 0.05, seed=nt).astype(np.float32)
+    t = t[:nt]
+    used, t = np.unique(t, return_inverse=True)
+    v, t = v[used], t.reshape(-1, 3).astype(np.int32)
+    print("geometry", nt, flush=True)
+    m = Mesh(torch.tensor(v, device=_dev()), torch.tensor(t, device=_dev()))
+    moved = (v * np.float32(1.7) + np.float32(0.3)).astype(np.float32)
+    for x, source in ((v, None), (moved, "device"), (v, "host")):
+        if source == "device":
+            m.set_vertices(torch.tensor(x, device=_dev()))
+        elif source == "host":
+            _lib.check(_lib.load().bem_mesh_set_vertices(m.handle, x.ctypes.data, 0, ctypes.c_void_p(0)))
+        n, c = (a.cpu().numpy() for a in m.normals_curls())
+        rn, rc = _normals_curls(x, t)
+        assert np.abs(n - rn).max() < 1.2e-7
+        assert np.abs(c - rc).max() < 1.2e-7 * np.abs(rc).max()
+
+
+def test_faults_are_reported_and_change_nothing():
+    from neuralat_amd.bem import GeometrySet, Mesh
+
+    v, t = mesh.icosphere(1, 0.1)
+    v = v.astype(np.float32)
+    nan, flat = v.copy(), v.copy()
+    nan[7, 1] = np.nan
+    flat[t[5, 1]] = flat[t[5, 0]]
+    for bad, what in ((nan, "non-finite"), (flat, "zero area")):
+        with pytest.raises(ValueError, match=what):
+            Mesh(torch.tensor(bad, device=_dev()), torch.tensor(t, device=_dev()))
+    m = Mesh(torch.tensor(v, device=_dev()), torch.tensor(t, device=_dev()))
+    before = m.normals_curls()[0].clone()
+    for bad, what in ((nan, "non-finite"), (flat, "zero area")):
+        with pytest.raises(ValueError, match=what):
+            m.set_vertices(torch.tensor(bad, device=_dev()))
+        with pytest.raises(ValueError, match=f"sample 2: .*{what}"):
+            GeometrySet(m, np.stack([v, v, bad, v]))
+    assert torch.equal(before, m.normals_curls()[0])
