@@ -527,6 +527,15 @@ __global__ __launch_bounds__(64 * kFinWaves) void batch_cbie_finalize_kernel(con
 // (the RHS operator itself is never stored)
 enum { kSweepAll = 0, kSweepSym = 1, kSweepPair = 2, kSweepAllRg = 3 };
 
+// Finished neighbour-pair blocks for the sweeps over every ordered pair (blk
+// null: the neighbour pairs are added elsewhere)
+struct P1PairBlocks {
+    const float2* blk = nullptr;  // [systems, npairs, 9]
+    const int4* pairs = nullptr;  // (i, j) order
+    const int64_t* pair_ptr = nullptr;
+    int64_t npairs = 0;
+};
+
 // The 3 x 3 block B(i, j) (row-basis a, column-basis b) of one regular pair
 // of the P1 operator OP with the Q-point rule: rr = the row triangle's
 // quadrature record, rci its curls (HYP, BM_LHS); py, wy, ny, cj the column
@@ -919,7 +928,8 @@ __global__ __launch_bounds__(256) void p1_regular_kernel(const float* __restrict
                                                          const KBatch kb, float2* __restrict__ out, int64_t ld,
                                                          const int32_t* __restrict__ vmap,
                                                          const float2* __restrict__ rg_g,
-                                                         float2* __restrict__ rg_out, int64_t plane)
+                                                         float2* __restrict__ rg_out, int64_t plane,
+                                                         const P1PairBlocks pb)
 {
     const float k = kb.k[blockIdx.z];
     out += (int64_t)blockIdx.z * kb.zstride;
@@ -977,7 +987,8 @@ __global__ __launch_bounds__(256) void p1_regular_kernel(const float* __restrict
         rrec[q][e - q * S] = rec[(int64_t)tl.perm[r0 + q] * S + (e - q * S)];
     }
     for (int q = threadIdx.x; q < r1 - r0; q += CT) {
-        rtri[q] = tris[tl.perm[r0 + q]];
+        const int4 tv = tris[tl.perm[r0 + q]];
+        rtri[q] = make_int4(tv.x, tv.y, tv.z, tl.perm[r0 + q]);
         rslot[q] = tl.row_slot[r0 + q];
     }
     if constexpr (OP == HYP || base_op(OP) == BM_LHS)
@@ -1067,6 +1078,7 @@ __global__ __launch_bounds__(256) void p1_regular_kernel(const float* __restrict
     float accTr[PAIR ? kP1RowVerts : 1], accTi[PAIR ? kP1RowVerts : 1];
 #pragma unroll
     for (int q = 0; q < (PAIR ? kP1RowVerts : 1); ++q) accTr[q] = accTi[q] = 0.f;
+    bool near = false;  // this lane's triangle shares a vertex with a row triangle
     __syncthreads();
 
     for (int rp = r0; rp < r1; ++rp) {
@@ -1088,6 +1100,7 @@ __global__ __launch_bounds__(256) void p1_regular_kernel(const float* __restrict
 #pragma unroll
         for (int e = 0; e < (RG ? 6 : 1); ++e) rgs[e] = 0.f;
         const bool eval = active && !shared;
+        if constexpr (!HALF) near = near || (active && shared);
         if (eval) {
             float ci[9];
             if constexpr (OP == HYP || base_op(OP) == BM_LHS) {
@@ -1140,6 +1153,34 @@ __global__ __launch_bounds__(256) void p1_regular_kernel(const float* __restrict
             accTr[sx] += s0.x; accTi[sx] += s0.y;
             accTr[sy] += s1.x; accTi[sy] += s1.y;
             accTr[sz] += s2.x; accTi[sz] += s2.y;
+            __syncthreads();
+        }
+    }
+    if constexpr (!HALF) {
+        // the tile's neighbour pairs, as finished blocks (p1_pairs_kernel): a
+        // wavefront per row triangle, a lane per pair, into the accumulator
+        // before its flush.  Looked up inside the row loop instead, the
+        // lookups' latency cost every workgroup near the diagonal a third
+        if (pb.blk && __syncthreads_or(near)) {
+            const float2* blk = pb.blk + (int64_t)blockIdx.z * pb.npairs * 9;
+            for (int q = threadIdx.x >> 6; q < r1 - r0; q += CT / 64) {
+                const int4 rs = rslot[q];
+                const int64_t e1 = pb.pair_ptr[rtri[q].w + 1];
+                for (int64_t e = pb.pair_ptr[rtri[q].w] + (threadIdx.x & 63); e < e1; e += 64) {
+                    const int p = tl.pos[pb.pairs[e].y];
+                    if (p < c0 || p >= c1) continue;
+                    const int4 cs = tl.col_slot[p];
+                    const int ra[3] = {rs.x, rs.y, rs.z}, cb[3] = {cs.x, cs.y, cs.z};
+#pragma unroll
+                    for (int a = 0; a < 3; ++a)
+#pragma unroll
+                        for (int b = 0; b < 3; ++b) {
+                            const float2 v = blk[e * 9 + 3 * a + b];
+                            atomicAdd(&acc[ra[a]][cb[b]].x, v.x);
+                            atomicAdd(&acc[ra[a]][cb[b]].y, v.y);
+                        }
+                }
+            }
             __syncthreads();
         }
     }
@@ -1256,11 +1297,14 @@ __device__ __forceinline__ double wave_sum(double v)
 }
 
 // sum over aligned groups of N lanes (N a power of two <= 64), in every lane
-// (16 and 64: DPP row moves, bem_device.hpp; others: cross-lane permutes)
+// (4, 16 and 64: DPP row moves, bem_device.hpp; others: cross-lane permutes)
 template <int N>
 __device__ __forceinline__ double group_sum(double v)
 {
-    if constexpr (N == 16) {
+    if constexpr (N == 4) {
+        v += dpp_row_d<0xB1>(v);
+        return v + dpp_row_d<0x4E>(v);
+    } else if constexpr (N == 16) {
         return row_sum16(v);
     } else if constexpr (N == 64) {
         return wave_sum64(v);
@@ -1339,24 +1383,18 @@ __device__ __forceinline__ void ss_pair_setup(const float* __restrict__ geo, con
     g.jij = gi[12] * gj[12];
 }
 
-// MODE 0: write (DP0: out = alpha * entry) or add (P1) the entries;
-// MODE 2 (P1): contract them with psi into vpsi, nothing stored.
-template <int OP, int NL, int BASIS, bool CLAMP, int MODE = 0>
+// Writes (DP0: out = alpha * entry) or adds (P1) the pairs' entries.
+template <int OP, int NL, int BASIS, bool CLAMP>
 __global__ __launch_bounds__(256) void singular_kernel(const float* __restrict__ geo, const int4* __restrict__ tris,
                                                        const float* __restrict__ curls,
                                                        const int4* __restrict__ pairs, int64_t p0, int64_t p1,
                                                        const KBatch kb, float2* __restrict__ out, int64_t ld,
-                                                       int64_t row0, float alpha, const float2* __restrict__ psi,
-                                                       float2* __restrict__ vpsi)
+                                                       int64_t row0, float alpha)
 {
     const float k = kb.k[blockIdx.z];
     out += (int64_t)blockIdx.z * kb.zstride;
     geo += (int64_t)blockIdx.z * kb.gstride;
     curls += (int64_t)blockIdx.z * kb.gstride;
-    if constexpr (MODE == 2) {
-        psi += (int64_t)blockIdx.z * kb.vstride;
-        vpsi += (int64_t)blockIdx.z * kb.vstride;
-    }
     const int lane = threadIdx.x & 63;
     // lanes per pair: a wavefront per pair, except the 2-point line rule of the
     // P1 operators (16 points): 16 lanes per pair, 4 pairs per wavefront, so
@@ -1443,34 +1481,6 @@ __global__ __launch_bounds__(256) void singular_kernel(const float* __restrict__
     if constexpr (BASIS == DP0) {
         if (lane == 0)
             out[((int64_t)i - row0) * ld + j] = make_float2((float)(alpha * ar[9]), (float)(alpha * ai[9]));
-    } else if constexpr (MODE == 2) {
-        // P1 contraction (the operator is not stored): entry (a, b) times psi
-        // at its column vertex; the three lanes 3a, 3a + 1, 3a + 2 of the
-        // pair's group are summed, so each pair adds three values (one per
-        // row corner) into vpsi instead of nine (on small meshes every row
-        // vertex takes hundreds of these atomics)
-        static_assert(OP == BM_RHS, "the contraction is the Burton-Miller right-hand side's");
-        float cr = 0.f, cim = 0.f;
-        int oa = 0;
-        if (valid && ll < 9) {
-            const int a = ll / 3, b = ll % 3;
-            double vr = 0.0, vi = 0.0;
-#pragma unroll
-            for (int e = 0; e < 9; ++e)
-                if (e == ll) { vr = ar[e]; vi = ai[e]; }
-            oa = pick3(g.pi, a);
-            const float2 gv = psi[pick3(g.ja, pick3(g.pj, b))];
-            cr = (float)(vr * gv.x - vi * gv.y);
-            cim = (float)(vr * gv.y + vi * gv.x);
-        }
-        // every lane takes part in the shuffles; lanes 3a + 1, 3a + 2 stay in the group (ll <= 8 < 16)
-        const float r1 = __shfl_down(cr, 1, 64), i1 = __shfl_down(cim, 1, 64);
-        const float r2 = __shfl_down(cr, 2, 64), i2 = __shfl_down(cim, 2, 64);
-        if (valid && ll < 9 && ll % 3 == 0) {
-            float* dst = reinterpret_cast<float*>(&vpsi[pick3(g.ia, oa)]);
-            unsafeAtomicAdd(dst, cr + r1 + r2);
-            unsafeAtomicAdd(dst + 1, cim + i1 + i2);
-        }
     } else {
         if (valid && ll < 9) {
             // ll = reordered (a, b) pair; its original local indices are (g.pi[a], g.pj[b])
@@ -1507,6 +1517,211 @@ __global__ __launch_bounds__(256) void singular_kernel(const float* __restrict__
             unsafeAtomicAdd(dst, (float)vr);
             unsafeAtomicAdd(dst + 1, (float)vi);
         }
+    }
+}
+
+// The neighbour pairs of a P1 operator as finished 3 x 3 blocks: block p of
+// system z at blk + (z npairs + p) 9, row corner 3 a + column corner b in the
+// triangles' own order, p the pair's place in the (i, j) order.  The regular
+// sweep over every ordered pair picks them up as it meets the pair, so they reach
+// the matrix through its tile accumulators (nine complex float atomics per
+// pair into the matrix bound this step before).  LPP lanes per pair share its
+// points: few lanes leave each more points, and the pair's set-up and its FP64
+// sums over the lanes, which cost as much as the points, are shared by more
+// pairs of the wavefront.
+// lhs_mass: times the mass matrix added (with the coincident pairs).
+// RG (Burton-Miller LHS): the right-hand side operator's entries at the same
+// points, contracted with g, and -(i/2k) M g: three row sums per pair at
+// rg + (z npairs + p) 3.
+template <int OP, int NL, bool CLAMP, int LPP, bool RG>
+__global__ __launch_bounds__(256) void p1_pairs_kernel(const float* __restrict__ geo, const int4* __restrict__ tris,
+                                                       const float* __restrict__ curls,
+                                                       const int4* __restrict__ pairs, int64_t npairs, const KBatch kb,
+                                                       float lhs_mass, float2* __restrict__ blk,
+                                                       const float2* __restrict__ g_vec, float2* __restrict__ rg)
+{
+    static_assert(!RG || OP == BM_LHS, "the right-hand side rides on the Burton-Miller LHS");
+    constexpr int PPW = 64 / LPP;
+    constexpr int NP = NL * NL * NL * NL;
+    static_assert(NP % LPP == 0, "points shared evenly");
+    const float k = kb.k[blockIdx.z], krev = k * kInv2Pi;
+    geo += (int64_t)blockIdx.z * kb.gstride;
+    curls += (int64_t)blockIdx.z * kb.gstride;
+    const int lane = threadIdx.x & 63, ll = lane % LPP;
+    const int64_t pw = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * PPW;  // the wavefront's first pair
+    if (pw >= npairs) return;  // uniform per wavefront
+    const bool valid = pw + lane / LPP < npairs;  // groups past the end compute on the last pair and write nothing
+    const int4 pr = pairs[valid ? pw + lane / LPP : npairs - 1];
+    const int i = PPW == 1 ? __builtin_amdgcn_readfirstlane(pr.x) : pr.x;
+    const int j = PPW == 1 ? __builtin_amdgcn_readfirstlane(pr.y) : pr.y;
+    const int shared = PPW == 1 ? __builtin_amdgcn_readfirstlane(pr.z) : pr.z;
+    const int64_t out = (int64_t)blockIdx.z * npairs + pr.w;  // the pair's place in the (i, j) order
+    SSPair g;
+    ss_pair_setup(geo, tris, i, j, shared, g);
+    const float nx0 = g.nx[0], nx1 = g.nx[1], nx2 = g.nx[2], ny0 = g.ny[0], ny1 = g.ny[1], ny2 = g.ny[2];
+    float2 gv[3];  // RG: g at the column corners, reordered
+    if constexpr (RG) {
+        g_vec += (int64_t)blockIdx.z * kb.vstride;
+#pragma unroll
+        for (int b = 0; b < 3; ++b) gv[b] = g_vec[pick3(g.ja, g.pj[b])];
+    }
+    constexpr bool CURL = OP == HYP || base_op(OP) == BM_LHS;
+    constexpr int NE = CURL ? 10 : 9;  // entry 9: the plain sum of the curl term
+    double ar[NE], ai[NE], rr[RG ? 3 : 1], ri[RG ? 3 : 1];
+#pragma unroll
+    for (int e = 0; e < NE; ++e) ar[e] = ai[e] = 0.0;
+#pragma unroll
+    for (int a = 0; a < (RG ? 3 : 1); ++a) rr[a] = ri[a] = 0.0;
+    ss_dispatch(shared, [&](auto kind) {
+        constexpr int S = decltype(kind)::value;
+        constexpr int NR = kSSRegions<S>;
+#pragma unroll 1
+        for (int q = ll; q < NP; q += LPP) {
+            const int q0 = q / (NL * NL * NL), q1 = (q / (NL * NL)) % NL, q2 = (q / NL) % NL, q3 = q % NL;
+            const float wq =
+                LineRule01<NL>::w[q0] * LineRule01<NL>::w[q1] * LineRule01<NL>::w[q2] * LineRule01<NL>::w[q3];
+            float reg[NR][7];
+            const float jac = ss_regions<S>(LineRule01<NL>::t[q0], LineRule01<NL>::t[q1], LineRule01<NL>::t[q2],
+                                            LineRule01<NL>::t[q3], reg);
+            float br[NE], bi[NE], cr[RG ? 3 : 1], ci[RG ? 3 : 1];
+#pragma unroll
+            for (int e = 0; e < NE; ++e) br[e] = bi[e] = 0.f;
+#pragma unroll
+            for (int a = 0; a < (RG ? 3 : 1); ++a) cr[a] = ci[a] = 0.f;
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                const float x1 = reg[r][0], x2 = reg[r][1], y1 = reg[r][2], y2 = reg[r][3], ww = reg[r][4];
+                float dx, dy, dz;
+                ss_disp<S>(reg[r], g.e1, g.e2, g.f1, g.f2, dx, dy, dz);
+                float vr, vi, gr = 0.f, gi = 0.f;
+                kernel4pi<OP, CLAMP>(dx, dy, dz, nx0, nx1, nx2, ny0, ny1, ny2, k, krev, vr, vi, gr, gi);
+                vr *= ww;
+                vi *= ww;
+                const float px[3] = {1.f - x1, x1 - x2, x2};
+                const float py[3] = {1.f - y1, y1 - y2, y2};
+#pragma unroll
+                for (int a = 0; a < 3; ++a)
+#pragma unroll
+                    for (int b = 0; b < 3; ++b) {
+                        const float pp = px[a] * py[b];
+                        br[3 * a + b] = fmaf(vr, pp, br[3 * a + b]);
+                        bi[3 * a + b] = fmaf(vi, pp, bi[3 * a + b]);
+                    }
+                if constexpr (OP == HYP) {  // plain G
+                    br[9] += vr;
+                    bi[9] += vi;
+                } else if constexpr (CURL) {
+                    br[9] = fmaf(gr, ww, br[9]);
+                    bi[9] = fmaf(gi, ww, bi[9]);
+                }
+                if constexpr (RG) {
+                    float v2r, v2i, u0 = 0.f, u1 = 0.f;
+                    kernel4pi<BM_RHS, CLAMP>(dx, dy, dz, nx0, nx1, nx2, ny0, ny1, ny2, k, krev, v2r, v2i, u0, u1);
+                    const float hr = ww * (py[0] * gv[0].x + py[1] * gv[1].x + py[2] * gv[2].x);
+                    const float hi = ww * (py[0] * gv[0].y + py[1] * gv[1].y + py[2] * gv[2].y);
+                    const float tr = v2r * hr - v2i * hi, ti = v2r * hi + v2i * hr;
+#pragma unroll
+                    for (int a = 0; a < 3; ++a) {
+                        cr[a] = fmaf(px[a], tr, cr[a]);
+                        ci[a] = fmaf(px[a], ti, ci[a]);
+                    }
+                }
+            }
+            const double sc = (double)(jac * wq) * (double)g.jij;
+#pragma unroll
+            for (int e = 0; e < NE; ++e) {
+                ar[e] += sc * (double)br[e];
+                ai[e] += sc * (double)bi[e];
+            }
+            if constexpr (RG) {
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    rr[a] += sc * (double)cr[a];
+                    ri[a] += sc * (double)ci[a];
+                }
+            }
+        }
+    });
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+        ar[e] = group_sum<LPP>(ar[e]) * (double)kInv4Pi;
+        ai[e] = group_sum<LPP>(ai[e]) * (double)kInv4Pi;
+    }
+    if constexpr (RG) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            rr[a] = group_sum<LPP>(rr[a]) * (double)kInv4Pi;
+            ri[a] = group_sum<LPP>(ri[a]) * (double)kInv4Pi;
+        }
+    }
+    if (!valid) return;
+    const float m24 = geo[(int64_t)i * 16 + 12] * (1.0f / 24.0f);  // mass entries |c| (1 + delta) / 24
+#pragma unroll
+    for (int e = 0; e < 9; ++e) {  // lane ll writes entries ll, ll + LPP, ...
+        if (e % LPP != ll) continue;
+        const int oa = g.pi[e / 3], ob = g.pj[e % 3];
+        double vr = ar[e], vi = ai[e];
+        if constexpr (CURL) {
+            const float* ci = curls + (int64_t)i * 12 + 3 * oa;
+            const float* cj = curls + (int64_t)j * 12 + 3 * ob;
+            const double c = ci[0] * cj[0] + ci[1] * cj[1] + ci[2] * cj[2];
+            if constexpr (OP == HYP) {
+                const double kk = (double)k * (double)k * (double)(nx0 * ny0 + nx1 * ny1 + nx2 * ny2);
+                vr = ar[9] * c - vr * kk;
+                vi = ai[9] * c - vi * kk;
+            } else {
+                const double invk = 1.0 / (double)k;
+                vr += -ai[9] * invk * c;
+                vi += ar[9] * invk * c;
+            }
+        }
+        if (i == j) vr += (double)(lhs_mass * (oa == ob ? 2.0f * m24 : m24));
+        blk[out * 9 + 3 * oa + ob] = make_float2((float)vr, (float)vi);
+    }
+    if constexpr (RG) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            if (a % LPP != ll) continue;
+            float tr = (float)rr[a], ti = (float)ri[a];
+            if (i == j) {  // -(i/2k) (M g) of this corner
+                const float mx = m24 * (gv[0].x + gv[1].x + gv[2].x + gv[a].x);
+                const float my = m24 * (gv[0].y + gv[1].y + gv[2].y + gv[a].y);
+                const float h = 0.5f / k;
+                tr = fmaf(h, my, tr);
+                ti = fmaf(-h, mx, ti);
+            }
+            rg[out * 3 + g.pi[a]] = make_float2(tr, ti);
+        }
+    }
+}
+
+// rhs[v] += the pairs' row sums at v's corners (its triangles ascending, each
+// one's pairs in order); four lanes per vertex share them
+__global__ __launch_bounds__(256) void p1_pairs_rhs_kernel(const float2* __restrict__ rg, int64_t npairs,
+                                                           const int64_t* __restrict__ pair_ptr,
+                                                           const int32_t* __restrict__ vt_ptr,
+                                                           const int32_t* __restrict__ vt_corner, int64_t nv,
+                                                           float2* __restrict__ rhs, int64_t vstride)
+{
+    const int64_t v = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 2;
+    const int part = threadIdx.x & 3;
+    rg += (int64_t)blockIdx.y * npairs * 3;
+    rhs += (int64_t)blockIdx.y * vstride;
+    double sr = 0.0, si = 0.0;
+    if (v < nv)
+        for (int q = vt_ptr[v] + part; q < vt_ptr[v + 1]; q += 4) {
+            const int code = vt_corner[q], t = code / 3, c = code - 3 * t;
+            for (int64_t e = pair_ptr[t]; e < pair_ptr[t + 1]; ++e) {
+                const float2 x = rg[e * 3 + c];
+                sr += x.x;
+                si += x.y;
+            }
+        }
+    sr = group_sum<4>(sr);
+    si = group_sum<4>(si);
+    if (v < nv && part == 0) {
+        const float2 o = rhs[v];
+        rhs[v] = make_float2((float)(o.x + sr), (float)(o.y + si));
     }
 }
 
@@ -1622,41 +1837,9 @@ __global__ __launch_bounds__(256) void p1_rg_reduce_kernel(const float2* __restr
     unsafeAtomicAdd(dst + 1, sy);
 }
 
-// out[v] += alpha (M g)[v] for the P1 mass matrix M_ab = |c| (1 + delta_ab) / 24
-// per triangle (the closed form of identity_p1_kernel's entries); one thread
-// per triangle, atomics into the three corners.
 struct AlphaBatch {
     float2 a[kMaxBatchK];
 };
-
-// system z = blockIdx.y: geometry z (gstride floats on), g and out z * vstride
-// elements on, factor ab.a[z]
-__global__ __launch_bounds__(256) void p1_mass_apply_kernel(const float* __restrict__ geo, int64_t gstride,
-                                                            const int4* __restrict__ tris, int64_t nt,
-                                                            const float2* __restrict__ g, const AlphaBatch ab,
-                                                            float2* __restrict__ out, int64_t vstride)
-{
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (t >= nt) return;
-    const int z = blockIdx.y;
-    geo += (int64_t)z * gstride;
-    g += (int64_t)z * vstride;
-    out += (int64_t)z * vstride;
-    const float2 alpha = ab.a[z];
-    const int4 tr = tris[t];
-    const float c = geo[t * 16 + 12] * (1.0f / 24.0f);
-    const float2 g0 = g[tr.x], g1 = g[tr.y], g2 = g[tr.z];
-    const float sx = g0.x + g1.x + g2.x, sy = g0.y + g1.y + g2.y;
-    const int v3[3] = {tr.x, tr.y, tr.z};
-    const float2 gv[3] = {g0, g1, g2};
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        const float mx = c * (sx + gv[a].x), my = c * (sy + gv[a].y);  // (M g)_a from this triangle
-        float* dst = reinterpret_cast<float*>(&out[v3[a]]);
-        unsafeAtomicAdd(dst, alpha.x * mx - alpha.y * my);
-        unsafeAtomicAdd(dst + 1, alpha.x * my + alpha.y * mx);
-    }
-}
 
 // ---------------------------------------------------------------------------
 // mass matrix, triangle -> vertex average, potentials
@@ -1953,10 +2136,18 @@ __global__ __launch_bounds__(256) void p1_permute_planar_kernel(const float* __r
 // transposed flush, whose destination rows take 20 values each, cost more
 // than the halved evaluations save); one_sided evaluates every ordered pair.
 constexpr int64_t kP1PairMinVerts = 4096;
+template <int OP, int Q>
+static bool p1_ordered_sweep(const MeshDev& m, bool one_sided)
+{
+    const int64_t nb = (m.nv + kSymT - 1) / kSymT;
+    if (one_sided || m.tiles.nsym > 0x7fffffffLL || nb * nb > 0x7fffffffLL) return true;
+    if (OP == SLP || OP == HYP) return false;
+    return !((OP == DLP || OP == ADLP) && Q == 6 && m.nv >= kP1PairMinVerts);
+}
 template <int OP, int Q, bool CLAMP>
 static hipError_t p1_regular_t(const MeshDev& m, const KBatch& kb, int nz, float2* out, int64_t ld, bool one_sided,
-                               const int32_t* vmap, hipStream_t s, const float2* rg_g = nullptr,
-                               float2* rg_out = nullptr, bool* planar = nullptr)
+                               const int32_t* vmap, hipStream_t s, const P1PairBlocks& pb,
+                               const float2* rg_g = nullptr, float2* rg_out = nullptr, bool* planar = nullptr)
 {
     // planar (an [n, n] scratch per z, ld == n): the every-ordered-pair and
     // paired sweeps flush real and imaginary planes; *planar says whether the
@@ -1967,35 +2158,32 @@ static hipError_t p1_regular_t(const MeshDev& m, const KBatch& kb, int nz, float
     constexpr bool sym = OP == SLP || OP == HYP;
     constexpr bool pair = (OP == DLP || OP == ADLP) && Q == 6;
     const int64_t plane = planar ? n * n : 0;
-    if (!one_sided && m.tiles.nsym <= 0x7fffffffLL && nb * nb <= 0x7fffffffLL) {
+    if (!p1_ordered_sweep<OP, Q>(m, one_sided)) {
         if constexpr (sym) {
             hipLaunchKernelGGL((p1_regular_kernel<OP, Q, CLAMP, kSweepSym>), dim3((unsigned)m.tiles.nsym, 1, nz),
                                dim3(256), 0, s, rec, m.tris, m.curls, m.tiles, kb, out, ld, vmap, nullptr, nullptr,
-                               (int64_t)0);
+                               (int64_t)0, P1PairBlocks{});
             hipLaunchKernelGGL(p1_symmetrize_kernel, dim3((unsigned)(nb * (nb + 1) / 2), 1, nz), dim3(256), 0, s, out,
                                n, ld, kb.zstride);
-            return hipGetLastError();
         } else if constexpr (pair) {
-            if (n >= kP1PairMinVerts) {
-                if (planar) *planar = true;
-                hipLaunchKernelGGL((p1_regular_kernel<OP, Q, CLAMP, kSweepPair>), dim3((unsigned)m.tiles.nsym, 1, nz),
-                                   dim3(256), 0, s, rec, m.tris, m.curls, m.tiles, kb, out, ld, vmap, nullptr, nullptr,
-                                   plane);
-                return hipGetLastError();
-            }
+            if (planar) *planar = true;
+            hipLaunchKernelGGL((p1_regular_kernel<OP, Q, CLAMP, kSweepPair>), dim3((unsigned)m.tiles.nsym, 1, nz),
+                               dim3(256), 0, s, rec, m.tris, m.curls, m.tiles, kb, out, ld, vmap, nullptr, nullptr,
+                               plane, P1PairBlocks{});
         }
+        return hipGetLastError();
     }
     dim3 grid((unsigned)m.tiles.ncol_tiles, (unsigned)m.tiles.nrow_tiles, (unsigned)nz);
     if (planar) *planar = true;
     if constexpr (OP == BM_LHS) {
         if (rg_out) {
             hipLaunchKernelGGL((p1_regular_kernel<OP, Q, CLAMP, kSweepAllRg>), grid, dim3(256), 0, s, rec, m.tris,
-                               m.curls, m.tiles, kb, out, ld, vmap, rg_g, rg_out, plane);
+                               m.curls, m.tiles, kb, out, ld, vmap, rg_g, rg_out, plane, pb);
             return hipGetLastError();
         }
     }
     hipLaunchKernelGGL((p1_regular_kernel<OP, Q, CLAMP, kSweepAll>), grid, dim3(256), 0, s, rec, m.tris, m.curls,
-                       m.tiles, kb, out, ld, vmap, nullptr, nullptr, plane);
+                       m.tiles, kb, out, ld, vmap, nullptr, nullptr, plane, pb);
     return hipGetLastError();
 }
 
@@ -2010,8 +2198,43 @@ static hipError_t singular_t(const MeshDev& m, int64_t p0, int64_t p1, const KBa
     // P1 takes every pair (p0 = 0, p1 = npairs): the list grouped by kind
     const int4* pl = BASIS == P1 ? m.pairs_by_kind : m.pairs;
     hipLaunchKernelGGL((singular_kernel<OP, NL, BASIS, CLAMP>), dim3(g, 1, nz), dim3(256), 0, s, m.geo, m.tris,
-                       m.curls, pl, p0, p1, kb, out, ld, row0, 1.0f, nullptr, nullptr);
+                       m.curls, pl, p0, p1, kb, out, ld, row0, 1.0f);
     return hipGetLastError();
+}
+
+// Neighbour-pair blocks of a P1 operator (p1_pairs_kernel).  Lanes per pair: 4
+// (2-point line rule, 16 points) or 16 (4-point, 256 points), and four times as
+// many while the pairs are too few to fill the GPU's wavefronts that way.
+constexpr int64_t kPairsFill2 = 1 << 15, kPairsFill4 = 1 << 15;
+template <int OP, bool CLAMP, bool RG>
+static hipError_t launch_p1_pairs(const MeshDev& m, int quad, const KBatch& kb, int nz, float lhs_mass, float2* blk,
+                                  const float2* g, float2* rg, hipStream_t s)
+{
+    const int64_t total = m.npairs * nz;
+    auto run = [&](auto nl, auto lpp) {
+        constexpr int NL = decltype(nl)::value, LPP = decltype(lpp)::value;
+        const int64_t per = 4 * (64 / LPP);
+        hipLaunchKernelGGL((p1_pairs_kernel<OP, NL, CLAMP, LPP, RG>),
+                           dim3((unsigned)((m.npairs + per - 1) / per), 1, (unsigned)nz), dim3(256), 0, s, m.geo, m.tris,
+                           m.curls, m.pairs_by_kind, m.npairs, kb, lhs_mass, blk, g, rg);
+    };
+    if (quad == 0) {
+        if (total >= kPairsFill4) run(std::integral_constant<int, 4>{}, std::integral_constant<int, 16>{});
+        else run(std::integral_constant<int, 4>{}, std::integral_constant<int, 64>{});
+    } else {
+        if (total >= kPairsFill2) run(std::integral_constant<int, 2>{}, std::integral_constant<int, 4>{});
+        else run(std::integral_constant<int, 2>{}, std::integral_constant<int, 16>{});
+    }
+    return hipGetLastError();
+}
+static P1PairBlocks pair_blocks(const MeshDev& m, const float2* blk)
+{
+    P1PairBlocks pb;
+    pb.blk = blk;
+    pb.pairs = m.pairs;
+    pb.pair_ptr = m.pair_ptr;
+    pb.npairs = m.npairs;
+    return pb;
 }
 
 // ---- fused DP0 CBIE system -------------------------------------------------
@@ -2141,19 +2364,36 @@ static hipError_t assemble_op(const MeshDev& m, int basis, int quad, int parts, 
         // are in P1 order, so the mapped addresses are scattered).
         const bool one_sided = (parts & 4) != 0;
         const int64_t n = m.nv;
+        // sweeps over every ordered pair take the neighbour pairs along as
+        // finished blocks; the half sweeps leave them to singular_kernel
+        float2* blk = nullptr;
+        const bool ordered = quad == 0   ? p1_ordered_sweep<OP, 6>(m, one_sided)
+                             : quad == 1 ? p1_ordered_sweep<OP, 3>(m, one_sided)
+                                         : p1_ordered_sweep<OP, 1>(m, one_sided);
+        if (ordered && (parts & 2)) {
+            if (hipMallocAsync((void**)&blk, sizeof(float2) * 9 * (size_t)m.npairs * (size_t)nz, s) == hipSuccess) {
+                e = launch_p1_pairs<OP, CLAMP, false>(m, quad, kb, nz, 0.f, blk, nullptr, nullptr, s);
+                parts &= ~2;
+            } else {
+                (void)hipGetLastError();
+                blk = nullptr;
+            }
+        }
+        const P1PairBlocks pb = pair_blocks(m, blk);
         auto regular = [&](float2* dst, int64_t ldd, const KBatch& kbd, const int32_t* vmap,
                            bool* planar) -> hipError_t {
             hipError_t er = launch_fill_z(dst, n, n, ldd, kbd.zstride, nz, make_float2(0.f, 0.f), s);
             if (er != hipSuccess) return er;
-            if (quad == 0) return p1_regular_t<OP, 6, CLAMP>(m, kbd, nz, dst, ldd, one_sided, vmap, s, nullptr,
+            if (quad == 0) return p1_regular_t<OP, 6, CLAMP>(m, kbd, nz, dst, ldd, one_sided, vmap, s, pb, nullptr,
                                                              nullptr, planar);
-            if (quad == 1) return p1_regular_t<OP, 3, CLAMP>(m, kbd, nz, dst, ldd, one_sided, vmap, s, nullptr,
+            if (quad == 1) return p1_regular_t<OP, 3, CLAMP>(m, kbd, nz, dst, ldd, one_sided, vmap, s, pb, nullptr,
                                                              nullptr, planar);
-            return p1_regular_t<OP, 1, CLAMP>(m, kbd, nz, dst, ldd, one_sided, vmap, s, nullptr, nullptr, planar);
+            return p1_regular_t<OP, 1, CLAMP>(m, kbd, nz, dst, ldd, one_sided, vmap, s, pb, nullptr, nullptr, planar);
         };
         float2* S = nullptr;
-        if (!(parts & 8) &&
-            hipMallocAsync((void**)&S, sizeof(float2) * (size_t)n * (size_t)n * (size_t)nz, s) == hipSuccess) {
+        if (e != hipSuccess) {
+        } else if (!(parts & 8) &&
+                   hipMallocAsync((void**)&S, sizeof(float2) * (size_t)n * (size_t)n * (size_t)nz, s) == hipSuccess) {
             KBatch kbs = kb;
             kbs.zstride = n * n;
             bool planar = false;
@@ -2172,6 +2412,10 @@ static hipError_t assemble_op(const MeshDev& m, int basis, int quad, int parts, 
         } else {
             (void)hipGetLastError();  // no room for the scratch, or none asked for (parts & 8)
             e = regular(out, ld, kb, m.p1_vold, nullptr);
+        }
+        if (blk) {
+            const hipError_t ef = hipFreeAsync(blk, s);
+            if (e == hipSuccess) e = ef;
         }
         if (e != hipSuccess) return e;
     }
@@ -2307,9 +2551,12 @@ hipError_t launch_add_identity(const MeshDev& m, int basis, float2 alpha, float2
 // The Burton-Miller system of neumann2dirichlet in the P1 basis:
 // lhs = bm_lhs + M/2, rhs = (bm_rhs - (i/2k) M) g.  The RHS operator is never
 // stored: its regular pairs are contracted with g inside the LHS tile kernel
-// (the same Gauss-point pairs, sharing e^{ikr}/r), its neighbour pairs by the
-// contraction mode of the neighbour-pair kernel, its mass term by one pass
-// over the triangles.
+// (the same Gauss-point pairs, sharing e^{ikr}/r).  The neighbour pairs of both
+// operators and both mass terms come from one kernel, as blocks the tile kernel
+// takes along and as row sums per pair (two neighbour-pair kernels with
+// atomics and two mass kernels took 970 us of 32 systems of 1002 vertices).
+// Without room for the scratch matrix the tile kernel flushes to lhs through
+// the vertex map (slower: scattered addresses).
 template <bool CLAMP>
 static hipError_t bm_system_p1_t(const MeshDev& m, int64_t gstride, const KBatch& kbin, int nz, int quad,
                                  const float2* g, float2* lhs, int64_t ld, int64_t lstride, float2* rhs,
@@ -2322,21 +2569,30 @@ static hipError_t bm_system_p1_t(const MeshDev& m, int64_t gstride, const KBatch
     kb.vstride = n;
     hipError_t e = launch_fill(rhs, nz, n, n, make_float2(0.f, 0.f), s);
     if (e != hipSuccess) return e;
-    // the right-hand side's regular pairs: one partial row per column tile and system
+    // scratch: the pairs' blocks and row sums, the regular pairs' row sums (one
+    // partial row per column tile and system), the matrix in the tiles' numbering
     const int64_t nslots = m.h_row_slots;
-    float2* part = nullptr;
-    e = hipMallocAsync((void**)&part, sizeof(float2) * (size_t)m.tiles.ncol_tiles * (size_t)nslots * (size_t)nz, s);
-    if (e != hipSuccess) return e;
+    const size_t nblk = 9 * (size_t)m.npairs * nz, nrg = 3 * (size_t)m.npairs * nz,
+                 npart = (size_t)m.tiles.ncol_tiles * (size_t)nslots * nz, nmat = (size_t)n * (size_t)n * nz;
+    float2* blk = nullptr;
+    bool mat = hipMallocAsync((void**)&blk, sizeof(float2) * (nblk + nrg + npart + nmat), s) == hipSuccess;
+    if (!mat) {
+        (void)hipGetLastError();
+        e = hipMallocAsync((void**)&blk, sizeof(float2) * (nblk + nrg + npart), s);
+        if (e != hipSuccess) return e;
+    }
+    float2 *rg = blk + nblk, *part = rg + nrg, *S = part + npart;
+    const P1PairBlocks pb = pair_blocks(m, blk);
+    e = launch_p1_pairs<BM_LHS, CLAMP, true>(m, quad, kb, nz, 0.5f, blk, g, rg, s);
     auto regular = [&](float2* dst, int64_t ldd, const KBatch& kbd, const int32_t* vmap,
                        bool* planar) -> hipError_t {
         hipError_t er = launch_fill_z(dst, n, n, ldd, kbd.zstride, nz, make_float2(0.f, 0.f), s);
         if (er != hipSuccess) return er;
-        if (quad == 0) return p1_regular_t<BM_LHS, 6, CLAMP>(m, kbd, nz, dst, ldd, true, vmap, s, g, part, planar);
-        if (quad == 1) return p1_regular_t<BM_LHS, 3, CLAMP>(m, kbd, nz, dst, ldd, true, vmap, s, g, part, planar);
-        return p1_regular_t<BM_LHS, 1, CLAMP>(m, kbd, nz, dst, ldd, true, vmap, s, g, part, planar);
+        if (quad == 0) return p1_regular_t<BM_LHS, 6, CLAMP>(m, kbd, nz, dst, ldd, true, vmap, s, pb, g, part, planar);
+        if (quad == 1) return p1_regular_t<BM_LHS, 3, CLAMP>(m, kbd, nz, dst, ldd, true, vmap, s, pb, g, part, planar);
+        return p1_regular_t<BM_LHS, 1, CLAMP>(m, kbd, nz, dst, ldd, true, vmap, s, pb, g, part, planar);
     };
-    float2* S = nullptr;
-    if (hipMallocAsync((void**)&S, sizeof(float2) * (size_t)n * (size_t)n * (size_t)nz, s) == hipSuccess) {
+    if (e == hipSuccess && mat) {
         KBatch kbs = kb;
         kbs.zstride = n * n;
         bool planar = false;
@@ -2350,52 +2606,18 @@ static hipError_t bm_system_p1_t(const MeshDev& m, int64_t gstride, const KBatch
                                    m.p1_vnew, lhs, ld, lstride);
             e = hipGetLastError();
         }
-        const hipError_t ef = hipFreeAsync(S, s);
-        if (e == hipSuccess) e = ef;
-    } else {
-        (void)hipGetLastError();  // no room for the scratch: flush through the vertex map
+    } else if (e == hipSuccess) {
         e = regular(lhs, ld, kb, m.p1_vold, nullptr);
     }
     if (e == hipSuccess) {
         hipLaunchKernelGGL(p1_rg_reduce_kernel, dim3(grid1d(nslots), (unsigned)nz), dim3(256), 0, s,
                            (const float2*)part, m.tiles.ncol_tiles, nslots, m.tiles.row_verts, m.p1_vold, rhs, n);
+        hipLaunchKernelGGL(p1_pairs_rhs_kernel, dim3((unsigned)((4 * n + 255) / 256), (unsigned)nz), dim3(256), 0, s,
+                           (const float2*)rg, m.npairs, m.pair_ptr, m.vt_ptr, m.vt_corner, n, rhs, n);
         e = hipGetLastError();
     }
-    {
-        const hipError_t ef = hipFreeAsync(part, s);
-        if (e == hipSuccess) e = ef;
-    }
-    if (e != hipSuccess) return e;
-    // neighbour pairs: the LHS into lhs, the RHS contracted with g into rhs
-    if (quad == 0) e = singular_t<BM_LHS, 4, P1, CLAMP>(m, 0, m.npairs, kb, nz, lhs, ld, 0, s);
-    else e = singular_t<BM_LHS, 2, P1, CLAMP>(m, 0, m.npairs, kb, nz, lhs, ld, 0, s);
-    if (e != hipSuccess) return e;
-    if (m.npairs > 0) {
-        if (quad == 0) {
-            const unsigned gs = (unsigned)((m.npairs + 3) / 4);  // one pair per wavefront
-            hipLaunchKernelGGL((singular_kernel<BM_RHS, 4, P1, CLAMP, 2>), dim3(gs, 1, (unsigned)nz), dim3(256), 0, s,
-                               m.geo, m.tris, m.curls, m.pairs_by_kind, (int64_t)0, m.npairs, kb, (float2*)nullptr,
-                               (int64_t)0, (int64_t)0, 1.0f, g, rhs);
-        } else {
-            const unsigned gs = (unsigned)((m.npairs + 15) / 16);  // four pairs per wavefront
-            hipLaunchKernelGGL((singular_kernel<BM_RHS, 2, P1, CLAMP, 2>), dim3(gs, 1, (unsigned)nz), dim3(256), 0, s,
-                               m.geo, m.tris, m.curls, m.pairs_by_kind, (int64_t)0, m.npairs, kb, (float2*)nullptr,
-                               (int64_t)0, (int64_t)0, 1.0f, g, rhs);
-        }
-        e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
-    // mass terms: rhs_z -= (i/2k_z) M_z g_z, lhs_z += M_z/2
-    AlphaBatch ar{}, al{};
-    for (int z = 0; z < nz; ++z) {
-        ar.a[z] = make_float2(0.f, -0.5f / kb.k[z]);
-        al.a[z] = make_float2(0.5f, 0.f);
-    }
-    hipLaunchKernelGGL(p1_mass_apply_kernel, dim3(grid1d(m.nt), (unsigned)nz), dim3(256), 0, s, m.geo, gstride, m.tris,
-                       m.nt, g, ar, rhs, n);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    return add_identity_z(m, gstride, P1, al, nz, lhs, ld, lstride, s);
+    const hipError_t ef = hipFreeAsync(blk, s);
+    return e != hipSuccess ? e : ef;
 }
 
 hipError_t launch_bm_system_p1(const MeshDev& m, float k, int quad, int clamp, const float2* g, float2* lhs,

@@ -26,6 +26,7 @@ constexpr int kP1ColVerts = 200;
 // Locality-ordered tiling of the triangle list for the P1 scatter.
 struct P1Tiles {
     const int32_t* perm;       // [nt] triangle id at ordered position
+    const int32_t* pos;        // [nt] ordered position of each triangle
     const int32_t* row_ptr;    // [nrow_tiles+1] position ranges
     const int32_t* row_vptr;   // [nrow_tiles+1] ranges into row_verts
     const int32_t* row_verts;  // global vertex ids of each row tile

@@ -390,12 +390,21 @@ int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t 
         }
     }
     m.npairs = (int64_t)pairs.size();
+    if (m.npairs > INT32_MAX) {
+        err = "mesh has more than 2^31 neighbour pairs";
+        return 1;
+    }
     // the P1 neighbour-pair launches take every pair in any order: grouped by
     // kind, the pairs that share a wavefront take the same quadrature branch
+    // (the last entry: the pair's place in the (i, j) order)
     std::vector<Pair> pairs_kind(pairs.size());
     {
         int64_t next[4] = {0, kinds[3] + kinds[2], kinds[3], 0};
-        for (const Pair& p : pairs) pairs_kind[(size_t)next[p.shared]++] = p;
+        for (size_t q = 0; q < pairs.size(); ++q) {
+            Pair& p = pairs_kind[(size_t)next[pairs[q].shared]++];
+            p = pairs[q];
+            p.pad = (int32_t)q;
+        }
     }
     m.max_neighbors = maxnb;
 
@@ -438,6 +447,8 @@ int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t 
         }
         for (int64_t t = 0; t < nt; ++t) perm[t] = key[t].t;
     }
+    std::vector<int32_t> pos((size_t)nt);
+    for (int64_t q = 0; q < nt; ++q) pos[perm[q]] = (int32_t)q;
     // P1 numbering: vertices in the order they first appear along the Morton
     // order of the triangles, so the vertices of a tile are (nearly)
     // consecutive and its accumulator flush lands in few cache lines; the
@@ -513,10 +524,11 @@ int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t 
     parts.push_back({vt_ptr.data(), vt_ptr.size() * 4, (void**)&m.vt_ptr});
     parts.push_back({vt_idx.data(), vt_idx.size() * 4, (void**)&m.vt_idx});
     parts.push_back({vt_corner.data(), vt_corner.size() * 4, (void**)&m.vt_corner});
-    int32_t *d_perm, *d_rp, *d_rvp, *d_rv, *d_cp, *d_cvp, *d_cv, *d_cip, *d_ci, *d_rct;
+    int32_t *d_perm, *d_pos, *d_rp, *d_rvp, *d_rv, *d_cp, *d_cvp, *d_cv, *d_cip, *d_ci, *d_rct;
     int64_t* d_sym;
     int4 *d_rs, *d_cs;
     parts.push_back({perm.data(), perm.size() * 4, (void**)&d_perm});
+    parts.push_back({pos.data(), pos.size() * 4, (void**)&d_pos});
     parts.push_back({rowT.ptr.data(), rowT.ptr.size() * 4, (void**)&d_rp});
     parts.push_back({rowT.vptr.data(), rowT.vptr.size() * 4, (void**)&d_rvp});
     parts.push_back({rowT.verts.data(), rowT.verts.size() * 4, (void**)&d_rv});
@@ -575,6 +587,7 @@ int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t 
         }
     }
     m.tiles.perm = d_perm;
+    m.tiles.pos = d_pos;
     m.tiles.row_ptr = d_rp;
     m.tiles.row_vptr = d_rvp;
     m.tiles.row_verts = d_rv;

@@ -1,0 +1,77 @@
+"""Neighbour pairs of the P1 operators as finished blocks inside the
+every-ordered-pair sweep: each operator and rule, with few pairs (many lanes per
+pair) and with many (few lanes: eight wavenumbers of one mesh), and the
+Burton-Miller systems whose right-hand side and mass terms ride on them.  Against
+the FP64 oracle at the operators' 1e-5."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from neuralat_amd import mesh
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-5
+KS = [3.0, 5.0, 8.0, -6.0, 11.0, 14.0, 2.0, 9.5]
+
+
+def _dev():
+    return torch.device("cuda:0")
+
+
+def _rel(a, b):
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
+
+
+@pytest.fixture(scope="module")
+def surface():
+    v, t = mesh.icosphere(2, 0.2)
+    return mesh.sh_perturb(v, 4, 0.05, seed=8).astype(np.float32), t
+
+
+def _solver(surface, clamp=True):
+    from neuralat_amd.bem import BEM_Solver
+
+    v, t = surface
+    return BEM_Solver(torch.tensor(v, device=_dev()), torch.tensor(t, device=_dev()), clamp=clamp)
+
+
+@pytest.mark.parametrize("quad", ["full", "approx", "approx1"])
+@pytest.mark.parametrize("op", ["double", "adjointdouble", "bm_lhs", "bm_rhs"])
+def test_operator_blocks(surface, op, quad):
+    v, t = surface
+    s = _solver(surface)
+    approx = {"full": False, "approx": True, "approx1": "approx_1"}[quad]
+    print("p1 pairs", op, quad, s.mesh.n_neighbor_pairs, flush=True)
+    many = s.assemble_boundary_matrix_batch(KS, op, approx=approx)
+    for z in (0, 3, 7):
+        R = oracle.assemble(v, t, KS[z], op, "P1", quad=quad)
+        assert _rel(many[z].cpu().numpy(), R) < TOL, z
+        one = s.assemble_boundary_matrix(KS[z], op, approx=approx)
+        assert _rel(one.cpu().numpy(), R) < TOL, z
+
+
+@pytest.mark.parametrize("clamp", [True, False])
+@pytest.mark.parametrize("quad", ["full", "approx"])
+def test_burton_miller_systems(surface, quad, clamp):
+    v, t = surface
+    s = _solver(surface, clamp)
+    rng = np.random.default_rng(4)
+    g = (rng.standard_normal((len(KS), len(v))) + 1j * rng.standard_normal((len(KS), len(v)))).astype(np.complex64)
+    e = v[t].astype(np.float64)
+    J = np.linalg.norm(np.cross(e[:, 1] - e[:, 0], e[:, 2] - e[:, 0]), axis=1)
+    M = np.zeros((len(v), len(v)))
+    for a in range(3):
+        for b in range(3):
+            np.add.at(M, (t[:, a], t[:, b]), J / 24 * (2.0 if a == b else 1.0))
+    print("burton-miller systems", quad, clamp, flush=True)
+    gt = torch.tensor(g, device=_dev())
+    singles = [s.burton_miller_system(KS[z], gt[z], approx=quad == "approx") for z in (0, 3)]
+    batch = s.burton_miller_systems(KS, gt) if quad == "approx" else None
+    for q, z in enumerate((0, 3)):
+        L = oracle.assemble(v, t, KS[z], "bm_lhs", "P1", quad=quad, clamp=clamp) + 0.5 * M
+        R = oracle.assemble(v, t, KS[z], "bm_rhs", "P1", quad=quad, clamp=clamp) - (0.5j / KS[z]) * M
+        r = R @ g[z].astype(np.complex128)
+        for lhs, rhs in [singles[q]] + ([(batch[0][z], batch[1][z])] if batch else []):
+            assert _rel(lhs.cpu().numpy(), L) < TOL
+            assert _rel(rhs.cpu().numpy(), r) < TOL
