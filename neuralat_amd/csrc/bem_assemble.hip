@@ -929,12 +929,15 @@ __global__ __launch_bounds__(256) void p1_regular_kernel(const float* __restrict
                                                          const int32_t* __restrict__ vmap,
                                                          const float2* __restrict__ rg_g,
                                                          float2* __restrict__ rg_out, int64_t plane,
-                                                         const P1PairBlocks pb)
+                                                         const P1PairBlocks pb, const int rparts)
 {
-    const float k = kb.k[blockIdx.z];
-    out += (int64_t)blockIdx.z * kb.zstride;
-    rec += (int64_t)blockIdx.z * kb.gstride;
-    curls += (int64_t)blockIdx.z * kb.gstride;
+    // rparts workgroups share a row tile's triangles (small grids)
+    const int zb = rparts == 1 ? blockIdx.z : blockIdx.z / rparts;
+    const int rpart = blockIdx.z - zb * rparts;
+    const float k = kb.k[zb];
+    out += (int64_t)zb * kb.zstride;
+    rec += (int64_t)zb * kb.gstride;
+    curls += (int64_t)zb * kb.gstride;
     constexpr int CT = kP1ColTris;  // one lane per column triangle and per column vertex
     constexpr int NCV = kP1ColVerts;
     static_assert(CT == 256 && NCV <= CT, "one lane per column triangle and per column vertex");
@@ -976,7 +979,8 @@ __global__ __launch_bounds__(256) void p1_regular_kernel(const float* __restrict
         own = ct == tl.row_ctile[rt];
     }
     const int c0 = tl.col_ptr[ct], c1 = tl.col_ptr[ct + 1];
-    const int r0 = tl.row_ptr[rt], r1 = tl.row_ptr[rt + 1];
+    const int rper = (tl.row_ptr[rt + 1] - tl.row_ptr[rt] + rparts - 1) / rparts;
+    const int r0 = min(tl.row_ptr[rt] + rpart * rper, tl.row_ptr[rt + 1]), r1 = min(r0 + rper, tl.row_ptr[rt + 1]);
     const int rv0 = tl.row_vptr[rt], nrv = tl.row_vptr[rt + 1] - rv0;
     const int cv0 = tl.col_vptr[ct], ncv = tl.col_vptr[ct + 1] - cv0;
     for (int e = threadIdx.x; e < nrv * ncv; e += CT) acc[e / ncv][e % ncv] = make_float2(0.f, 0.f);
@@ -1017,7 +1021,7 @@ __global__ __launch_bounds__(256) void p1_regular_kernel(const float* __restrict
     const float krev = k * kInv2Pi;
     const float invk = 1.0f / k;
     if constexpr (RG) {  // this launch's vertex vector and partial rows
-        rg_g += (int64_t)blockIdx.z * kb.vstride;
+        rg_g += (int64_t)zb * kb.vstride;
         rg_out += (int64_t)blockIdx.z * tl.ncol_tiles * (int64_t)tl.row_vptr[tl.nrow_tiles];
     }
     // RG: g at the column triangle's quadrature points (caller's vertex ids)
@@ -1162,7 +1166,7 @@ __global__ __launch_bounds__(256) void p1_regular_kernel(const float* __restrict
         // before its flush.  Looked up inside the row loop instead, the
         // lookups' latency cost every workgroup near the diagonal a third
         if (pb.blk && __syncthreads_or(near)) {
-            const float2* blk = pb.blk + (int64_t)blockIdx.z * pb.npairs * 9;
+            const float2* blk = pb.blk + (int64_t)zb * pb.npairs * 9;
             for (int q = threadIdx.x >> 6; q < r1 - r0; q += CT / 64) {
                 const int4 rs = rslot[q];
                 const int64_t e1 = pb.pair_ptr[rtri[q].w + 1];
@@ -1193,6 +1197,7 @@ __global__ __launch_bounds__(256) void p1_regular_kernel(const float* __restrict
             gc = vmap[gc];
         }
         const float2 v = acc[rvi][cvi];
+        if (rparts > 1 && v.x == 0.f && v.y == 0.f) continue;  // a row of the tile's other triangles
         if (plane) {  // real and imaginary planes: a wavefront's 64 atomics span half the cache lines
             float* dst = reinterpret_cast<float*>(out) + (gr * ld + gc);
             unsafeAtomicAdd(dst, v.x);
@@ -1241,6 +1246,7 @@ __global__ __launch_bounds__(256) void p1_regular_kernel(const float* __restrict
                 gc = vmap[gc];
             }
             const float2 v = acc[rvi][cvi];
+            if (rparts > 1 && v.x == 0.f && v.y == 0.f) continue;
             if (plane) {
                 float* dst = reinterpret_cast<float*>(out) + (gc * ld + gr);
                 unsafeAtomicAdd(dst, v.x);
@@ -1396,10 +1402,11 @@ __global__ __launch_bounds__(256) void singular_kernel(const float* __restrict__
     geo += (int64_t)blockIdx.z * kb.gstride;
     curls += (int64_t)blockIdx.z * kb.gstride;
     const int lane = threadIdx.x & 63;
-    // lanes per pair: a wavefront per pair, except the 2-point line rule of the
-    // P1 operators (16 points): 16 lanes per pair, 4 pairs per wavefront, so
-    // the FP64 reductions run over 16 lanes and serve four pairs
-    constexpr int LPP = (NL == 2 && BASIS == P1) ? 16 : 64;
+    // lanes per pair: DP0 a wavefront; P1 16 lanes, four pairs per wavefront, so
+    // the pair's set-up and its twenty FP64 sums serve four pairs (they cost
+    // as much as the 256 points of the 4-point line rule: 25 -> 17 us for the
+    // single layer at 162 vertices, 452 -> 342 us for the double layer at 7842)
+    constexpr int LPP = BASIS == P1 ? 16 : 64;
     constexpr int PPW = 64 / LPP;
     const int ll = lane % LPP;
     const int64_t pw = p0 + ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * PPW;  // the wavefront's first pair
@@ -2136,6 +2143,18 @@ __global__ __launch_bounds__(256) void p1_permute_planar_kernel(const float* __r
 // transposed flush, whose destination rows take 20 values each, cost more
 // than the halved evaluations save); one_sided evaluates every ordered pair.
 constexpr int64_t kP1PairMinVerts = 4096;
+// Workgroups per row tile: a grid that would leave CUs idle splits each row
+// tile's (up to 16) triangles over several workgroups, whose row sweeps are
+// serial (162 vertices, single layer, 6-point rule: 54 us whole, 14 us in 16
+// parts).  The CUs hold three workgroups each, so splits stop at 3 x 256; past
+// that a split only repeats the tile's set-up and flush.
+constexpr int64_t kP1FillGroups = 768;
+static int p1_row_parts(int64_t groups, int nz)
+{
+    int parts = 1;
+    while (parts < kP1RowTris && groups * nz * parts * 2 <= kP1FillGroups) parts *= 2;
+    return parts;
+}
 template <int OP, int Q>
 static bool p1_ordered_sweep(const MeshDev& m, bool one_sided)
 {
@@ -2149,6 +2168,7 @@ static hipError_t p1_regular_t(const MeshDev& m, const KBatch& kb, int nz, float
                                const int32_t* vmap, hipStream_t s, const P1PairBlocks& pb,
                                const float2* rg_g = nullptr, float2* rg_out = nullptr, bool* planar = nullptr)
 {
+    const int64_t tiles = (int64_t)m.tiles.ncol_tiles * m.tiles.nrow_tiles;
     // planar (an [n, n] scratch per z, ld == n): the every-ordered-pair and
     // paired sweeps flush real and imaginary planes; *planar says whether the
     // sweep taken did
@@ -2159,31 +2179,33 @@ static hipError_t p1_regular_t(const MeshDev& m, const KBatch& kb, int nz, float
     constexpr bool pair = (OP == DLP || OP == ADLP) && Q == 6;
     const int64_t plane = planar ? n * n : 0;
     if (!p1_ordered_sweep<OP, Q>(m, one_sided)) {
+        const int parts = p1_row_parts(m.tiles.nsym, nz);
         if constexpr (sym) {
-            hipLaunchKernelGGL((p1_regular_kernel<OP, Q, CLAMP, kSweepSym>), dim3((unsigned)m.tiles.nsym, 1, nz),
+            hipLaunchKernelGGL((p1_regular_kernel<OP, Q, CLAMP, kSweepSym>), dim3((unsigned)m.tiles.nsym, 1, nz * parts),
                                dim3(256), 0, s, rec, m.tris, m.curls, m.tiles, kb, out, ld, vmap, nullptr, nullptr,
-                               (int64_t)0, P1PairBlocks{});
+                               (int64_t)0, P1PairBlocks{}, parts);
             hipLaunchKernelGGL(p1_symmetrize_kernel, dim3((unsigned)(nb * (nb + 1) / 2), 1, nz), dim3(256), 0, s, out,
                                n, ld, kb.zstride);
         } else if constexpr (pair) {
             if (planar) *planar = true;
-            hipLaunchKernelGGL((p1_regular_kernel<OP, Q, CLAMP, kSweepPair>), dim3((unsigned)m.tiles.nsym, 1, nz),
+            hipLaunchKernelGGL((p1_regular_kernel<OP, Q, CLAMP, kSweepPair>), dim3((unsigned)m.tiles.nsym, 1, nz * parts),
                                dim3(256), 0, s, rec, m.tris, m.curls, m.tiles, kb, out, ld, vmap, nullptr, nullptr,
-                               plane, P1PairBlocks{});
+                               plane, P1PairBlocks{}, parts);
         }
         return hipGetLastError();
     }
-    dim3 grid((unsigned)m.tiles.ncol_tiles, (unsigned)m.tiles.nrow_tiles, (unsigned)nz);
+    const int parts = p1_row_parts(tiles, nz);
+    dim3 grid((unsigned)m.tiles.ncol_tiles, (unsigned)m.tiles.nrow_tiles, (unsigned)(nz * parts));
     if (planar) *planar = true;
     if constexpr (OP == BM_LHS) {
         if (rg_out) {
             hipLaunchKernelGGL((p1_regular_kernel<OP, Q, CLAMP, kSweepAllRg>), grid, dim3(256), 0, s, rec, m.tris,
-                               m.curls, m.tiles, kb, out, ld, vmap, rg_g, rg_out, plane, pb);
+                               m.curls, m.tiles, kb, out, ld, vmap, rg_g, rg_out, plane, pb, parts);
             return hipGetLastError();
         }
     }
     hipLaunchKernelGGL((p1_regular_kernel<OP, Q, CLAMP, kSweepAll>), grid, dim3(256), 0, s, rec, m.tris, m.curls,
-                       m.tiles, kb, out, ld, vmap, nullptr, nullptr, plane, pb);
+                       m.tiles, kb, out, ld, vmap, nullptr, nullptr, plane, pb, parts);
     return hipGetLastError();
 }
 
@@ -2192,8 +2214,8 @@ static hipError_t singular_t(const MeshDev& m, int64_t p0, int64_t p1, const KBa
                              int64_t ld, int64_t row0, hipStream_t s)
 {
     if (p1 <= p0) return hipSuccess;
-    // pairs per workgroup: 4 wavefronts, 4 pairs each for the 2-point P1 rule
-    const int64_t per = (NL == 2 && BASIS == P1) ? 16 : 4;
+    // pairs per workgroup: 4 wavefronts, 4 pairs each in the P1 basis
+    const int64_t per = BASIS == P1 ? 16 : 4;
     unsigned g = (unsigned)((p1 - p0 + per - 1) / per);
     // P1 takes every pair (p0 = 0, p1 = npairs): the list grouped by kind
     const int4* pl = BASIS == P1 ? m.pairs_by_kind : m.pairs;
@@ -2205,7 +2227,7 @@ static hipError_t singular_t(const MeshDev& m, int64_t p0, int64_t p1, const KBa
 // Neighbour-pair blocks of a P1 operator (p1_pairs_kernel).  Lanes per pair: 4
 // (2-point line rule, 16 points) or 16 (4-point, 256 points), and four times as
 // many while the pairs are too few to fill the GPU's wavefronts that way.
-constexpr int64_t kPairsFill2 = 1 << 15, kPairsFill4 = 1 << 15;
+constexpr int64_t kPairsFill2 = 1 << 13, kPairsFill4 = 1 << 12;
 template <int OP, bool CLAMP, bool RG>
 static hipError_t launch_p1_pairs(const MeshDev& m, int quad, const KBatch& kb, int nz, float lhs_mass, float2* blk,
                                   const float2* g, float2* rg, hipStream_t s)
@@ -2570,10 +2592,13 @@ static hipError_t bm_system_p1_t(const MeshDev& m, int64_t gstride, const KBatch
     hipError_t e = launch_fill(rhs, nz, n, n, make_float2(0.f, 0.f), s);
     if (e != hipSuccess) return e;
     // scratch: the pairs' blocks and row sums, the regular pairs' row sums (one
-    // partial row per column tile and system), the matrix in the tiles' numbering
+    // partial row per column tile, row part and system), the matrix in the tiles'
+    // numbering
     const int64_t nslots = m.h_row_slots;
     const size_t nblk = 9 * (size_t)m.npairs * nz, nrg = 3 * (size_t)m.npairs * nz,
-                 npart = (size_t)m.tiles.ncol_tiles * (size_t)nslots * nz, nmat = (size_t)n * (size_t)n * nz;
+                 nrows = (size_t)m.tiles.ncol_tiles *
+                         (size_t)p1_row_parts((int64_t)m.tiles.ncol_tiles * m.tiles.nrow_tiles, nz),
+                 npart = nrows * (size_t)nslots * nz, nmat = (size_t)n * (size_t)n * nz;
     float2* blk = nullptr;
     bool mat = hipMallocAsync((void**)&blk, sizeof(float2) * (nblk + nrg + npart + nmat), s) == hipSuccess;
     if (!mat) {
@@ -2611,7 +2636,7 @@ static hipError_t bm_system_p1_t(const MeshDev& m, int64_t gstride, const KBatch
     }
     if (e == hipSuccess) {
         hipLaunchKernelGGL(p1_rg_reduce_kernel, dim3(grid1d(nslots), (unsigned)nz), dim3(256), 0, s,
-                           (const float2*)part, m.tiles.ncol_tiles, nslots, m.tiles.row_verts, m.p1_vold, rhs, n);
+                           (const float2*)part, (int)nrows, nslots, m.tiles.row_verts, m.p1_vold, rhs, n);
         hipLaunchKernelGGL(p1_pairs_rhs_kernel, dim3((unsigned)((4 * n + 255) / 256), (unsigned)nz), dim3(256), 0, s,
                            (const float2*)rg, m.npairs, m.pair_ptr, m.vt_ptr, m.vt_corner, n, rhs, n);
         e = hipGetLastError();
