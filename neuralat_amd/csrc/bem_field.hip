@@ -131,18 +131,28 @@ __global__ __launch_bounds__(64 * kFieldWaves) void field_kernel(const float* __
         out[(int64_t)z * np + p] = make_float2((float)accr, (float)acci);
 }
 
-// out[z][p] = sum over the triangle splits, in order
+// out[z][p] = sum over the triangle splits: a workgroup takes 16 points, 16
+// threads each every 16th split, combined in order
 __global__ __launch_bounds__(256) void field_reduce_kernel(const double2* __restrict__ part, int ns, int64_t np,
                                                            float2* __restrict__ out)
 {
-    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (p >= np) return;
-    part += (int64_t)blockIdx.y * ns * np + p;
+    __shared__ double2 red[16][16];
+    const int q = threadIdx.x & 15, sl = threadIdx.x >> 4;
+    const int64_t p = (int64_t)blockIdx.x * 16 + q;
+    part += (int64_t)blockIdx.y * ns * np;
     double sr = 0.0, si = 0.0;
-    for (int s = 0; s < ns; ++s) {
-        const double2 v = part[(int64_t)s * np];
-        sr += v.x;
-        si += v.y;
+    if (p < np)
+        for (int s = sl; s < ns; s += 16) {
+            const double2 v = part[(int64_t)s * np + p];
+            sr += v.x;
+            si += v.y;
+        }
+    red[sl][q] = make_double2(sr, si);
+    __syncthreads();
+    if (sl != 0 || p >= np) return;
+    for (int s = 1; s < 16; ++s) {
+        sr += red[s][q].x;
+        si += red[s][q].y;
     }
     out[(int64_t)blockIdx.y * np + p] = make_float2((float)sr, (float)si);
 }
@@ -210,7 +220,7 @@ hipError_t launch_field(const MeshDev& mg, int64_t gstride, const float* pts, in
             hipLaunchKernelGGL(field_kernel<false>, grid, dim3(64 * kFieldWaves), 0, s, rec, nt, pz, np, kb,
                                (const float4*)pre, sp.tper, part, oz);
         if (part)
-            hipLaunchKernelGGL(field_reduce_kernel, dim3((unsigned)((np + 255) / 256), (unsigned)nz), dim3(256), 0, s,
+            hipLaunchKernelGGL(field_reduce_kernel, dim3((unsigned)((np + 15) / 16), (unsigned)nz), dim3(256), 0, s,
                                (const double2*)part, sp.ns, np, oz);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
