@@ -31,6 +31,7 @@ constexpr int kChunkMaxQ = 1024;     // basis vectors (their coefficients sit in
 constexpr int kChunkMaxPart = 4096;  // partial sums per system: 64 KB each workgroup reads
 constexpr int kLdsThreads = 1024;
 constexpr size_t kLdsBytes = 128 << 10;  // of a CU's 160 KB
+constexpr int64_t kLdsMaxN = 2048;       // one workgroup took 40 us at 8000 unknowns, the chunked form 24
 
 // system s: its length and where its vectors start
 struct SysView {
@@ -391,13 +392,13 @@ void arnoldi_set_part(ArnoldiDesc& D, double2* part, double* partn)
 
 bool arnoldi_fused(const ArnoldiDesc& D, int j)
 {
-    return lds_bytes(D.n, j) <= kLdsBytes || j < D.qcap;
+    return (D.n <= kLdsMaxN && lds_bytes(D.n, j) <= kLdsBytes) || j < D.qcap;
 }
 
 hipError_t launch_arnoldi_step(const ArnoldiDesc& D, int j, int passes, hipStream_t s)
 {
     const size_t lb = lds_bytes(D.n, j);
-    if (lb <= kLdsBytes) {
+    if (D.n <= kLdsMaxN && lb <= kLdsBytes) {
         if (lb > (64 << 10)) {  // more than the default limit of dynamic LDS
             const hipError_t e = hipFuncSetAttribute((const void*)arnoldi_lds_kernel,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
