@@ -161,13 +161,6 @@ __global__ __launch_bounds__(256) void dp0_regular_kernel(const float* __restric
 constexpr int kSymBlock = 64;
 constexpr int kStageCols = 16;
 
-__device__ __forceinline__ float wave_sum_f32(float v)
-{
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 // block pair index p -> (I, J), I <= J, p = J (J + 1) / 2 + I
 __device__ __forceinline__ void tri_block_pair(int64_t p, int64_t& I, int64_t& J)
 {
@@ -278,11 +271,10 @@ __device__ __forceinline__ void cbie_sym_task(const float* __restrict__ rec, con
                                 ti4.y == tj.y || ti4.y == tj.z || ti4.z == tj.x || ti4.z == tj.y || ti4.z == tj.z;
             const bool use = valid && !shared;
             const float2 pi_ = psi[i];
-            float rsr = use ? vr * pj.x - vi * pj.y : 0.f;
-            float rsi = use ? vr * pj.y + vi * pj.x : 0.f;
-            rsr = wave_sum_f32(rsr);
-            rsi = wave_sum_f32(rsi);
-            if (lane == 0) prow[J * nt + i] = make_float2(rsr, rsi);
+            const float rsr = use ? vr * pj.x - vi * pj.y : 0.f;
+            const float rsi = use ? vr * pj.y + vi * pj.x : 0.f;
+            const float rs = wave_sum_pair(rsr, rsi);  // real in the low half, imaginary in the high
+            if ((lane & 31) == 0) reinterpret_cast<float*>(&prow[J * nt + i])[lane >> 5] = rs;
             if (use) {
                 cr_acc = fmaf(vr, pi_.x, fmaf(-vi, pi_.y, cr_acc));
                 ci_acc = fmaf(vr, pi_.y, fmaf(vi, pi_.x, ci_acc));
@@ -818,10 +810,19 @@ __device__ __forceinline__ void p1_pair_block_bm3(const float* __restrict__ rr, 
     const float nx0 = rr[4 * Q], nx1 = rr[4 * Q + 1], nx2 = rr[4 * Q + 2];
     // (x_0 - y_b).n_x per column point (constant along the row plane)
     float qn[Q];
+    // RG: qn ghat and (i / k) qn ghat
+    float qgr[RG ? Q : 1], qgi[RG ? Q : 1], qhr[RG ? Q : 1], qhi[RG ? Q : 1];
     if constexpr (OP == BM_RHS || RG) {
 #pragma unroll
-        for (int b = 0; b < Q; ++b)
+        for (int b = 0; b < Q; ++b) {
             qn[b] = -((py[3 * b] - rr[0]) * nx0 + (py[3 * b + 1] - rr[1]) * nx1 + (py[3 * b + 2] - rr[2]) * nx2);
+            if constexpr (RG) {
+                qgr[b] = qn[b] * ghat[2 * b];
+                qgi[b] = qn[b] * ghat[2 * b + 1];
+                qhr[b] = -qgi[b] * invk;
+                qhi[b] = qgr[b] * invk;
+            }
+        }
     }
     float qw[Q], qkw[Q];  // BM_RHS: w qn and w qn / k
     if constexpr (OP == BM_RHS) {
@@ -867,11 +868,11 @@ __device__ __forceinline__ void p1_pair_block_bm3(const float* __restrict__ rr, 
                 gsr += gr;
                 gsi += gi;
                 if constexpr (RG) {
-                    // RHS: (x - y).n_x / r - 1 + i (x - y).n_x / (k r^2), times g(y_b)
-                    const float e2r = fmaf(qn[b], rinv, -1.0f), e2i = qn[b] * invk * rinv2;
-                    const float v2r = gr * e2r - gi * e2i, v2i = gr * e2i + gi * e2r;
-                    tr_[a] = fmaf(v2r, ghat[2 * b], fmaf(-v2i, ghat[2 * b + 1], tr_[a]));
-                    ti_[a] = fmaf(v2r, ghat[2 * b + 1], fmaf(v2i, ghat[2 * b], ti_[a]));
+                    // RHS: [(x - y).n_x / r - 1 + i (x - y).n_x / (k r^2)] g(y_b), times G
+                    const float e2r = fmaf(qhr[b], rinv2, fmaf(qgr[b], rinv, -ghat[2 * b]));
+                    const float e2i = fmaf(qhi[b], rinv2, fmaf(qgi[b], rinv, -ghat[2 * b + 1]));
+                    tr_[a] = fmaf(gr, e2r, fmaf(-gi, e2i, tr_[a]));
+                    ti_[a] = fmaf(gr, e2i, fmaf(gi, e2r, ti_[a]));
                 }
             } else {
                 // w [-1 + (i/k)(1 - i k r)(x - y).n_x / r^2]
@@ -1026,7 +1027,9 @@ __global__ __launch_bounds__(256) void p1_regular_kernel(const float* __restrict
     }
     // RG: g at the column triangle's quadrature points (caller's vertex ids)
     float ghat[RG ? 2 * Q : 1];
-    float2 rgacc = make_float2(0.f, 0.f);  // RG: lane 3 r + c keeps row triangle r's corner c
+    // RG: lane 16 g + r keeps row triangle r's corner sums as wave_sum_six
+    // leaves them in row group g
+    float rgp = 0.f, rgq = 0.f;
     if constexpr (RG) {
         const float2 g0 = rg_g[tj.x], g1 = rg_g[tj.y], g2 = rg_g[tj.z];
 #pragma unroll
@@ -1118,12 +1121,16 @@ __global__ __launch_bounds__(256) void p1_regular_kernel(const float* __restrict
                 p1_pair_block<OP, Q, CLAMP, PAIR, EOP, RG>(rrec[rp - r0], ci, py, wy, ny0, ny1, ny2, cj, k, krev,
                                                             invk, br, bi, tr, tii, ghat, rgs);
         }
-        if constexpr (RG) {  // the row triangle's three corner sums over this wavefront's columns
-            const int lane = threadIdx.x & 63;
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                const float sr = wave_sum_f32(rgs[2 * c]), si = wave_sum_f32(rgs[2 * c + 1]);
-                if (lane == 3 * (rp - r0) + c) rgacc = make_float2(sr, si);
+        // RG: the row triangle's three corner sums over this wavefront's columns
+        // (by half and row exchanges; as six permuted sums of one value each they
+        // were 36 LDS operations a row: Burton-Miller system of 3612 vertices
+        // 1132 us a pass, now 1070)
+        if constexpr (RG) {
+            float p, q;
+            wave_sum_six(rgs, p, q);
+            if ((int)(threadIdx.x & 15) == rp - r0) {
+                rgp = p;
+                rgq = q;
             }
         }
         if (!kBm3 || eval) {
@@ -1214,13 +1221,12 @@ __global__ __launch_bounds__(256) void p1_regular_kernel(const float* __restrict
         // (rg_out [ncol_tiles, row slots]; p1_rg_reduce_kernel sums the
         // column tiles in a fixed order): no global atomics, which at level 6
         // (every row vertex hit from 320 column tiles) serialised the kernel
-        const int lane = threadIdx.x & 63;
-        if (lane < 3 * (r1 - r0)) {
-            const int4 rs = rslot[lane / 3];
-            const int c = lane % 3;
-            const int slot = c == 0 ? rs.x : (c == 1 ? rs.y : rs.z);
-            atomicAdd(&rgslot[slot].x, rgacc.x);
-            atomicAdd(&rgslot[slot].y, rgacc.y);
+        const int r = threadIdx.x & 15, g = (threadIdx.x >> 4) & 3;  // g: re 0, re 1, im 0, im 1 of corners 0 and 1
+        if (r < r1 - r0) {
+            const int4 rs = rslot[r];
+            float2* dst = &rgslot[g & 1 ? rs.y : rs.x];
+            atomicAdd(g & 2 ? &dst->y : &dst->x, rgp);
+            if (!(g & 1)) atomicAdd(g & 2 ? &rgslot[rs.z].y : &rgslot[rs.z].x, rgq);
         }
         __syncthreads();
         const int64_t nslots = tl.row_vptr[tl.nrow_tiles];

@@ -119,7 +119,53 @@ __device__ __forceinline__ double wave_sum64(double v)
     v += __shfl_xor(v, 16, 64);
     return v + __shfl_xor(v, 32, 64);
 }
-// the same over each 16-lane row alone
+// Two values' sums over a wavefront: lanes 0-31 end with a's, lanes 32-63 with
+// b's.  The lane-half and odd-even row exchanges swap between two registers, so
+// one exchange and one addition serve both values and nothing goes through LDS
+// (six permutes a value before).
+__device__ __forceinline__ void swap_half(float& a, float& b)  // a.hi <-> b.lo
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap_row(float& a, float& b)  // a's rows 1, 3 <-> b's rows 0, 2
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float row_sum16(float v)
+{
+    v += dpp_row_f<0xB1>(v);
+    v += dpp_row_f<0x4E>(v);
+    v += dpp_row_f<0x141>(v);
+    return v + dpp_row_f<0x140>(v);
+}
+__device__ __forceinline__ float wave_sum_pair(float a, float b)
+{
+    swap_half(a, b);
+    float c = a + b, d = c;
+    swap_row(c, d);
+    return row_sum16(c + d);
+}
+// Six values' sums: by 16-lane row, p holds v0, v2, v1, v3 and q holds v4, v4, v5, v5
+__device__ __forceinline__ void wave_sum_six(const float* v, float& p, float& q)
+{
+    float a = v[0], b = v[1], c = v[2], d = v[3], e = v[4], f = v[5];
+    swap_half(a, b);
+    swap_half(c, d);
+    swap_half(e, f);
+    a += b;
+    c += d;
+    e += f;
+    f = e;
+    swap_row(a, c);
+    swap_row(e, f);
+    p = row_sum16(a + c);
+    q = row_sum16(e + f);
+}
+// a sum over each 16-lane row alone
 __device__ __forceinline__ double row_sum16(double v)
 {
     v += dpp_row_d<0xB1>(v);
