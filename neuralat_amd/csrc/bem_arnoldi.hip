@@ -31,7 +31,8 @@ constexpr int kChunkMaxQ = 1024;     // basis vectors (their coefficients sit in
 constexpr int kChunkMaxPart = 4096;  // partial sums per system: 64 KB each workgroup reads
 constexpr int kLdsThreads = 1024;
 constexpr size_t kLdsBytes = 128 << 10;  // of a CU's 160 KB
-constexpr int64_t kLdsMaxN = 2048;       // one workgroup took 40 us at 8000 unknowns, the chunked form 24
+// one workgroup takes 15 us a step at 3380 unknowns, 25 at 5120, 40 at 8000; the chunked form 24 to 28
+constexpr int64_t kLdsMaxN = 5120;
 
 // system s: its length and where its vectors start
 struct SysView {
