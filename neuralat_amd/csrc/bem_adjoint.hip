@@ -146,10 +146,19 @@ __device__ __forceinline__ void column_chain(const float* geo_j, const float (*g
 // ---------------------------------------------------------------------------
 // regular pairs (DP0, 6-point rule): lane = column triangle, row tile uniform
 // ---------------------------------------------------------------------------
-constexpr int kAdjRowTile = 64;
+// Bound by vector issue: about 66 slots a Gauss-point pair (107 with the general
+// evaluation; 5120 triangles, row sums and scatter included: 2577 -> 1523 us).
+// What the column plane and the pair keep constant leaves the inner loop: s =
+// (x_a - y_b).n_y per row point, the n_y part of the position gradients (its
+// coefficients A2 are summed, the normal applied once), the factors 2 and k.
+// A row triangle's ten sums over a wavefront go to LDS; the tile's row triangles
+// are chained to their vertices at its end, a lane each (one lane a row and
+// wavefront before, with nine single-lane FP64 atomics).  32 rows a tile: at
+// 5120 triangles 64 left 1.5 rounds of workgroups.
+constexpr int kAdjRowTile = 32;
 
 template <bool CLAMP>
-__global__ __launch_bounds__(256) void adj_regular_kernel(const float* __restrict__ rec, const float* __restrict__ geo,
+__global__ __launch_bounds__(256, 3) void adj_regular_kernel(const float* __restrict__ rec, const float* __restrict__ geo,
                                                           const int4* __restrict__ tris, int64_t nt, float k,
                                                           const float2* __restrict__ lam,
                                                           const float2* __restrict__ psi,
@@ -158,7 +167,10 @@ __global__ __launch_bounds__(256) void adj_regular_kernel(const float* __restric
 {
     constexpr int Q = 6;
     constexpr int S = Rec<Q>::kFloats;
-    const int lane = threadIdx.x & 63;
+    // per wavefront and row: -1/2 x the nine vertex gradients, 1/2 x e
+    __shared__ float rowsum[4][kAdjRowTile][10];
+    __shared__ float gkw[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const bool active = j < nt;
     const int64_t jj = active ? j : nt - 1;
@@ -171,12 +183,13 @@ __global__ __launch_bounds__(256) void adj_regular_kernel(const float* __restric
     const float ny0 = cr[4 * Q], ny1 = cr[4 * Q + 1], ny2 = cr[4 * Q + 2];
     const int4 tj = tris[jj];
     const float2 psj = psi[jj], phj = phi[jj];
-    const float krev = k * kInv2Pi;
+    const float krev = k * kInv2Pi, k2 = k * k, k3 = -3.f * k;
 
-    float gy[Q][3];
+    // half gradients: gy[b] without, gs[b] the coefficients of the n_y part
+    float gy[Q][3], gs[Q];
 #pragma unroll
-    for (int b = 0; b < Q; ++b) gy[b][0] = gy[b][1] = gy[b][2] = 0.f;
-    float gn[3] = {0.f, 0.f, 0.f}, ecol = 0.f, gk = 0.f, vr = 0.f, vi = 0.f;
+    for (int b = 0; b < Q; ++b) gy[b][0] = gy[b][1] = gy[b][2] = gs[b] = 0.f;
+    float gn[3] = {0.f, 0.f, 0.f}, ecol = 0.f, gk = 0.f, gks = 0.f, vr = 0.f, vi = 0.f;
 
     const int64_t i_begin = (int64_t)blockIdx.y * kAdjRowTile;
     const int64_t i_end = min(i_begin + (int64_t)kAdjRowTile, nt);
@@ -192,79 +205,128 @@ __global__ __launch_bounds__(256) void adj_regular_kernel(const float* __restric
         const float br = on ? (li.x * phj.x + li.y * phj.y) : 0.f;
         const float bi = on ? (li.x * phj.y - li.y * phj.x) : 0.f;
         const float* rr = rec + i * S;
-        float gxv[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-        float erow = 0.f, pv_r = 0.f, pv_i = 0.f;
+        float red[10] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        float pv_r = 0.f, pv_i = 0.f;
 #pragma unroll 1
         for (int a = 0; a < Q; ++a) {
             const float xa0 = rr[3 * a], xa1 = rr[3 * a + 1], xa2 = rr[3 * a + 2];
             const float ua = rr[3 * Q + a];
-            float gxa[3] = {0.f, 0.f, 0.f};
+            const float s = (py[0] - xa0) * ny0 + (py[1] - xa1) * ny1 + (py[2] - xa2) * ny2;
+            float gxa[3] = {0.f, 0.f, 0.f}, gsa = 0.f;
 #pragma unroll
             for (int b = 0; b < Q; ++b) {
-                AdjEval o;
-                adj_eval<CLAMP>(py[3 * b] - xa0, py[3 * b + 1] - xa1, py[3 * b + 2] - xa2, ny0, ny1, ny2, k, krev, ar,
-                                ai, br, bi, o);
-                const float w = ua * wy[b];
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    gxa[c] -= w * o.gd[c];
-                    gy[b][c] += w * o.gd[c];
-                    gn[c] += w * o.gn[c];
-                }
-                erow += w * o.e;
-                gk += w * o.gk;
-                pv_r += w * o.gr;
-                pv_i += w * o.gi;
+                const float dx = py[3 * b] - xa0, dy = py[3 * b + 1] - xa1, dz = py[3 * b + 2] - xa2;
+                float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                const bool clamped = CLAMP && r2 < kEps2;
+                if (CLAMP) r2 = fmaxf(r2, kEps2);
+                const float rinv = __builtin_amdgcn_rsqf(r2);
+                const float r = r2 * rinv;
+                float sn, cs;
+                sincos_rev(r * krev, sn, cs);
+                const float wr = rinv * (ua * wy[b]);
+                const float gr = cs * wr, gi = sn * wr;  // the weighted G
+                const float agr = ar * gr - ai * gi, agi = ar * gi + ai * gr;
+                const float bgr = br * gr - bi * gi, bgi = br * gi + bi * gr;
+                // Re(alpha G q + beta G c1), c1 = s / r (3 / r^2 - k^2 - 3 i k / r)
+                const float rinv2 = rinv * rinv, sr = s * rinv;
+                const float c1r = sr * fmaf(3.f, rinv2, -k2), c1i = sr * (k3 * rinv);
+                const float A1 = fmaf(bgr, c1r, fmaf(-bgi, c1i, fmaf(-agr, rinv, -agi * k)));
+                const float A2 = -fmaf(bgr, rinv, bgi * k) * rinv;  // Re(beta G q) / r
+                const float w1 = clamped ? 0.f : A1 * rinv;
+                gxa[0] = fmaf(w1, dx, gxa[0]);
+                gxa[1] = fmaf(w1, dy, gxa[1]);
+                gxa[2] = fmaf(w1, dz, gxa[2]);
+                gsa += A2;
+                gy[b][0] = fmaf(w1, dx, gy[b][0]);
+                gy[b][1] = fmaf(w1, dy, gy[b][1]);
+                gy[b][2] = fmaf(w1, dz, gy[b][2]);
+                gs[b] += A2;
+                gn[0] = fmaf(A2, dx, gn[0]);
+                gn[1] = fmaf(A2, dy, gn[1]);
+                gn[2] = fmaf(A2, dz, gn[2]);
+                red[9] += fmaf(A2, s, agr);
+                gk = fmaf(r, agi, gk);
+                gks = fmaf(s, bgr, gks);
+                pv_r += gr;
+                pv_i += gi;
             }
+            gxa[0] = fmaf(gsa, ny0, gxa[0]);
+            gxa[1] = fmaf(gsa, ny1, gxa[1]);
+            gxa[2] = fmaf(gsa, ny2, gxa[2]);
             const float p1 = c_rule6_x1[a], p2 = c_rule6_x2[a], p0 = 1.f - p1 - p2;
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-                gxv[0][c] += p0 * gxa[c];
-                gxv[1][c] += p1 * gxa[c];
-                gxv[2][c] += p2 * gxa[c];
+                red[c] = fmaf(p0, gxa[c], red[c]);
+                red[3 + c] = fmaf(p1, gxa[c], red[3 + c]);
+                red[6 + c] = fmaf(p2, gxa[c], red[6 + c]);
             }
         }
-        ecol += erow;
+        ecol += red[9];
         // V^H lambda: conj(V_ij) l_i
         if (on) {
             vr += pv_r * li.x + pv_i * li.y;
             vi += pv_r * li.y - pv_i * li.x;
         }
-        // row triangle: reduce over the 64 columns of this wavefront
+        // the row triangle's sums over the 64 columns of this wavefront
+        float p, q;
+        wave_sum_six(red, p, q);
+        const float t = wave_sum_four(red + 6);
+        const int g = lane >> 4, o4 = (g & 1) * 2 + (g >> 1);  // row group -> value index 0, 2, 1, 3
+        float* dst = rowsum[wave][i - i_begin];
+        if ((lane & 15) == 0) {
+            dst[o4] = p;
+            dst[6 + o4] = t;
+            if (!(g & 1)) dst[4 + (g >> 1)] = q;
+        }
+    }
+    __syncthreads();
+    if (i_begin + (int)threadIdx.x < i_end) {
+        const int64_t i = i_begin + threadIdx.x;
         float red[10];
+#pragma unroll
+        for (int e = 0; e < 10; ++e)
+            red[e] = (float)(((double)rowsum[0][threadIdx.x][e] + rowsum[1][threadIdx.x][e]) +
+                             ((double)rowsum[2][threadIdx.x][e] + rowsum[3][threadIdx.x][e]));
+        const float* gi = geo + i * 16;
+        float gv[3][3];
 #pragma unroll
         for (int a = 0; a < 3; ++a)
 #pragma unroll
-            for (int c = 0; c < 3; ++c) red[3 * a + c] = wsum(gxv[a][c]);
-        red[9] = wsum(erow);
-        if (lane == 0) {
-            const float* gi = geo + i * 16;
-            float gv[3][3];
-#pragma unroll
-            for (int a = 0; a < 3; ++a)
-#pragma unroll
-                for (int c = 0; c < 3; ++c) gv[a][c] = red[3 * a + c];
-            const float eJ = red[9] / gi[12];
-            const float gc[3] = {eJ * gi[9], eJ * gi[10], eJ * gi[11]};
-            chain_c(gi, gc, gv);
-            add_vertex_grads(gvert, ti, gv);
-        }
+            for (int c = 0; c < 3; ++c) gv[a][c] = -2.f * red[3 * a + c];
+        const float eJ = 2.f * red[9] / gi[12];
+        const float gc[3] = {eJ * gi[9], eJ * gi[10], eJ * gi[11]};
+        chain_c(gi, gc, gv);
+        add_vertex_grads(gvert, tris[i], gv);
     }
     if (active) {
         float gv[3][3];
-        column_chain(geo + jj * 16, gy, TriRule<Q>::x1, TriRule<Q>::x2, Q, gn, ecol, gv);
+#pragma unroll
+        for (int b = 0; b < Q; ++b) {
+            gy[b][0] = 2.f * fmaf(gs[b], ny0, gy[b][0]);
+            gy[b][1] = 2.f * fmaf(gs[b], ny1, gy[b][1]);
+            gy[b][2] = 2.f * fmaf(gs[b], ny2, gy[b][2]);
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) gn[c] *= 2.f;
+        column_chain(geo + jj * 16, gy, TriRule<Q>::x1, TriRule<Q>::x2, Q, gn, 2.f * ecol, gv);
         add_vertex_grads(gvert, tj, gv);
         vhl_part[(int64_t)blockIdx.y * nt + j] = make_float2(vr, vi);
     }
-    const float gks = wsum(gk);
-    if (lane == 0) unsafeAtomicAdd(gk_out, (double)gks);
+    const float gksum = wsum(-2.f * fmaf(k, gks, gk));
+    if (lane == 0) gkw[wave] = gksum;
+    __syncthreads();
+    if (threadIdx.x == 0) unsafeAtomicAdd(gk_out, ((double)gkw[0] + gkw[1]) + ((double)gkw[2] + gkw[3]));
 }
 
 // ---------------------------------------------------------------------------
 // neighbour pairs: Sauter-Schwab, one wavefront per pair
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double wsum_d(double v) { return wave_sum64(v); }
-
+// 16 lanes per pair: the set-up, the sums over lanes, the chain to the vertices
+// and the scatter serve four pairs of a wavefront (grouped by kind, so that the
+// four take the same region loop), and dk is added once a workgroup (every pair's
+// FP64 atomic met at one address).  The gradient of corner 0 follows from the
+// total, so 22 FP64 sums are kept, not 25.  66560 pairs: 905 -> 240 us (a
+// wavefront per pair before).
 template <bool CLAMP>
 __global__ __launch_bounds__(256) void adj_singular_kernel(const float* __restrict__ geo, const int4* __restrict__ tris,
                                                            const int4* __restrict__ pairs, int64_t npairs, float k,
@@ -274,112 +336,88 @@ __global__ __launch_bounds__(256) void adj_singular_kernel(const float* __restri
                                                            double* __restrict__ gvert, double* __restrict__ gk_out,
                                                            double* __restrict__ vhl)
 {
-    constexpr int NL = 4;
-    const int lane = threadIdx.x & 63;
-    const int64_t p = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (p >= npairs) return;  // uniform per wavefront
-    const int4 pr = pairs[p];
-    const int i = __builtin_amdgcn_readfirstlane(pr.x);
-    const int j = __builtin_amdgcn_readfirstlane(pr.y);
-    const int shared = __builtin_amdgcn_readfirstlane(pr.z);
-    const int4 ti = tris[i], tj = tris[j];
-    const int ia[3] = {ti.x, ti.y, ti.z}, ja[3] = {tj.x, tj.y, tj.z};
-    int pi[3] = {0, 1, 2}, pj[3] = {0, 1, 2};
-    if (shared == 2) {
-        int c = 0;
-        for (int b = 0; b < 3; ++b)
-            for (int a = 0; a < 3; ++a)
-                if (ia[a] == ja[b]) { pi[c] = a; pj[c] = b; ++c; }
-        pi[2] = 3 - pi[0] - pi[1];
-        pj[2] = 3 - pj[0] - pj[1];
-    } else if (shared == 1) {
-        for (int a = 0; a < 3; ++a)
-            for (int b = 0; b < 3; ++b)
-                if (ia[a] == ja[b]) {
-                    if (a != 0) { pi[0] = a; pi[a] = 0; }
-                    if (b != 0) { pj[0] = b; pj[b] = 0; }
-                }
-    }
-    const float* gi = geo + (int64_t)i * 16;
-    const float* gj = geo + (int64_t)j * 16;
-    float v[3][3], w[3][3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            v[a][d] = gi[3 * pi[a] + d];
-            w[a][d] = gj[3 * pj[a] + d];
-        }
-    float e1[3], e2[3], f1[3], f2[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        e1[d] = v[1][d] - v[0][d];
-        e2[d] = v[2][d] - v[1][d];
-        f1[d] = w[1][d] - w[0][d];
-        f2[d] = w[2][d] - w[1][d];
-    }
-    const float ny0 = gj[9], ny1 = gj[10], ny2 = gj[11];
-    const float jij = gi[12] * gj[12];
+    constexpr int NL = 4, LPP = 16;
+    __shared__ double gks[256 / LPP];
+    const int ll = threadIdx.x % LPP;
+    const int64_t p = (int64_t)blockIdx.x * (256 / LPP) + threadIdx.x / LPP;
+    const bool valid = p < npairs;  // groups past the end work on the last pair and add nothing
+    const int4 pr = pairs[valid ? p : npairs - 1];
+    const int i = pr.x, j = pr.y;
+    SSPair g;
+    ss_pair_setup(geo, tris, i, j, pr.z, g);
+    const float ny0 = g.ny[0], ny1 = g.ny[1], ny2 = g.ny[2];
     const float krev = k * kInv2Pi;
     const float2 li = lam[i], psj = psi[j], phj = phi[j];
     const float ar = -(li.x * psj.x + li.y * psj.y) * kInv4Pi, ai = -(li.x * psj.y - li.y * psj.x) * kInv4Pi;
     const float br = (li.x * phj.x + li.y * phj.y) * kInv4Pi, bi = (li.x * phj.y - li.y * phj.x) * kInv4Pi;
 
-    // accumulators (reordered local vertices): row 9, col 9, gn 3, e 1, gk 1, V 2
-    double acc[25];
+    // (reordered corners) total 3, row corners 1 and 2, column corners 1 and 2, gn 3, e, gk, V 2
+    double acc[22];
 #pragma unroll
-    for (int e = 0; e < 25; ++e) acc[e] = 0.0;
+    for (int e = 0; e < 22; ++e) acc[e] = 0.0;
     constexpr int NP = NL * NL * NL * NL;
-    ss_dispatch(shared, [&](auto kind) {
+    ss_dispatch(pr.z, [&](auto kind) {
         constexpr int S = decltype(kind)::value;
         constexpr int NR = kSSRegions<S>;
-        for (int q = lane; q < NP; q += 64) {
+        for (int q = ll; q < NP; q += LPP) {
             const int q0 = q / (NL * NL * NL), q1 = (q / (NL * NL)) % NL, q2 = (q / NL) % NL, q3 = q % NL;
             const float wq =
                 LineRule01<NL>::w[q0] * LineRule01<NL>::w[q1] * LineRule01<NL>::w[q2] * LineRule01<NL>::w[q3];
             float reg[NR][7];
             const float jac = ss_regions<S>(LineRule01<NL>::t[q0], LineRule01<NL>::t[q1], LineRule01<NL>::t[q2],
                                             LineRule01<NL>::t[q3], reg);
-            const float W = jac * wq * jij;
+            const float W = jac * wq * g.jij;
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
                 const float x1 = reg[r][0], x2 = reg[r][1], y1 = reg[r][2], y2 = reg[r][3];
                 float dx, dy, dz;
-                ss_disp<S>(reg[r], e1, e2, f1, f2, dx, dy, dz);
+                ss_disp<S>(reg[r], g.e1, g.e2, g.f1, g.f2, dx, dy, dz);
                 AdjEval o;
                 adj_eval<CLAMP>(dx, dy, dz, ny0, ny1, ny2, k, krev, ar, ai, br, bi, o);
                 const float ww = W * reg[r][4];
-                const float px[3] = {1.f - x1, x1 - x2, x2};
-                const float py[3] = {1.f - y1, y1 - y2, y2};
 #pragma unroll
-                for (int a = 0; a < 3; ++a)
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) {
-                        acc[3 * a + c] -= (double)(ww * px[a] * o.gd[c]);
-                        acc[9 + 3 * a + c] += (double)(ww * py[a] * o.gd[c]);
-                    }
-#pragma unroll
-                for (int c = 0; c < 3; ++c) acc[18 + c] += (double)(ww * o.gn[c]);
-                acc[21] += (double)(ww * o.e);
-                acc[22] += (double)(ww * o.gk);
-                acc[23] += (double)(ww * o.gr);
-                acc[24] += (double)(ww * o.gi);
+                for (int c = 0; c < 3; ++c) {
+                    const float wd = ww * o.gd[c];
+                    acc[c] += (double)wd;
+                    acc[3 + c] += (double)((x1 - x2) * wd);
+                    acc[6 + c] += (double)(x2 * wd);
+                    acc[9 + c] += (double)((y1 - y2) * wd);
+                    acc[12 + c] += (double)(y2 * wd);
+                    acc[15 + c] += (double)(ww * o.gn[c]);
+                }
+                acc[18] += (double)(ww * o.e);
+                acc[19] += (double)(ww * o.gk);
+                acc[20] += (double)(ww * o.gr);
+                acc[21] += (double)(ww * o.gi);
             }
         }
     });
 #pragma unroll
-    for (int e = 0; e < 25; ++e) acc[e] = wsum_d(acc[e]);
-    if (lane != 0) return;
+    for (int e = 0; e < 22; ++e) acc[e] = row_sum16(acc[e]);
+    if (ll == 0) gks[threadIdx.x / LPP] = valid ? acc[19] : 0.0;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double s = 0.0;
+#pragma unroll
+        for (int e = 0; e < 256 / LPP; ++e) s += gks[e];
+        unsafeAtomicAdd(gk_out, s);
+    }
+    if (ll != 0 || !valid) return;
     // un-permute to the original local vertex order
     float gvi[3][3], gvj[3][3];
 #pragma unroll
-    for (int a = 0; a < 3; ++a)
+    for (int c = 0; c < 3; ++c) {
+        const float rc[3] = {(float)(acc[3 + c] + acc[6 + c] - acc[c]), (float)-acc[3 + c], (float)-acc[6 + c]};
+        const float cc[3] = {(float)(acc[c] - acc[9 + c] - acc[12 + c]), (float)acc[9 + c], (float)acc[12 + c]};
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            gvi[pi[a]][c] = (float)acc[3 * a + c];
-            gvj[pj[a]][c] = (float)acc[9 + 3 * a + c];
+        for (int o = 0; o < 3; ++o) {
+            gvi[o][c] = g.pi[0] == o ? rc[0] : (g.pi[1] == o ? rc[1] : rc[2]);
+            gvj[o][c] = g.pj[0] == o ? cc[0] : (g.pj[1] == o ? cc[1] : cc[2]);
         }
-    const float E = (float)acc[21];
+    }
+    const float* gi = geo + (int64_t)i * 16;
+    const float* gj = geo + (int64_t)j * 16;
+    const float E = (float)acc[18];
     {
         const float eJ = E / gi[12];
         const float gc[3] = {eJ * gi[9], eJ * gi[10], eJ * gi[11]};
@@ -387,7 +425,7 @@ __global__ __launch_bounds__(256) void adj_singular_kernel(const float* __restri
     }
     {
         const float n[3] = {ny0, ny1, ny2};
-        const float gn[3] = {(float)acc[18], (float)acc[19], (float)acc[20]};
+        const float gn[3] = {(float)acc[15], (float)acc[16], (float)acc[17]};
         const float gnn = gn[0] * n[0] + gn[1] * n[1] + gn[2] * n[2];
         const float J = gj[12];
         float gc[3];
@@ -395,11 +433,10 @@ __global__ __launch_bounds__(256) void adj_singular_kernel(const float* __restri
         for (int c = 0; c < 3; ++c) gc[c] = (E * n[c] + gn[c] - gnn * n[c]) / J;
         chain_c(gj, gc, gvj);
     }
-    add_vertex_grads(gvert, ti, gvi);
-    add_vertex_grads(gvert, tj, gvj);
-    unsafeAtomicAdd(gk_out, acc[22]);
-    // conj(V_ij) l_i into (V^H lambda)_j ; V_ij = acc[23..24] / (4 pi)
-    const double Vr = acc[23] * (double)kInv4Pi, Vi = acc[24] * (double)kInv4Pi;
+    add_vertex_grads(gvert, tris[i], gvi);
+    add_vertex_grads(gvert, tris[j], gvj);
+    // conj(V_ij) l_i into (V^H lambda)_j ; V_ij = acc[20..21] / (4 pi)
+    const double Vr = acc[20] * (double)kInv4Pi, Vi = acc[21] * (double)kInv4Pi;
     unsafeAtomicAdd(&vhl[2 * (int64_t)j], Vr * li.x + Vi * li.y);
     unsafeAtomicAdd(&vhl[2 * (int64_t)j + 1], Vr * li.y - Vi * li.x);
 }
@@ -485,6 +522,7 @@ __global__ __launch_bounds__(256) void adj_mass_vhl_kernel(const float* __restri
     chain_c(g, gc, gv);
     add_vertex_grads(gvert, tris[i], gv);
     double sr = 0.0, si = 0.0;
+#pragma unroll 8
     for (int64_t b = 0; b < nby; ++b) {
         const float2 v = vhl_part[b * nt + i];
         sr += v.x;
@@ -515,12 +553,12 @@ hipError_t launch_adjoint_pairs(const MeshDev& m, float k, int clamp, const floa
     else
         hipLaunchKernelGGL(adj_regular_kernel<false>, grid, dim3(256), 0, s, m.rec6, m.geo, m.tris, m.nt, k, lam, psi,
                            phi, gvert, gk, part);
-    const unsigned g = (unsigned)((m.npairs + 3) / 4);
+    const unsigned g = (unsigned)((m.npairs + 15) / 16);
     if (clamp)
-        hipLaunchKernelGGL(adj_singular_kernel<true>, dim3(g), dim3(256), 0, s, m.geo, m.tris, m.pairs, m.npairs, k,
+        hipLaunchKernelGGL(adj_singular_kernel<true>, dim3(g), dim3(256), 0, s, m.geo, m.tris, m.pairs_by_kind, m.npairs, k,
                            lam, psi, phi, gvert, gk, vhl);
     else
-        hipLaunchKernelGGL(adj_singular_kernel<false>, dim3(g), dim3(256), 0, s, m.geo, m.tris, m.pairs, m.npairs, k,
+        hipLaunchKernelGGL(adj_singular_kernel<false>, dim3(g), dim3(256), 0, s, m.geo, m.tris, m.pairs_by_kind, m.npairs, k,
                            lam, psi, phi, gvert, gk, vhl);
     hipLaunchKernelGGL(adj_mass_vhl_kernel, dim3((unsigned)((m.nt + 255) / 256)), dim3(256), 0, s, m.geo, m.tris, m.nt,
                        lam, phi, part, nby, gvert, vhl);

@@ -1327,74 +1327,6 @@ __device__ __forceinline__ double group_sum(double v)
     }
 }
 
-// A neighbour pair made ready for its quadrature: the shared vertices moved to
-// local 0 (and 1) on both triangles, edge vectors, normals, |J_i| |J_j|.
-// Everything is picked by selects: arrays indexed at run time went to scratch
-// memory (128 bytes per lane).
-__device__ __forceinline__ int pick3(const int (&v)[3], int i) { return i == 0 ? v[0] : (i == 1 ? v[1] : v[2]); }
-struct SSPair {
-    int pi[3], pj[3];   // local index in the caller's order of reordered corner a / b
-    int ia[3], ja[3];   // vertex ids (caller's order)
-    float e1[3], e2[3], f1[3], f2[3], nx[3], ny[3];
-    float jij;
-};
-__device__ __forceinline__ void ss_pair_setup(const float* __restrict__ geo, const int4* __restrict__ tris, int i,
-                                              int j, int shared, SSPair& g)
-{
-    const int4 ti = tris[i], tj = tris[j];
-    g.ia[0] = ti.x; g.ia[1] = ti.y; g.ia[2] = ti.z;
-    g.ja[0] = tj.x; g.ja[1] = tj.y; g.ja[2] = tj.z;
-    // m_b: the row corner equal to column corner b, -1 if none
-    auto match = [&](int v) { return ti.x == v ? 0 : (ti.y == v ? 1 : (ti.z == v ? 2 : -1)); };
-    const int m0 = match(tj.x), m1 = match(tj.y), m2 = match(tj.z);
-    g.pi[0] = g.pj[0] = 0;
-    g.pi[1] = g.pj[1] = 1;
-    g.pi[2] = g.pj[2] = 2;
-    if (shared == 2) {
-        // common edge first, same order on both triangles, ordered by position
-        // in the column triangle (integrand.h:351-364)
-        const int ub = m0 < 0 ? 0 : (m1 < 0 ? 1 : 2);
-        g.pj[0] = ub == 0 ? 1 : 0;
-        g.pj[1] = ub == 2 ? 1 : 2;
-        g.pj[2] = ub;
-        g.pi[0] = ub == 0 ? m1 : m0;
-        g.pi[1] = ub == 2 ? m1 : m2;
-        g.pi[2] = 3 - g.pi[0] - g.pi[1];
-    } else if (shared == 1) {
-        // common vertex swapped to local 0 (integrand.h:365-382)
-        const int b = m0 >= 0 ? 0 : (m1 >= 0 ? 1 : 2), a = m0 >= 0 ? m0 : (m1 >= 0 ? m1 : m2);
-        g.pi[0] = a;
-        g.pi[1] = a == 1 ? 0 : 1;
-        g.pi[2] = a == 2 ? 0 : 2;
-        g.pj[0] = b;
-        g.pj[1] = b == 1 ? 0 : 1;
-        g.pj[2] = b == 2 ? 0 : 2;
-    }
-    // geo record: v0 v1 v2 (9), n (3), jac (1), pad
-    const float* gi = geo + (int64_t)i * 16;
-    const float* gj = geo + (int64_t)j * 16;
-    float v[3][3], w[3][3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            v[a][d] = gi[3 * g.pi[a] + d];
-            w[a][d] = gj[3 * g.pj[a] + d];
-        }
-    // x = v0 + x1 (v1 - v0) + x2 (v2 - v1) on (0,0),(1,0),(1,1); the shared
-    // local vertex 0 (v0 = w0 in all three cases) cancels in d = y - x.
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        g.e1[d] = v[1][d] - v[0][d];
-        g.e2[d] = v[2][d] - v[1][d];
-        g.f1[d] = w[1][d] - w[0][d];
-        g.f2[d] = w[2][d] - w[1][d];
-        g.nx[d] = gi[9 + d];
-        g.ny[d] = gj[9 + d];
-    }
-    g.jij = gi[12] * gj[12];
-}
-
 // Writes (DP0: out = alpha * entry) or adds (P1) the pairs' entries.
 template <int OP, int NL, int BASIS, bool CLAMP>
 __global__ __launch_bounds__(256) void singular_kernel(const float* __restrict__ geo, const int4* __restrict__ tris,

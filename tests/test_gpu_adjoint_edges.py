@@ -1,0 +1,35 @@
+"""The DP0 adjoint kernels where their row tiles (32 triangles) and pair groups
+(16 pairs a workgroup) are only partly filled: vertex gradients of 20, 77 and 80
+triangles along random directions against central differences of the FP64 oracle
+pipeline, at the bound of the same comparison on larger meshes (2e-3)."""
+import numpy as np
+import pytest
+import torch
+
+import fp64_grad
+from neuralat_amd import mesh
+from test_gpu_grad import _dev, _loss_gpu, _setup
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("level,drop", [(0, 0), (1, 0), (1, 3)])
+def test_vertex_gradient(level, drop):
+    v, t, pts, src = _setup(level, seed=5)
+    t = t[: len(t) - drop]  # an open surface: the discrete problem stays well posed
+    assert len(np.unique(t)) == len(v)
+    k0 = 2.5
+    vt = torch.tensor(v, device=_dev(), requires_grad=True)
+    print("adjoint edges", len(t), flush=True)
+    L = _loss_gpu(vt, torch.tensor(t, device=_dev()), torch.tensor(k0, device=_dev()), src, torch.tensor(pts, device=_dev()))
+    L.backward()
+    gv = vt.grad.detach().cpu().numpy().astype(np.float64)
+    v64, h = v.astype(np.float64), 1e-6
+    rng = np.random.default_rng(3)
+    ad, fd = [], []
+    for _ in range(6):
+        d = rng.standard_normal(v.shape)
+        d /= np.linalg.norm(d)
+        fd.append((fp64_grad.loss(v64 + h * d, t, k0, src, pts) - fp64_grad.loss(v64 - h * d, t, k0, src, pts)) / (2 * h))
+        ad.append(np.sum(gv * d))
+    assert np.linalg.norm(np.array(ad) - fd) < 2e-3 * np.linalg.norm(fd)
