@@ -66,6 +66,16 @@ template <> struct LineRule01<2> {
     static constexpr float w[2] = {0.5f, 0.5f};
 };
 
+// The 6-point rule's points are two orbits of three: points 0, 2, 3 and points
+// 1, 4, 5, each with one weight, whose c-th point has the shape value 1 - 2 a at
+// corner c and a at the other two.  A corner's sum over an orbit is therefore
+// a * (the sum of the three) + (1 - 3 a) * (its c-th).
+struct TriRule6Orbit {
+    static constexpr float a0 = TriRule<6>::x1[0], a1 = TriRule<6>::x1[1];
+    static_assert(TriRule<6>::x2[0] == a0 && TriRule<6>::x2[2] == a0 && TriRule<6>::x1[3] == a0, "orbit of points 0, 2, 3");
+    static_assert(TriRule<6>::x2[1] == a1 && TriRule<6>::x2[4] == a1 && TriRule<6>::x1[5] == a1, "orbit of points 1, 4, 5");
+};
+
 // ---- per-triangle records ----------------------------------------------------
 // Quadrature record of one triangle for rule Q, float4-aligned:
 //   pts[3Q]   quadrature points (x,y,z interleaved)
