@@ -172,11 +172,11 @@ __device__ __forceinline__ void curl_grads(const cf* s, const cf* V, float invk,
 }  // namespace
 
 // ---------------------------------------------------------------------------
-// regular pairs (3-point rule): lane = column triangle, a row tile of 64 row
+// regular pairs (3-point rule): lane = column triangle, a row tile of 32 row
 // triangles per workgroup row; row-side gradients are reduced over the
 // wavefront per row triangle, column-side ones kept per lane.
 // ---------------------------------------------------------------------------
-constexpr int kAdjP1RowTile = 64;
+constexpr int kAdjP1RowTile = 32;
 
 template <bool CLAMP>
 __global__ __launch_bounds__(256) void adj_bm_p1_regular_kernel(const float* __restrict__ rec,
@@ -190,6 +190,10 @@ __global__ __launch_bounds__(256) void adj_bm_p1_regular_kernel(const float* __r
 {
     constexpr int Q = 3;
     constexpr int S = Rec<Q>::kFloats;
+    // per wavefront and row: its sums, chained to the vertices at the tile's end,
+    // a lane per row triangle (one lane a row and wavefront in the row loop
+    // before; 4500 triangles: 1123 -> 807 us)
+    __shared__ float rowsum[4][kAdjP1RowTile][19];
     const int lane = threadIdx.x & 63;
     const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const bool active = j < nt;
@@ -261,11 +265,14 @@ __global__ __launch_bounds__(256) void adj_bm_p1_regular_kernel(const float* __r
         float gxv[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
         float gnx[3] = {0.f, 0.f, 0.f}, erow = 0.f;
         cf Gs = {0.f, 0.f};
-#pragma unroll
+        // one row point at a time: unrolled the three take 300 registers
+#pragma unroll 1
         for (int a = 0; a < Q; ++a) {
             const float xa0 = rr[3 * a], xa1 = rr[3 * a + 1], xa2 = rr[3 * a + 2];
             const float ua = rr[3 * Q + a];
-            const float p1 = TriRule<Q>::x1[a], p2 = TriRule<Q>::x2[a], p0 = 1.f - p1 - p2;
+            const float p1 = a == 0 ? TriRule<Q>::x1[0] : (a == 1 ? TriRule<Q>::x1[1] : TriRule<Q>::x1[2]);
+            const float p2 = a == 0 ? TriRule<Q>::x2[0] : (a == 1 ? TriRule<Q>::x2[1] : TriRule<Q>::x2[2]);
+            const float p0 = 1.f - p1 - p2;
             // l(x_a) = sum conj(lambda_c) phi_c(x_a)
             const cf la = on ? cf{p0 * l3[0].x + p1 * l3[1].x + p2 * l3[2].x,
                                   -(p0 * l3[0].y + p1 * l3[1].y + p2 * l3[2].y)}
@@ -315,33 +322,47 @@ __global__ __launch_bounds__(256) void adj_bm_p1_regular_kernel(const float* __r
             colcurl[c].i += t.i;
             RC[c] = cmul(Gs, CF[c]);
         }
+        // the row triangle's sums over this wavefront's columns: vertex
+        // gradients 9, n_x gradient 3, curl sums 3 complex, e
+        const float red[18] = {gxv[0][0], gxv[0][1], gxv[0][2], gxv[1][0], gxv[1][1], gxv[1][2],
+                               gxv[2][0], gxv[2][1], gxv[2][2], gnx[0],    gnx[1],    gnx[2],
+                               RC[0].r,   RC[0].i,   RC[1].r,   RC[1].i,   RC[2].r,   RC[2].i};
+        const int grp = lane >> 4, o4 = (grp & 1) * 2 + (grp >> 1);  // 16-lane row -> value 0, 2, 1, 3
+        float* dst = rowsum[threadIdx.x >> 6][i - i_begin];
+#pragma unroll
+        for (int c = 0; c < 18; c += 6) {
+            float p, q;
+            wave_sum_six(red + c, p, q);
+            if ((lane & 15) == 0) {
+                dst[c + o4] = p;
+                if (!(grp & 1)) dst[c + 4 + (grp >> 1)] = q;
+            }
+        }
+        const float er = wsum(erow);
+        if (lane == 0) dst[18] = er;
+    }
+    __syncthreads();
+    if (i_begin + (int)threadIdx.x < i_end) {
+        const int64_t i = i_begin + threadIdx.x;
+        const int4 ti = tris[i];
         float red[19];
+#pragma unroll
+        for (int e = 0; e < 19; ++e)
+            red[e] = (float)(((double)rowsum[0][threadIdx.x][e] + rowsum[1][threadIdx.x][e]) +
+                             ((double)rowsum[2][threadIdx.x][e] + rowsum[3][threadIdx.x][e]));
+        const float* g = geo + i * 16;
+        float gv[3][3];
 #pragma unroll
         for (int a = 0; a < 3; ++a)
 #pragma unroll
-            for (int c = 0; c < 3; ++c) red[3 * a + c] = wsum(gxv[a][c]);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            red[9 + c] = wsum(gnx[c]);
-            red[12 + 2 * c] = wsum(RC[c].r);
-            red[13 + 2 * c] = wsum(RC[c].i);
-        }
-        red[18] = wsum(erow);
-        if (lane == 0) {
-            const float* g = geo + i * 16;
-            float gv[3][3];
-#pragma unroll
-            for (int a = 0; a < 3; ++a)
-#pragma unroll
-                for (int c = 0; c < 3; ++c) gv[a][c] = red[3 * a + c];
-            const cf s3[3] = {cconj(l3[0]), cconj(l3[1]), cconj(l3[2])};
-            const cf V3[3] = {{red[12], red[13]}, {red[14], red[15]}, {red[16], red[17]}};
-            float gcu[3][3];
-            curl_grads(s3, V3, invk, gcu);
-            const float gnv[3] = {red[9], red[10], red[11]};
-            triangle_chain(g, gnv, red[18] / g[12], gcu, gv);
-            add_vertex_grads(gvert, ti, gv);
-        }
+            for (int c = 0; c < 3; ++c) gv[a][c] = red[3 * a + c];
+        const cf s3[3] = {cconj(lam[ti.x]), cconj(lam[ti.y]), cconj(lam[ti.z])};
+        const cf V3[3] = {{red[12], red[13]}, {red[14], red[15]}, {red[16], red[17]}};
+        float gcu[3][3];
+        curl_grads(s3, V3, invk, gcu);
+        const float gnv[3] = {red[9], red[10], red[11]};
+        triangle_chain(g, gnv, red[18] / g[12], gcu, gv);
+        add_vertex_grads(gvert, ti, gv);
     }
     if (active) {
         float gv[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};

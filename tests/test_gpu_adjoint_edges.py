@@ -1,7 +1,8 @@
 """The DP0 adjoint kernels where their row tiles (32 triangles) and pair groups
 (16 pairs a workgroup) are only partly filled: vertex gradients of 20, 77 and 80
 triangles along random directions against central differences of the FP64 oracle
-pipeline, at the bound of the same comparison on larger meshes (2e-3)."""
+pipeline, at the bound of the same comparison on larger meshes (2e-3); the same
+for the P1 Burton-Miller gradient (row tiles of 32 triangles)."""
 import numpy as np
 import pytest
 import torch
@@ -9,6 +10,7 @@ import torch
 import fp64_grad
 from neuralat_amd import mesh
 from test_gpu_grad import _dev, _loss_gpu, _setup
+from test_gpu_grad_bm import _fp64_ops, _gpu_geometry, _loss64
 
 pytestmark = pytest.mark.gpu
 
@@ -32,4 +34,25 @@ def test_vertex_gradient(level, drop):
         d /= np.linalg.norm(d)
         fd.append((fp64_grad.loss(v64 + h * d, t, k0, src, pts) - fp64_grad.loss(v64 - h * d, t, k0, src, pts)) / (2 * h))
         ad.append(np.sum(gv * d))
+    assert np.linalg.norm(np.array(ad) - fd) < 2e-3 * np.linalg.norm(fd)
+
+
+@pytest.mark.parametrize("level", [0, 1])
+def test_p1_vertex_gradient(level):
+    k = 7.0
+    v, t = mesh.icosphere(level, 0.1)
+    v = mesh.sh_perturb(v, 4, 0.05, seed=6).astype(np.float32)
+    _, dn = mesh.sources_field(np.array([[0.01, -0.005, 0.002]]), None, k)
+    psi = mesh.project_p1(v, t, lambda x, n: dn(x, n))
+    pts = mesh.random_exterior_points(24, 0.2, 0.5, seed=2)
+    print("P1 adjoint edges", len(t), flush=True)
+    gv, _ = _gpu_geometry(v, t, k, psi, pts)
+    v64, h = v.astype(np.float64), 1e-6
+    rng = np.random.default_rng(11)
+    ad, fd = [], []
+    for _ in range(6):
+        d = rng.standard_normal(v.shape)
+        lp, lm = (_loss64(_fp64_ops(v64 + s * h * d, t, k, pts), psi) for s in (1, -1))
+        fd.append((lp - lm) / (2 * h))
+        ad.append(float(np.sum(gv * d)))
     assert np.linalg.norm(np.array(ad) - fd) < 2e-3 * np.linalg.norm(fd)
