@@ -204,6 +204,9 @@ __global__ __launch_bounds__(256, 3) void adj_regular_kernel(const float* __rest
         const float ai = on ? -(li.x * psj.y - li.y * psj.x) : 0.f;
         const float br = on ? (li.x * phj.x + li.y * phj.y) : 0.f;
         const float bi = on ? (li.x * phj.y - li.y * phj.x) : 0.f;
+        // without the clamp a triangle meets its own points at r = 0, where the
+        // zero coefficients would multiply infinities: off-pair lanes move off it
+        const float away = CLAMP || on ? 0.f : 1.f;
         const float* rr = rec + i * S;
         float red[10] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         float pv_r = 0.f, pv_i = 0.f;
@@ -216,7 +219,7 @@ __global__ __launch_bounds__(256, 3) void adj_regular_kernel(const float* __rest
 #pragma unroll
             for (int b = 0; b < Q; ++b) {
                 const float dx = py[3 * b] - xa0, dy = py[3 * b + 1] - xa1, dz = py[3 * b + 2] - xa2;
-                float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                float r2 = fmaf(dx, dx, fmaf(dy, dy, CLAMP ? dz * dz : fmaf(dz, dz, away)));
                 const bool clamped = CLAMP && r2 < kEps2;
                 if (CLAMP) r2 = fmaxf(r2, kEps2);
                 const float rinv = __builtin_amdgcn_rsqf(r2);
