@@ -1779,11 +1779,12 @@ __global__ __launch_bounds__(256) void cbie_pairs_kernel(const CbiePairItem it)
     cbie_pair<NL, CLAMP>(it, (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6));
 }
 // every item of a batch (full rules): wavefront w takes the pair w - pair0 of
-// the item with the largest pair0 <= w
+// the item with the largest pair0 <= w; w counts from wave0, the launch's first
 template <bool CLAMP>
-__global__ __launch_bounds__(256) void batch_cbie_pairs_kernel(const CbiePairItem* __restrict__ items, int nitems)
+__global__ __launch_bounds__(256) void batch_cbie_pairs_kernel(const CbiePairItem* __restrict__ items, int nitems,
+                                                               int64_t wave0)
 {
-    const int64_t w = uniform_i64((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6));
+    const int64_t w = uniform_i64(wave0 + (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6));
     int lo = 0, hi = nitems - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
@@ -2284,15 +2285,17 @@ CbiePairItem cbie_pair_item(const MeshDev& m, float k, const float2* psi, float2
 }
 
 // the neighbour pairs and the row reduction of every item (full rules), one
-// launch each: items in table order, nwaves = the sum of their pair counts,
-// ntmax the largest item
+// launch each up to the grid's limits (2^32 work-items a dimension: half of it
+// a pair launch, 2^25 pairs): items in table order, nwaves = the sum of their
+// pair counts, ntmax the largest item
+constexpr int64_t kPairLaunchWaves = (int64_t)1 << 25;
 hipError_t launch_batch_cbie_finish(const CbiePairItem* items, int nitems, int64_t nwaves, int64_t ntmax, int clamp,
                                     hipStream_t s)
 {
-    const unsigned g = (unsigned)((nwaves + 3) / 4);
-    if (nwaves > 0) {
-        if (clamp) hipLaunchKernelGGL(batch_cbie_pairs_kernel<true>, dim3(g), dim3(256), 0, s, items, nitems);
-        else hipLaunchKernelGGL(batch_cbie_pairs_kernel<false>, dim3(g), dim3(256), 0, s, items, nitems);
+    for (int64_t w0 = 0; w0 < nwaves; w0 += kPairLaunchWaves) {
+        const unsigned g = (unsigned)((std::min(kPairLaunchWaves, nwaves - w0) + 3) / 4);
+        if (clamp) hipLaunchKernelGGL(batch_cbie_pairs_kernel<true>, dim3(g), dim3(256), 0, s, items, nitems, w0);
+        else hipLaunchKernelGGL(batch_cbie_pairs_kernel<false>, dim3(g), dim3(256), 0, s, items, nitems, w0);
     }
     for (int q0 = 0; q0 < nitems; q0 += 65535) {  // grid y limit
         const int cq = nitems - q0 < 65535 ? nitems - q0 : 65535;

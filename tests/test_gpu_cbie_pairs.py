@@ -79,3 +79,26 @@ def test_batch_of_uneven_items(row_tile):
     outs = batch_cbie(handles, ks, [torch.tensor(p, device=_dev()) for p in psis], row_tile=row_tile)
     for (v, t), k, p, (lhs, rhs) in zip(meshes, ks, psis, outs):
         _check(v, t, k, True, p, lhs.cpu().numpy(), rhs.cpu().numpy(), "full")
+
+
+def test_batch_past_the_grid_limit():
+    """A batch of more neighbour pairs than one launch can take at a wavefront
+    each (2^26 pairs are 2^32 work-items): 65 items of a 1024-triangle fan, whose
+    triangles are all neighbours.  Items at both ends of the split equal the
+    same item alone, bit for bit."""
+    from neuralat_amd.bem.batch import Mesh, allocate_systems, batch_cbie
+
+    d, items = 1024, 65
+    a = 2 * np.pi * np.arange(d) / d
+    v = np.concatenate([[[0, 0, 0.05]], np.stack([0.1 * np.cos(a), 0.1 * np.sin(a), 0 * a], 1)]).astype(np.float32)
+    t = np.stack([0 * np.arange(d), 1 + np.arange(d), 1 + (np.arange(d) + 1) % d], 1).astype(np.int32)
+    m = Mesh(torch.tensor(v, device=_dev()), torch.tensor(t, device=_dev()))
+    assert m.n_neighbor_pairs * items > 2 ** 26
+    ks = [2.0 + 0.25 * q for q in range(items)]
+    psis = [torch.tensor(_psi(d, q), device=_dev()) for q in range(items)]
+    outs = [(lhs.fill_(float("nan")), rhs.fill_(float("nan"))) for lhs, rhs in allocate_systems([m] * items, _dev())]
+    print("cbie batch past the grid limit", m.n_neighbor_pairs * items, flush=True)
+    batch_cbie([m] * items, ks, psis, outs=outs, row_tile=64)
+    for q in (0, 31, 32, 63, 64):
+        (lhs, rhs), = batch_cbie([m], [ks[q]], [psis[q]], row_tile=64)
+        assert torch.equal(lhs, outs[q][0]) and torch.equal(rhs, outs[q][1]), q
