@@ -20,7 +20,13 @@ namespace bem {
 
 namespace {
 size_t al(size_t b) { return (b + 255) / 256 * 256; }
-constexpr int kFirstWindow = 3, kMaxWindow = 8;  // steps per read of the convergence flags
+// Steps per read of the convergence flags: the first step of a cycle alone
+// (a cycle of one step would pay for products it does not need: with a first
+// read after three, 16 FP32 right-hand sides that converge in one step took 2155
+// us at 16384 unknowns, now 1357), then up to kMaxWindow; beyond kWindowMaxN
+// unknowns, where a product costs several reads, every step.
+constexpr int kMaxWindow = 8;
+constexpr int64_t kWindowMaxN = 12288;
 }  // namespace
 
 hipError_t MultiOp::apply(const float2* X, int64_t ldx, int ns, float2* Y, int64_t ldy, float2 alpha, float2 beta,
@@ -175,7 +181,7 @@ hipError_t gmres_multi(const MultiOp& op, int64_t n, int ns, const float2* B, in
         // 20 us, a step costs 50 us and more.  The systems' own step counts
         // stop at convergence, so steps past it change nothing; the window is
         // the number of steps the slowest system needs at the decay seen so far.
-        int checked = 0, window = prec ? 1 : kFirstWindow, steps = 0;
+        int checked = 0, window = 1, steps = 0;
         for (int q = 0; q < ns; ++q) before[q] = std::sqrt(hr[q]);
         for (int j = 0; j < m && its + steps < maxiter; ++j) {
             const float2* Vj = V + (int64_t)j * ns * ldn;
@@ -224,7 +230,7 @@ hipError_t gmres_multi(const MultiOp& op, int64_t n, int ns, const float2* B, in
                 before[q] = hres[q];
             }
             checked = steps;
-            if (!prec) window = (int)std::min<double>(kMaxWindow, std::ceil(left));
+            if (!prec && n <= kWindowMaxN) window = (int)std::min<double>(kMaxWindow, std::ceil(left));
             if (all) {
                 steps = 0;  // the steps the slowest system took
                 for (int q = 0; q < ns; ++q) steps = std::max(steps, hk[q]);

@@ -3,6 +3,8 @@ separate kernels beyond both) at the edges of its forms: 64-lane, 512-element
 chunk and LDS limits, step counts that cross from one form to the next, and
 systems of unequal length in lockstep.  Solutions against FP64 residuals and
 direct solves at the bars the solver tests use (1e-5)."""
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -87,3 +89,33 @@ def test_uneven_lockstep(use_graph):
                                   max_outer_cycles=6, use_graph=use_graph)
     for n, A, b, x, i in zip(sizes, As, bs, xs, infos):
         assert i["converged"] and _err(A, x, b) < 2e-6, (n, i)
+
+
+def _best(f, n=9):
+    f()
+    torch.cuda.synchronize()
+    out = []
+    for _ in range(n):
+        a = time.perf_counter()
+        f()
+        torch.cuda.synchronize()
+        out.append(time.perf_counter() - a)
+    return min(out)
+
+
+@pytest.mark.parametrize("n", [6000, 12000, 13000])
+def test_one_step_takes_one_product(n):
+    """A solve that converges in its first step takes no products past it: as
+    long as with maxiter=1, whose residual is read after that step whatever the
+    read window (two more steps would make five products of three)."""
+    from neuralat_amd.bem.precision import gmres_multi
+    from neuralat_amd.bem.solver import gmres
+
+    A, B = _system(n, 1e-8, n, 16)
+    print("arnoldi one step", n, flush=True)
+    for solve in (lambda **kw: gmres(A, B[0], tol=1e-5, restart=50, **kw)[1],
+                  lambda **kw: gmres_multi(A, B, tol=1e-5, restart=50, **kw)[1][0]):
+        info = solve()
+        assert info["converged"] and info["iterations"] == 1, info
+        free, held = _best(solve), _best(lambda: solve(maxiter=1))
+        assert free < 1.25 * held, (n, free, held)
