@@ -565,11 +565,13 @@ __global__ __launch_bounds__(256) void xto_fp8_kernel(const BSys* __restrict__ s
 }
 
 // amax_bits[s] = bits of max |Re|, |Im| over A_s (non-negative floats order as
-// their bit patterns); amax_bits zeroed beforehand; grid (at most
-// kAmaxBlocks row blocks, items): one atomic per workgroup, few workgroups (an
-// atomic per wavefront of 2048 workgroups per item serialised on the items'
-// words: 1770 us for 24 items of 320 to 3380 unknowns, 680 MB)
-constexpr int64_t kAmaxBlocks = 128;
+// their bit patterns); amax_bits zeroed beforehand; grid (row blocks, items):
+// one atomic per workgroup and few workgroups (an atomic per wavefront of 2048
+// workgroups per item serialised on the items' words: 1770 us for 24 items of
+// 320 to 3380 unknowns, 680 MB).  kAmaxBlocks an item, more where few items would
+// leave the chip idle: kAmaxFill in all (one item of 20480 unknowns, 3.4 GB, on
+// 128 workgroups: a whole solve of 5402 us, now 4261)
+constexpr int64_t kAmaxBlocks = 128, kAmaxFill = 2048;
 __global__ __launch_bounds__(256) void xamax_kernel(const BSys* __restrict__ sys, unsigned int* __restrict__ amax_bits)
 {
     const int s = blockIdx.y;
@@ -1317,8 +1319,10 @@ int bem_batch_fgmres(const bem_batch_system* sys, int ns, int dtype, float tol, 
     XTRY(hipMemcpyAsync(dlow, hl.data(), sizeof(BLow) * ns, hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(xfill_kernel, dim3((ns + 255) / 256), dim3(256), 0, s, amax, (int64_t)ns, 0u);
     const dim3 grow((unsigned)std::min<int64_t>(nmax, 2048), (unsigned)ns);
-    if (dtype == kDtFP16)
-        hipLaunchKernelGGL(xamax_kernel, dim3((unsigned)std::min(nmax, kAmaxBlocks), (unsigned)ns), dim3(256), 0, s, dsys, amax);
+    if (dtype == kDtFP16) {
+        const int64_t blocks = std::min(nmax, std::max(kAmaxBlocks, kAmaxFill / ns));
+        hipLaunchKernelGGL(xamax_kernel, dim3((unsigned)blocks, (unsigned)ns), dim3(256), 0, s, dsys, amax);
+    }
     hipLaunchKernelGGL(xscale_kernel, dim3((ns + 63) / 64), dim3(64), 0, s, amax, dtype, scale, inv, ns);
     if (dtype == kDtFP8)
         hipLaunchKernelGGL(xto_fp8_kernel, grow, dim3(256), 0, s, dsys, dlow);

@@ -119,3 +119,28 @@ def test_one_step_takes_one_product(n):
         assert info["converged"] and info["iterations"] == 1, info
         free, held = _best(solve), _best(lambda: solve(maxiter=1))
         assert free < 1.25 * held, (n, free, held)
+
+
+def test_fp16_scale_of_one_large_system():
+    """The scale of one large system's 16-bit copy reads its matrix at the
+    chip's rate: the fp16 solve takes one more read of 3.4 GB than the bf16 one
+    (0.7 ms of 3.8 at 5 TB/s; 1.7 ms on half the CUs)."""
+    from neuralat_amd.bem.batch import batch_solve_mixed
+
+    A, b = _system(20480, 1e-8, 1)
+    A[20479, 7] = 300.0  # the largest entry, in the last row: the scale must see it
+    print("fp16 scale", flush=True)
+    t = {}
+    for dtype in ("bf16", "fp16"):
+        solve = lambda: batch_solve_mixed([A], [b[0]], dtype=dtype, tol=1e-5, inner_tol=1e-2, inner_restart=10)  # noqa: E731
+        x, infos = solve()
+        assert infos[0]["converged"] and _err_rows(A, x[0], b[0]) < 2e-5, infos
+        t[dtype] = _best(solve)
+    assert t["fp16"] < 1.3 * t["bf16"], t
+
+
+def _err_rows(A, x, b):
+    """Relative residual, the product in FP64 row blocks."""
+    r = torch.cat([b[q:q + 2048].to(torch.complex128) - A[q:q + 2048].to(torch.complex128) @ x.to(torch.complex128)
+                   for q in range(0, len(b), 2048)])
+    return float(torch.linalg.vector_norm(r) / torch.linalg.vector_norm(b.to(torch.complex128)))
