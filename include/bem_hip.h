@@ -77,9 +77,11 @@ int bem_mesh_create(const float* verts, int64_t nv, const int32_t* tris, int64_t
 int bem_mesh_destroy(bem_mesh* mesh);
 /* New vertex positions [nv,3] for a mesh handle with the same triangles
  * (rigid or deformed objects in data generation: scene.py:218-291 builds a
- * new BEM_Solver per sample): the quadrature records, normals, curls and
- * geometry are recomputed and uploaded in one copy on `stream`, which is
- * waited for; neighbour pairs, vertex lists and the P1 tiling are kept.
+ * new BEM_Solver per sample): the positions are checked and the quadrature
+ * records, normals, curls and geometry recomputed by kernels on `stream` (of
+ * the mesh's device), which is waited for; neighbour pairs, vertex lists and
+ * the P1 tiling are kept.  on_device: 0 = host memory, else device memory,
+ * the mesh's own GPU's (read in place) or another's (copied first).
  * Kernels still reading the old positions on other streams must be done
  * first.  Results equal those of a new handle built from the positions (P1
  * sums in another order: the tiling is the first positions'). */

@@ -67,12 +67,15 @@ class Mesh:
         return self._h
 
     def set_vertices(self, vertices: torch.Tensor):
-        """New positions [V,3] for the same triangles (bem_mesh_set_vertices)."""
+        """New positions [V,3] for the same triangles (bem_mesh_set_vertices),
+        from any GPU."""
         check_tensor(vertices, torch.float32)
         if tuple(vertices.shape) != (self.nv, 3):
             raise ValueError(f"vertices must be [{self.nv},3]")
-        vertices = vertices.contiguous()
-        _lib.check(self._lib.bem_mesh_set_vertices(self._h, _ptr(vertices), 1, _stream()), "bem_mesh_set_vertices")
+        vertices = vertices.contiguous().to(self.device)
+        with torch.cuda.device(self.device):
+            rc = self._lib.bem_mesh_set_vertices(self._h, _ptr(vertices), 1, _stream())
+        _lib.check(rc, "bem_mesh_set_vertices")
 
     def normals_curls(self):
         n = torch.empty((self.nt, 3), dtype=torch.float32, device=self.device)

@@ -227,7 +227,7 @@ hipError_t launch_field(const MeshDev& mg, int64_t gstride, const float* pts, in
 // in `err`.
 int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t nt, hipStream_t stream, MeshDev& m,
                std::string& err);
-// New vertex positions (host or device) for a built mesh (same triangles):
+// New vertex positions (host, or device: any GPU's) for a built mesh (same triangles):
 // checked, then the position-dependent arrays recomputed by a kernel on s, which
 // is waited for.  Connectivity data and the tiling are kept; after a fault so
 // are the old positions.

@@ -666,6 +666,18 @@ int geomset_build(const MeshDev& m, const float* h_verts, int ns, hipStream_t s,
     return rc;
 }
 
+// memory the kernels of this device may read: its own allocation (another GPU's
+// need not be mapped here)
+static bool owned_by(const void* p, int device)
+{
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice && a.device == device;
+}
+
 int mesh_set_vertices(MeshDev& m, const float* verts, bool on_device, hipStream_t s, std::string& err)
 {
     if (!m.block) {
@@ -677,12 +689,12 @@ int mesh_set_vertices(MeshDev& m, const float* verts, bool on_device, hipStream_
     void* tmp = nullptr;
     const float* src = verts;
     hipError_t e = hipSuccess;
-    if (!on_device) {  // checked on the device as well: through a temporary
+    if (!on_device || !owned_by(verts, m.device)) {  // checked on this device as well: through a temporary
         e = hipMallocAsync(&tmp, vb, s);
         if (e == hipSuccess) {
-            char* host = st.get(vb);
-            std::memcpy(host, verts, vb);
-            e = hipMemcpyAsync(tmp, host, vb, hipMemcpyHostToDevice, s);
+            const void* from = verts;
+            if (!on_device) from = std::memcpy(st.get(vb), verts, vb);
+            e = hipMemcpyAsync(tmp, from, vb, on_device ? hipMemcpyDefault : hipMemcpyHostToDevice, s);
             src = (const float*)tmp;
         }
     }

@@ -100,3 +100,52 @@ def test_fem_rejects_bad_meshes():
         rc = lib.bem_fem_create(v.ctypes.data, len(v), t.ctypes.data, len(t), ctypes.byref(h))
         assert rc == _lib.BEM_ERR_BAD_MESH, tets
         assert lib.bem_fem_last_error()
+
+
+def test_set_vertices_brings_positions_to_the_mesh_device(monkeypatch):
+    """Positions on another GPU are moved to the mesh's device, and its stream is
+    the one passed, whatever device is current (stand-ins: no GPU here)."""
+    import contextlib
+
+    import torch
+
+    from neuralat_amd.bem import solver
+
+    class Positions:
+        dtype, is_cuda, shape = torch.float32, True, (3, 3)
+
+        def __init__(self, device):
+            self.device = torch.device(device)
+
+        def is_contiguous(self):
+            return True
+
+        def contiguous(self):
+            return self
+
+        def to(self, device):
+            return self if self.device == torch.device(device) else Positions(device)
+
+        def data_ptr(self):
+            return 1000 + self.device.index
+
+    class Lib:
+        def bem_mesh_set_vertices(self, handle, ptr, on_device, stream):
+            calls.append((ptr.value, on_device, stream))
+            return 0
+
+    calls, current = [], [1]
+
+    @contextlib.contextmanager
+    def device(d):
+        before, current[0] = current[0], torch.device(d).index
+        yield
+        current[0] = before
+
+    monkeypatch.setattr(torch.cuda, "device", device)
+    monkeypatch.setattr(solver, "_stream", lambda: f"stream of {current[0]}")
+    m = solver.Mesh.__new__(solver.Mesh)
+    m.nv, m.device, m._lib, m._h = 3, torch.device("cuda:0"), Lib(), None
+    for source in ("cuda:0", "cuda:1"):
+        m.set_vertices(Positions(source))
+    assert calls == [(1000, 1, "stream of 0")] * 2

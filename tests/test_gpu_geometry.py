@@ -66,3 +66,19 @@ def test_faults_are_reported_and_change_nothing():
         with pytest.raises(ValueError, match=f"sample 2: .*{what}"):
             GeometrySet(m, np.stack([v, v, bad, v]))
     assert torch.equal(before, m.normals_curls()[0])
+
+
+def test_positions_outside_the_device_are_copied():
+    """Positions that are not an allocation of the mesh's own GPU (here pinned host
+    memory passed as device memory) are copied, not read in place."""
+    from neuralat_amd.bem import Mesh
+
+    v, t = mesh.icosphere(1, 0.1)
+    v = v.astype(np.float32)
+    m = Mesh(torch.tensor(v, device=_dev()), torch.tensor(t, device=_dev()))
+    moved = torch.tensor(v * np.float32(1.3) + np.float32(0.1)).pin_memory()
+    print("positions in pinned memory", flush=True)
+    _lib.check(_lib.load().bem_mesh_set_vertices(m.handle, moved.data_ptr(), 1, ctypes.c_void_p(0)))
+    n, c = (a.cpu().numpy() for a in m.normals_curls())
+    rn, rc = _normals_curls(moved.numpy(), t)
+    assert np.abs(n - rn).max() < 1.2e-7 and np.abs(c - rc).max() < 1.2e-7 * np.abs(rc).max()
