@@ -1511,7 +1511,9 @@ __global__ __launch_bounds__(256) void singular_kernel(const float* __restrict__
 // lhs_mass: times the mass matrix added (with the coincident pairs).
 // RG (Burton-Miller LHS): the right-hand side operator's entries at the same
 // points, contracted with g, and -(i/2k) M g: three row sums per pair at
-// rg + (z npairs + p) 3.
+// rg + (z npairs + p) 3.  The products with g are FP64, per point (an FP32
+// product of the interpolated g took as long: 1058 us and 1060 for the system
+// of 3612 vertices).
 template <int OP, int NL, bool CLAMP, int LPP, bool RG>
 __global__ __launch_bounds__(256) void p1_pairs_kernel(const float* __restrict__ geo, const int4* __restrict__ tris,
                                                        const float* __restrict__ curls,
@@ -1562,11 +1564,11 @@ __global__ __launch_bounds__(256) void p1_pairs_kernel(const float* __restrict__
             float reg[NR][7];
             const float jac = ss_regions<S>(LineRule01<NL>::t[q0], LineRule01<NL>::t[q1], LineRule01<NL>::t[q2],
                                             LineRule01<NL>::t[q3], reg);
-            float br[NE], bi[NE], cr[RG ? 3 : 1], ci[RG ? 3 : 1];
+            float br[NE], bi[NE], cr[RG ? 9 : 1], ci[RG ? 9 : 1];  // cr, ci: the right-hand side operator's entries
 #pragma unroll
             for (int e = 0; e < NE; ++e) br[e] = bi[e] = 0.f;
 #pragma unroll
-            for (int a = 0; a < (RG ? 3 : 1); ++a) cr[a] = ci[a] = 0.f;
+            for (int e = 0; e < (RG ? 9 : 1); ++e) cr[e] = ci[e] = 0.f;
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
                 const float x1 = reg[r][0], x2 = reg[r][1], y1 = reg[r][2], y2 = reg[r][3], ww = reg[r][4];
@@ -1576,6 +1578,12 @@ __global__ __launch_bounds__(256) void p1_pairs_kernel(const float* __restrict__
                 kernel4pi<OP, CLAMP>(dx, dy, dz, nx0, nx1, nx2, ny0, ny1, ny2, k, krev, vr, vi, gr, gi);
                 vr *= ww;
                 vi *= ww;
+                float v2r = 0.f, v2i = 0.f, u0 = 0.f, u1 = 0.f;
+                if constexpr (RG) {
+                    kernel4pi<BM_RHS, CLAMP>(dx, dy, dz, nx0, nx1, nx2, ny0, ny1, ny2, k, krev, v2r, v2i, u0, u1);
+                    v2r *= ww;
+                    v2i *= ww;
+                }
                 const float px[3] = {1.f - x1, x1 - x2, x2};
                 const float py[3] = {1.f - y1, y1 - y2, y2};
 #pragma unroll
@@ -1585,6 +1593,10 @@ __global__ __launch_bounds__(256) void p1_pairs_kernel(const float* __restrict__
                         const float pp = px[a] * py[b];
                         br[3 * a + b] = fmaf(vr, pp, br[3 * a + b]);
                         bi[3 * a + b] = fmaf(vi, pp, bi[3 * a + b]);
+                        if constexpr (RG) {
+                            cr[3 * a + b] = fmaf(v2r, pp, cr[3 * a + b]);
+                            ci[3 * a + b] = fmaf(v2i, pp, ci[3 * a + b]);
+                        }
                     }
                 if constexpr (OP == HYP) {  // plain G
                     br[9] += vr;
@@ -1593,18 +1605,6 @@ __global__ __launch_bounds__(256) void p1_pairs_kernel(const float* __restrict__
                     br[9] = fmaf(gr, ww, br[9]);
                     bi[9] = fmaf(gi, ww, bi[9]);
                 }
-                if constexpr (RG) {
-                    float v2r, v2i, u0 = 0.f, u1 = 0.f;
-                    kernel4pi<BM_RHS, CLAMP>(dx, dy, dz, nx0, nx1, nx2, ny0, ny1, ny2, k, krev, v2r, v2i, u0, u1);
-                    const float hr = ww * (py[0] * gv[0].x + py[1] * gv[1].x + py[2] * gv[2].x);
-                    const float hi = ww * (py[0] * gv[0].y + py[1] * gv[1].y + py[2] * gv[2].y);
-                    const float tr = v2r * hr - v2i * hi, ti = v2r * hi + v2i * hr;
-#pragma unroll
-                    for (int a = 0; a < 3; ++a) {
-                        cr[a] = fmaf(px[a], tr, cr[a]);
-                        ci[a] = fmaf(px[a], ti, ci[a]);
-                    }
-                }
             }
             const double sc = (double)(jac * wq) * (double)g.jij;
 #pragma unroll
@@ -1612,11 +1612,18 @@ __global__ __launch_bounds__(256) void p1_pairs_kernel(const float* __restrict__
                 ar[e] += sc * (double)br[e];
                 ai[e] += sc * (double)bi[e];
             }
-            if constexpr (RG) {
+            if constexpr (RG) {  // times g in FP64, as the sums are
 #pragma unroll
                 for (int a = 0; a < 3; ++a) {
-                    rr[a] += sc * (double)cr[a];
-                    ri[a] += sc * (double)ci[a];
+                    double tr = 0.0, ti = 0.0;
+#pragma unroll
+                    for (int b = 0; b < 3; ++b) {
+                        const double er = cr[3 * a + b], ei = ci[3 * a + b], gr = gv[b].x, gi = gv[b].y;
+                        tr = fma(er, gr, fma(-ei, gi, tr));
+                        ti = fma(er, gi, fma(ei, gr, ti));
+                    }
+                    rr[a] = fma(sc, tr, rr[a]);
+                    ri[a] = fma(sc, ti, ri[a]);
                 }
             }
         }
