@@ -1517,8 +1517,9 @@ __global__ __launch_bounds__(256) void singular_kernel(const float* __restrict__
 template <int OP, int NL, bool CLAMP, int LPP, bool RG>
 __global__ __launch_bounds__(256) void p1_pairs_kernel(const float* __restrict__ geo, const int4* __restrict__ tris,
                                                        const float* __restrict__ curls,
-                                                       const int4* __restrict__ pairs, int64_t npairs, const KBatch kb,
-                                                       float lhs_mass, float2* __restrict__ blk,
+                                                       const int4* __restrict__ pairs,
+                                                       const int64_t* __restrict__ pair_ptr, int64_t npairs,
+                                                       const KBatch kb, float lhs_mass, float2* __restrict__ blk,
                                                        const float2* __restrict__ g_vec, float2* __restrict__ rg)
 {
     static_assert(!RG || OP == BM_LHS, "the right-hand side rides on the Burton-Miller LHS");
@@ -1536,7 +1537,7 @@ __global__ __launch_bounds__(256) void p1_pairs_kernel(const float* __restrict__
     const int i = PPW == 1 ? __builtin_amdgcn_readfirstlane(pr.x) : pr.x;
     const int j = PPW == 1 ? __builtin_amdgcn_readfirstlane(pr.y) : pr.y;
     const int shared = PPW == 1 ? __builtin_amdgcn_readfirstlane(pr.z) : pr.z;
-    const int64_t out = (int64_t)blockIdx.z * npairs + pr.w;  // the pair's place in the (i, j) order
+    const int64_t out = (int64_t)blockIdx.z * npairs + pair_ptr[i] + pr.w;  // the pair's place in the (i, j) order
     SSPair g;
     ss_pair_setup(geo, tris, i, j, shared, g);
     const float nx0 = g.nx[0], nx1 = g.nx[1], nx2 = g.nx[2], ny0 = g.ny[0], ny1 = g.ny[1], ny2 = g.ny[2];
@@ -2229,7 +2230,7 @@ static hipError_t launch_p1_pairs(const MeshDev& m, int quad, const KBatch& kb, 
         const int64_t per = 4 * (64 / LPP);
         hipLaunchKernelGGL((p1_pairs_kernel<OP, NL, CLAMP, LPP, RG>),
                            dim3((unsigned)((m.npairs + per - 1) / per), 1, (unsigned)nz), dim3(256), 0, s, m.geo, m.tris,
-                           m.curls, m.pairs_by_kind, m.npairs, kb, lhs_mass, blk, g, rg);
+                           m.curls, m.pairs_by_kind, m.pair_ptr, m.npairs, kb, lhs_mass, blk, g, rg);
     };
     if (quad == 0) {
         if (total >= kPairsFill4) run(std::integral_constant<int, 4>{}, std::integral_constant<int, 16>{});

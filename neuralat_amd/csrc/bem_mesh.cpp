@@ -390,20 +390,17 @@ int mesh_build(const float* h_verts, int64_t nv, const int32_t* h_tris, int64_t 
         }
     }
     m.npairs = (int64_t)pairs.size();
-    if (m.npairs > INT32_MAX) {
-        err = "mesh has more than 2^31 neighbour pairs";
-        return 1;
-    }
     // the P1 neighbour-pair launches take every pair in any order: grouped by
     // kind, the pairs that share a wavefront take the same quadrature branch
-    // (the last entry: the pair's place in the (i, j) order)
+    // (the last entry: the pair's place in its row of the (i, j) order, which
+    // fits 32 bits however many pairs there are)
     std::vector<Pair> pairs_kind(pairs.size());
     {
         int64_t next[4] = {0, kinds[3] + kinds[2], kinds[3], 0};
         for (size_t q = 0; q < pairs.size(); ++q) {
             Pair& p = pairs_kind[(size_t)next[pairs[q].shared]++];
             p = pairs[q];
-            p.pad = (int32_t)q;
+            p.pad = (int32_t)((int64_t)q - m.h_pair_ptr[p.i]);
         }
     }
     m.max_neighbors = maxnb;
