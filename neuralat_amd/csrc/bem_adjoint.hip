@@ -154,8 +154,13 @@ __device__ __forceinline__ void column_chain(const float* geo_j, const float (*g
 // A row triangle's ten sums over a wavefront go to LDS; the tile's row triangles
 // are chained to their vertices at its end, a lane each (one lane a row and
 // wavefront before, with nine single-lane FP64 atomics).  32 rows a tile: at
-// 5120 triangles 64 left 1.5 rounds of workgroups.
-constexpr int kAdjRowTile = 32;
+// 5120 triangles 64 left 1.5 rounds of workgroups.  From kAdjTallNt triangles on,
+// 20 rounds of 64-row tiles, the tail no longer matters and 64 rows halve the
+// partial sums of V^H lambda (8 bytes a tile and column, nt^2 / 8 in all): 20480
+// triangles 21.3 ms either way, 81920 326 ms, with 800 MiB where 32 rows took 1600.
+constexpr int kAdjRowTile = 64;  // the taller
+constexpr int64_t kAdjTallNt = 16384;
+static int adj_rows(int64_t nt) { return nt < kAdjTallNt ? kAdjRowTile / 2 : kAdjRowTile; }
 
 template <bool CLAMP>
 __global__ __launch_bounds__(256, 3) void adj_regular_kernel(const float* __restrict__ rec, const float* __restrict__ geo,
@@ -163,7 +168,8 @@ __global__ __launch_bounds__(256, 3) void adj_regular_kernel(const float* __rest
                                                           const float2* __restrict__ lam,
                                                           const float2* __restrict__ psi,
                                                           const float2* __restrict__ phi, double* __restrict__ gvert,
-                                                          double* __restrict__ gk_out, float2* __restrict__ vhl_part)
+                                                          double* __restrict__ gk_out, float2* __restrict__ vhl_part,
+                                                          int rows)
 {
     constexpr int Q = 6;
     constexpr int S = Rec<Q>::kFloats;
@@ -191,8 +197,8 @@ __global__ __launch_bounds__(256, 3) void adj_regular_kernel(const float* __rest
     for (int b = 0; b < Q; ++b) gy[b][0] = gy[b][1] = gy[b][2] = gs[b] = 0.f;
     float gn[3] = {0.f, 0.f, 0.f}, ecol = 0.f, gk = 0.f, gks = 0.f, vr = 0.f, vi = 0.f;
 
-    const int64_t i_begin = (int64_t)blockIdx.y * kAdjRowTile;
-    const int64_t i_end = min(i_begin + (int64_t)kAdjRowTile, nt);
+    const int64_t i_begin = (int64_t)blockIdx.y * rows;
+    const int64_t i_end = min(i_begin + (int64_t)rows, nt);
     for (int64_t i = i_begin; i < i_end; ++i) {
         const int4 ti = tris[i];
         const bool shared = ti.x == tj.x || ti.x == tj.y || ti.x == tj.z || ti.y == tj.x || ti.y == tj.y ||
@@ -540,22 +546,23 @@ __global__ __launch_bounds__(256) void adj_mass_vhl_kernel(const float* __restri
 // ---------------------------------------------------------------------------
 int64_t adjoint_work_bytes(const MeshDev& m)
 {
-    const int64_t nby = (m.nt + kAdjRowTile - 1) / kAdjRowTile;
-    return (int64_t)sizeof(float2) * nby * m.nt;
+    const int rows = adj_rows(m.nt);
+    return (int64_t)sizeof(float2) * ((m.nt + rows - 1) / rows) * m.nt;
 }
 
 hipError_t launch_adjoint_pairs(const MeshDev& m, float k, int clamp, const float2* lam, const float2* psi,
                                 const float2* phi, double* gvert, double* gk, double* vhl, void* work, hipStream_t s)
 {
-    const int64_t nby = (m.nt + kAdjRowTile - 1) / kAdjRowTile;
+    const int rows = adj_rows(m.nt);
+    const int64_t nby = (m.nt + rows - 1) / rows;
     float2* part = (float2*)work;
     dim3 grid((unsigned)((m.nt + 255) / 256), (unsigned)nby);
     if (clamp)
         hipLaunchKernelGGL(adj_regular_kernel<true>, grid, dim3(256), 0, s, m.rec6, m.geo, m.tris, m.nt, k, lam, psi,
-                           phi, gvert, gk, part);
+                           phi, gvert, gk, part, rows);
     else
         hipLaunchKernelGGL(adj_regular_kernel<false>, grid, dim3(256), 0, s, m.rec6, m.geo, m.tris, m.nt, k, lam, psi,
-                           phi, gvert, gk, part);
+                           phi, gvert, gk, part, rows);
     const unsigned g = (unsigned)((m.npairs + 15) / 16);
     if (clamp)
         hipLaunchKernelGGL(adj_singular_kernel<true>, dim3(g), dim3(256), 0, s, m.geo, m.tris, m.pairs_by_kind, m.npairs, k,

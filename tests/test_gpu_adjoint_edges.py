@@ -96,3 +96,40 @@ def test_p1_vertex_gradient(level):
         fd.append((lp - lm) / (2 * h))
         ad.append(float(np.sum(gv * d)))
     assert np.linalg.norm(np.array(ad) - fd) < 2e-3 * np.linalg.norm(fd)
+
+
+def test_tall_row_tiles():
+    """From 16384 triangles on a row tile holds 64 triangles: the scratch is an
+    eighth of a byte per pair, V^H lambda equals the product with the assembled
+    operator (1e-5, the operators' bar), and the vertex gradients add up to zero
+    (every pair term depends on differences of positions only: what a pair gives
+    its row triangle it takes from its column triangle; FP32 per triangle, 1e-3
+    allowed)."""
+    import ctypes
+
+    from neuralat_amd import _lib
+    from neuralat_amd.bem import BEM_Solver
+    from neuralat_amd.bem.solver import matvec
+
+    v, t = mesh.icosphere(5, 0.1)
+    v = mesh.sh_perturb(v, 4, 0.05, seed=6).astype(np.float32)
+    n = len(t)
+    s = BEM_Solver(torch.tensor(v, device=_dev()), torch.tensor(t, device=_dev()), basis="DP0")
+    lib = _lib.load()
+    size = lib.bem_adjoint_work_size(s.mesh.handle)
+    assert size <= n * n // 8
+    g = torch.Generator(_dev()).manual_seed(4)
+    lam, psi, phi = (torch.randn(n, dtype=torch.complex64, device=_dev(), generator=g) for _ in range(3))
+    gvert = torch.zeros((len(v), 3), dtype=torch.float64, device=_dev())
+    gk = torch.zeros(1, dtype=torch.float64, device=_dev())
+    vhl = torch.zeros((n, 2), dtype=torch.float64, device=_dev())
+    work = torch.empty(size, dtype=torch.uint8, device=_dev())
+    print("adjoint tall tiles", n, flush=True)
+    ptr = lambda x: ctypes.c_void_p(x.data_ptr())  # noqa: E731
+    _lib.check(lib.bem_adjoint_cbie_dp0(s.mesh.handle, 9.0, 1, ptr(lam), ptr(psi), ptr(phi), ptr(gvert), ptr(gk),
+                                        ptr(vhl), ptr(work), ctypes.c_void_p(0)))
+    torch.cuda.synchronize()
+    want = matvec(s.assemble_boundary_matrix(9.0, "single"), lam, trans=2)
+    got = torch.complex(vhl[:, 0], vhl[:, 1])
+    assert float((got - want).norm() / want.norm()) < 1e-5
+    assert float(gvert.sum(0).norm()) < 1e-3 * float(gvert.norm(dim=1).sum())
