@@ -102,8 +102,10 @@ Tiling make_tiling(const std::vector<int32_t>& perm, const int32_t* tris, int64_
 
 // Pinned host staging for uploads (a DMA copy instead of a staged pageable
 // one: 1 MB takes 27 us against 140 to 315).  One process-wide buffer, grown
-// on demand up to kPinnedStageMax and kept until the process ends; larger
-// uploads stage in pageable memory.  The lock is held until the copy is done.
+// on demand up to kPinnedStageMax and kept until the process ends.  Its user
+// holds it until the copy is done, which may be behind other work on its
+// stream, so nobody waits for it: while it is taken, and for larger uploads,
+// pageable memory is the stage.
 constexpr size_t kPinnedStageMax = (size_t)64 << 20;
 std::mutex g_stage_mu;
 char* g_stage = nullptr;
@@ -114,8 +116,8 @@ public:
     char* get(size_t bytes)
     {
         if (bytes <= kPinnedStageMax) {
-            lk_ = std::unique_lock<std::mutex>(g_stage_mu);
-            if (g_stage_cap < bytes) {
+            lk_ = std::unique_lock<std::mutex>(g_stage_mu, std::try_to_lock);
+            if (lk_.owns_lock() && g_stage_cap < bytes) {
                 if (g_stage) (void)hipHostFree(g_stage);
                 g_stage = nullptr;
                 g_stage_cap = 0;
@@ -127,8 +129,10 @@ public:
                     g_stage = nullptr;
                 }
             }
-            if (g_stage) return g_stage;
-            lk_.unlock();
+            if (lk_.owns_lock()) {
+                if (g_stage) return g_stage;
+                lk_.unlock();
+            }
         }
         pageable_.resize(bytes);
         return pageable_.data();

@@ -2,6 +2,7 @@
 checks, on meshes around its 256-triangle workgroups.  The arrays are FP64
 values rounded once, so they match numpy's to one FP32 rounding."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -82,3 +83,42 @@ def test_positions_outside_the_device_are_copied():
     n, c = (a.cpu().numpy() for a in m.normals_curls())
     rn, rc = _normals_curls(moved.numpy(), t)
     assert np.abs(n - rn).max() < 1.2e-7 and np.abs(c - rc).max() < 1.2e-7 * np.abs(rc).max()
+
+
+def test_setup_does_not_wait_for_another_stream():
+    """A geometry set created behind other work on its stream holds the pinned
+    stage until its upload is done; a mesh created by another thread on another
+    stream meanwhile stages elsewhere and finishes first."""
+    from neuralat_amd.bem import GeometrySet, Mesh
+
+    v, t = mesh.icosphere(2, 0.1)
+    v = v.astype(np.float32)
+    vt, tt = torch.tensor(v, device=_dev()), torch.tensor(t, device=_dev())
+    base = Mesh(vt, tt)
+    busy, other = torch.cuda.Stream(), torch.cuda.Stream()
+    big = torch.randn(8192, 8192, device=_dev())
+    kept = [big @ big]  # the library's own set-up and the allocation, done before
+    torch.cuda.synchronize()
+    print("set-up beside a busy stream", flush=True)
+
+    def queue_and_create():
+        with torch.cuda.stream(busy):
+            for _ in range(60):  # 7 ms each
+                torch.mm(big, big, out=kept[0])
+            queued.set()
+            kept.append(GeometrySet(base, np.stack([v, v * np.float32(1.1)])))
+
+    queued = threading.Event()
+    a = threading.Thread(target=queue_and_create)
+    a.start()
+    assert queued.wait(30)
+    a.join(0.05)  # into the upload
+    assert a.is_alive()
+    with torch.cuda.stream(other):
+        m = Mesh(vt, tt)
+        first = a.is_alive()
+    a.join()
+    assert first, "the mesh waited for the other thread's stream"
+    n, _ = m.normals_curls()
+    torch.cuda.synchronize()
+    assert np.abs(n.cpu().numpy() - _normals_curls(v, t)[0]).max() < 1.2e-7
