@@ -2649,8 +2649,9 @@ hipError_t launch_bm_systems_p1(const MeshDev& mg, int64_t gstride, const float*
                                 const float2* g, float2* lhs, int64_t ld, int64_t stride, float2* rhs, hipStream_t s)
 {
     const int64_t n = mg.nv;
-    for (int z0 = 0; z0 < nk; z0 += kMaxBatchK) {
-        const int nz = nk - z0 < kMaxBatchK ? nk - z0 : kMaxBatchK;
+    int most = kMaxBatchK;  // systems a launch: fewer once their pairs' scratch (96 bytes a pair and system) finds no room
+    for (int z0 = 0, nz; z0 < nk; z0 += nz) {
+        nz = nk - z0 < most ? nk - z0 : most;
         KBatch kb{};
         for (int z = 0; z < nz; ++z) kb.k[z] = ks[z0 + z];
         const MeshDev m = geometry_shift(mg, (int64_t)z0 * gstride);
@@ -2659,6 +2660,12 @@ hipError_t launch_bm_systems_p1(const MeshDev& mg, int64_t gstride, const float*
         float2* rz = rhs + (int64_t)z0 * n;
         const hipError_t e = clamp ? bm_system_p1_t<true>(m, gstride, kb, nz, quad, gz, lz, ld, stride, rz, s)
                                    : bm_system_p1_t<false>(m, gstride, kb, nz, quad, gz, lz, ld, stride, rz, s);
+        if (e == hipErrorOutOfMemory && nz > 1) {  // nothing but a fill was launched
+            (void)hipGetLastError();
+            most = (nz + 1) / 2;
+            nz = 0;
+            continue;
+        }
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

@@ -75,3 +75,33 @@ def test_burton_miller_systems(surface, quad, clamp):
         for lhs, rhs in [singles[q]] + ([(batch[0][z], batch[1][z])] if batch else []):
             assert _rel(lhs.cpu().numpy(), L) < TOL
             assert _rel(rhs.cpu().numpy(), r) < TOL
+
+
+def test_burton_miller_systems_with_little_memory():
+    """The systems' neighbour-pair scratch takes 96 bytes a pair and system: where
+    it does not fit for all systems of a launch, fewer go at a time.  A
+    1024-triangle fan (2^20 pairs, 100 MB a system), 24 systems, 1.5 GB free."""
+    from neuralat_amd.bem import BEM_Solver
+
+    d = 1024
+    a = 2 * np.pi * np.arange(d) / d
+    v = np.concatenate([[[0, 0, 0.05]], np.stack([0.1 * np.cos(a), 0.1 * np.sin(a), 0 * a], 1)]).astype(np.float32)
+    t = np.stack([0 * np.arange(d), 1 + np.arange(d), 1 + (np.arange(d) + 1) % d], 1).astype(np.int32)
+    s = BEM_Solver(torch.tensor(v, device=_dev()), torch.tensor(t, device=_dev()))
+    ks = [2.0 + 0.5 * z for z in range(24)]
+    g = torch.randn(24, d + 1, dtype=torch.complex64, device=_dev(), generator=torch.Generator(_dev()).manual_seed(5))
+    want = [s.burton_miller_system(ks[z], g[z], approx=True) for z in (0, 11, 23)]
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    free = torch.cuda.mem_get_info()[0]
+    hog = torch.empty(free - (3 << 29), dtype=torch.uint8, device=_dev())
+    print("burton-miller systems, 1.5 GB free", flush=True)
+    try:
+        L, R = s.burton_miller_systems(ks, g)
+        torch.cuda.synchronize()
+    finally:
+        del hog
+        torch.cuda.empty_cache()
+    for z, (l1, r1) in zip((0, 11, 23), want):
+        assert float((L[z] - l1).norm() / l1.norm()) < TOL
+        assert float((R[z] - r1).norm() / r1.norm()) < TOL
