@@ -62,6 +62,35 @@ def test_long_basis():
     assert _err(A, x, b[0]) < 1.2e-5, info
 
 
+def test_long_basis_in_lockstep():
+    """The same hand-over to the separate kernels inside a cycle for several
+    right-hand sides, for a batch (beside a short system) and for the one-pass
+    steps of a batch's 16-bit inner solves.  Those get one outer step, so that
+    one inner cycle takes over 227 steps; its solution is then off by the fp16
+    rounding of A, 2^-11 |A| |x| / |b| < 1e-2."""
+    from neuralat_amd.bem.batch import batch_gmres, batch_solve_mixed
+    from neuralat_amd.bem.precision import gmres_multi
+
+    A, B = _system(9000, 0.98, 9, 2)
+    print("arnoldi long basis, right-hand sides", flush=True)
+    X, infos = gmres_multi(A, B, tol=1e-5, restart=400, maxiter=1000)
+    for q in range(2):
+        assert infos[q]["converged"] and _err(A, X[q], B[q]) < 1.2e-5, infos[q]
+    assert 227 < infos[0]["iterations"] <= 400, infos[0]
+    C, c = _system(700, 0.6, 700)
+    print("arnoldi long basis, batch", flush=True)
+    xs, infos = batch_gmres([A, C], [B[0], c[0]], tol=1e-5, restart=400)
+    assert 227 < infos[0]["iterations"], infos
+    for M, b, x, i in zip((A, C), (B[0], c[0]), xs, infos):
+        assert i["converged"] and _err(M, x, b) < 1.2e-5, i
+    print("arnoldi long basis, inner solves", flush=True)
+    xs, infos = batch_solve_mixed([A, C], [B[0], c[0]], dtype="fp16", tol=1e-6, inner_tol=1e-5, outer_restart=1,
+                                  inner_restart=400, max_inner_cycles=1, max_outer_cycles=1)
+    assert 227 < infos[0]["inner_iterations"] < 400, infos
+    for M, b, x in zip((A, C), (B[0], c[0]), xs):
+        assert _err(M, x, b) < 1e-2
+
+
 @pytest.mark.parametrize("n,nrhs", [(65, 3), (700, 17), (5000, 2)])
 def test_many_right_hand_sides(n, nrhs):
     from neuralat_amd.bem.precision import gmres_multi
