@@ -1286,7 +1286,6 @@ __global__ __launch_bounds__(256) void p1_regular_kernel(const float* __restrict
                 gc = vmap[gc];
             }
             const float2 v = acc[rvi][cvi];
-            if (rparts > 1 && v.x == 0.f && v.y == 0.f) continue;
             if (plane) {
                 float* dst = reinterpret_cast<float*>(out) + (gc * ld + gr);
                 unsafeAtomicAdd(dst, v.x);
@@ -2171,8 +2170,8 @@ static hipError_t p1_regular_t(const MeshDev& m, const KBatch& kb, int nz, float
     constexpr bool pair = (OP == DLP || OP == ADLP) && Q == 6;
     const int64_t plane = planar ? n * n : 0;
     if (!p1_ordered_sweep<OP, Q>(m, one_sided)) {
-        const int parts = p1_row_parts(m.tiles.nsym, nz);
         if constexpr (sym) {
+            const int parts = p1_row_parts(m.tiles.nsym, nz);
             hipLaunchKernelGGL((p1_regular_kernel<OP, Q, CLAMP, kSweepSym>), dim3((unsigned)m.tiles.nsym, 1, nz * parts),
                                dim3(256), 0, s, rec, m.tris, m.curls, m.tiles, kb, out, ld, vmap, nullptr, nullptr,
                                (int64_t)0, P1PairBlocks{}, parts);
@@ -2180,9 +2179,10 @@ static hipError_t p1_regular_t(const MeshDev& m, const KBatch& kb, int nz, float
                                n, ld, kb.zstride);
         } else if constexpr (pair) {
             if (planar) *planar = true;
-            hipLaunchKernelGGL((p1_regular_kernel<OP, Q, CLAMP, kSweepPair>), dim3((unsigned)m.tiles.nsym, 1, nz * parts),
+            // whole row tiles: kP1PairMinVerts vertices make more tile pairs than p1_row_parts splits
+            hipLaunchKernelGGL((p1_regular_kernel<OP, Q, CLAMP, kSweepPair>), dim3((unsigned)m.tiles.nsym, 1, nz),
                                dim3(256), 0, s, rec, m.tris, m.curls, m.tiles, kb, out, ld, vmap, nullptr, nullptr,
-                               plane, P1PairBlocks{}, parts);
+                               plane, P1PairBlocks{}, 1);
         }
         return hipGetLastError();
     }
