@@ -328,7 +328,7 @@ __global__ __launch_bounds__(256, 3) void adj_regular_kernel(const float* __rest
 }
 
 // ---------------------------------------------------------------------------
-// neighbour pairs: Sauter-Schwab, one wavefront per pair
+// neighbour pairs: Sauter-Schwab
 // ---------------------------------------------------------------------------
 // 16 lanes per pair: the set-up, the sums over lanes, the chain to the vertices
 // and the scatter serve four pairs of a wavefront (grouped by kind, so that the

@@ -11,8 +11,8 @@
 //     triangle list; the 3x3 basis blocks of its pairs are summed in LDS on
 //     the tile's compacted vertex slots, then flushed once per tile entry.
 // Neighbour pairs (sharing >= 1 vertex; bind.cu:81-152, integrand.h:63-185,
-// 331-394) go to a separate Sauter-Schwab kernel: one wavefront per pair,
-// the n^4 tensor Gauss points spread over the lanes, FP64 accumulation.
+// 331-394) go to separate Sauter-Schwab kernels: the n^4 tensor Gauss points of
+// a pair spread over 4 to 64 lanes, FP64 accumulation.
 #include "bem_device.hpp"
 #include "bem_internal.hpp"
 
@@ -1332,15 +1332,8 @@ __global__ __launch_bounds__(256) void p1_symmetrize_kernel(float2* __restrict__
 }
 
 // ---------------------------------------------------------------------------
-// neighbour (singular) pairs: Sauter-Schwab, one wavefront per pair
+// neighbour (singular) pairs: Sauter-Schwab
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double wave_sum(double v)
-{
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 // sum over aligned groups of N lanes (N a power of two <= 64), in every lane
 // (4, 16 and 64: DPP row moves, bem_device.hpp; others: cross-lane permutes)
 template <int N>
@@ -2092,8 +2085,10 @@ static hipError_t dp0_regular_t(const MeshDev& m, int64_t row0, int64_t row1, co
 // imaginary ones.  One workgroup per output row, written whole.  Bound by HBM;
 // rows of up to kPermLdsVerts vertices are read in order into LDS and gathered
 // there (7842 vertices: 194 us, gathered from L2 446 us), longer ones
-// gathered from L2.
-constexpr int64_t kPermLdsVerts = 8192;  // 64 KB: two workgroups a CU
+// gathered from L2.  The line is the 64 KB of LDS a kernel gets without asking
+// for more (two workgroups a CU); longer rows in LDS, one workgroup a CU, were
+// not measured.
+constexpr int64_t kPermLdsVerts = 8192;
 template <bool PLANAR, bool LDS>
 __global__ __launch_bounds__(1024) void p1_permute_kernel(const float* __restrict__ S, int64_t n,
                                                           const int32_t* __restrict__ vnew, float2* __restrict__ out,
