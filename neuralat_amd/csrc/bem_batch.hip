@@ -21,6 +21,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <numeric>
@@ -874,13 +875,16 @@ hipError_t xcycle_fin(const XEng& E, hipStream_t st)
 // Arnoldi steps per graph segment; the host reads the flags between segments.
 // The first segment is short: a restart cycle that follows a nearly converged
 // one (the implicit residual reached the target, the true one not quite)
-// usually needs a step or two.
-constexpr int kSeg0 = 4, kSeg = 20;
+// usually needs a step or two.  A later one is read after kSegNear steps too
+// when the decay so far says that the slowest item will be done by then: the
+// launches of steps that every item skips cost 5 us a step (one system of 900
+// unknowns, done in 8 steps: 444 us with 16 such steps, 382 with 4).
+constexpr int kSeg0 = 4, kSeg = 20, kSegNear = 8;
 inline int seg_count(int m) { return m <= kSeg0 ? 1 : 1 + (m - kSeg0 + kSeg - 1) / kSeg; }
 inline int seg_begin(int k) { return k == 0 ? 0 : kSeg0 + (k - 1) * kSeg; }
 
-// A restart cycle as graphs: slot 0 the start, 1 .. nseg the step segments,
-// nseg + 1 the end.  A slot runs as direct launches on its first two uses, is
+// A restart cycle as graphs: slot 0 the start, three for each step segment (the
+// whole, its first kSegNear steps, the rest), the last one the end.  A slot runs as direct launches on its first two uses, is
 // captured on its third and replayed from then on: a capture pays only when
 // the graph is replayed (later restart cycles, the inner solves of later
 // outer steps), and solves done in one or two cycles capture nothing.
@@ -936,22 +940,43 @@ hipError_t xrun_slot(XGraphs* G, int nslots, int slot, hipStream_t s, F&& f)
 // the cycle early once every item is done.
 hipError_t xrun_cycle(const XEng& E, XGraphs* G, hipStream_t s, std::vector<int>& hd)
 {
-    const int nseg = seg_count(E.m), nslots = nseg + 2;
+    const int nseg = seg_count(E.m), nslots = 3 * nseg + 2;
     hipError_t e = xrun_slot(G, nslots, 0, s, [&](hipStream_t st) { return xcycle_init(E, st); });
     if (e != hipSuccess) return e;
-    for (int k = 0; k < nseg; ++k) {
-        e = xrun_slot(G, nslots, 1 + k, s,
-                      [&](hipStream_t st) { return xcycle_steps(E, seg_begin(k), std::min(E.m, seg_begin(k + 1)), st); });
+    // res, rn2, wn2, tgt and done lie in this order: read by one copy
+    const size_t done_at = (size_t)((char*)E.done - (char*)E.res);
+    std::vector<char> state(done_at + sizeof(int) * (size_t)E.ns);
+    const double* res = (const double*)state.data();
+    const double *rn2 = res + (E.rn2 - E.res), *tgt = res + (E.tgt - E.res);
+    std::vector<double> before(E.ns);  // the residuals at the last read
+    bool all = false, near = false;    // every item done; the slowest within kSegNear steps at the decay since then
+    auto steps = [&](int slot, int j0, int j1) {
+        hipError_t er = xrun_slot(G, nslots, slot, s, [&](hipStream_t st) { return xcycle_steps(E, j0, j1, st); });
+        if (er == hipSuccess) er = hipMemcpyAsync(state.data(), E.res, state.size(), hipMemcpyDeviceToHost, s);
+        if (er == hipSuccess) er = hipStreamSynchronize(s);
+        if (er != hipSuccess) return er;
+        std::memcpy(hd.data(), state.data() + done_at, sizeof(int) * (size_t)E.ns);
+        all = near = true;
+        for (int q = 0; q < E.ns; ++q) {
+            if (hd[q]) continue;
+            all = false;
+            const double rate = std::log((j0 ? before[q] : std::sqrt(rn2[q])) / res[q]) / (j1 - j0);
+            near = near && rate > 0.0 && std::log(res[q] / tgt[q]) <= rate * kSegNear;
+            before[q] = res[q];
+        }
+        return hipSuccess;
+    };
+    for (int k = 0; k < nseg && !all; ++k) {
+        const int j0 = seg_begin(k), j1 = std::min(E.m, seg_begin(k + 1)), jn = j0 + kSegNear;
+        if (k > 0 && near && jn < j1) {
+            e = steps(2 + 3 * k, j0, jn);
+            if (e == hipSuccess && !all) e = steps(3 + 3 * k, jn, j1);
+        } else {
+            e = steps(1 + 3 * k, j0, j1);
+        }
         if (e != hipSuccess) return e;
-        e = hipMemcpyAsync(hd.data(), E.done, sizeof(int) * E.ns, hipMemcpyDeviceToHost, s);
-        if (e != hipSuccess) return e;
-        e = hipStreamSynchronize(s);
-        if (e != hipSuccess) return e;
-        bool all = true;
-        for (int q = 0; q < E.ns && all; ++q) all = hd[q] != 0;
-        if (all) break;
     }
-    return xrun_slot(G, nslots, nseg + 1, s, [&](hipStream_t st) { return xcycle_fin(E, st); });
+    return xrun_slot(G, nslots, nslots - 1, s, [&](hipStream_t st) { return xcycle_fin(E, st); });
 }
 
 // Workspace of the mixed-precision batch solve

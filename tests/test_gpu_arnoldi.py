@@ -173,3 +173,16 @@ def _err_rows(A, x, b):
     r = torch.cat([b[q:q + 2048].to(torch.complex128) - A[q:q + 2048].to(torch.complex128) @ x.to(torch.complex128)
                    for q in range(0, len(b), 2048)])
     return float(torch.linalg.vector_norm(r) / torch.linalg.vector_norm(b.to(torch.complex128)))
+
+
+def test_short_lockstep_solve_stops_near_its_end():
+    """A batch that converges in its eighth step launches no whole segment (16
+    more steps) past it: as long as with restart=12, whose cycle ends at step 12."""
+    from neuralat_amd.bem.batch import batch_gmres
+
+    A, b = _system(1000, 0.2, 3)
+    print("arnoldi short lockstep", flush=True)
+    _, infos = batch_gmres([A], [b[0]], tol=1e-5, restart=50)
+    assert infos[0]["converged"] and 4 < infos[0]["iterations"] < 12, infos
+    free, held = (_best(lambda: batch_gmres([A], [b[0]], tol=1e-5, restart=r), 25) for r in (50, 12))
+    assert free < 1.1 * held, (free, held)
