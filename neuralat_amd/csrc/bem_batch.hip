@@ -884,10 +884,11 @@ inline int seg_count(int m) { return m <= kSeg0 ? 1 : 1 + (m - kSeg0 + kSeg - 1)
 inline int seg_begin(int k) { return k == 0 ? 0 : kSeg0 + (k - 1) * kSeg; }
 
 // A restart cycle as graphs: slot 0 the start, three for each step segment (the
-// whole, its first kSegNear steps, the rest), the last one the end.  A slot runs as direct launches on its first two uses, is
-// captured on its third and replayed from then on: a capture pays only when
-// the graph is replayed (later restart cycles, the inner solves of later
-// outer steps), and solves done in one or two cycles capture nothing.
+// whole, its first kSegNear steps, the rest), the last one the end.  A slot
+// runs as direct launches on its first two uses, is captured on its third and
+// replayed from then on: a capture pays only when the graph is replayed (later
+// restart cycles, the inner solves of later outer steps), and solves done in
+// one or two cycles capture nothing.
 struct XGraphs {
     std::vector<hipGraph_t> g;
     std::vector<hipGraphExec_t> x;
