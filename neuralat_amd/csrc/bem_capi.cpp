@@ -856,15 +856,16 @@ int bem_gmres_timed(const void* A_, int64_t n, int64_t lda, int trans, const voi
     double rnorm = 0.0, implicit = 0.0;
     bool conv = false;
     // The implicit residuals are read every few steps (a read idles the GPU for
-    // about 20 us): up to chk steps at a time, fewer once the decay seen so far
-    // says the target is near.  Steps taken past convergence are dropped, so
-    // only their time is lost: long windows where a step costs no more than
-    // a read, none where a product takes hundreds of microseconds.  In between
-    // a cycle's first step is read by itself: cycles of one step (a good initial
-    // guess, the last correction) would pay four products for one (such a solve
-    // of 12000 unknowns: 1228 us, now 669).
+    // about 20 us): up to kMaxWindow steps at a time, fewer once the decay seen
+    // so far says the target is near.  Steps taken past convergence are dropped,
+    // so only their time is lost: none are risked beyond 12288 unknowns, where a
+    // product costs several reads, and above 4096 a cycle's first step is read by
+    // itself.  Cycles of one step (a good initial guess, the last correction)
+    // would pay three more products there (12000 unknowns: 1217 us, now 667), and
+    // before that read no decay is known (5120 unknowns, 14 and 39 steps: windows
+    // of 4 from the start 1095 and 3195 us, now 1056 and 2872).
     constexpr int kMaxWindow = 8;
-    const int chk = timed ? 1 : (n <= 4096 ? kMaxWindow : (n <= 12288 ? 4 : 1));
+    const int chk = timed || n > 12288 ? 1 : kMaxWindow;
     bem::ArnoldiDesc D;
     D.m = m;
     D.hs = m + 1;
